@@ -744,120 +744,581 @@ __global__ __launch_bounds__(TS_THREADS) void k_ts_merge(int c0, int w, int nin,
 }
 
 // ---------------------------------------------------------------------------
-// Partial-pivoting strips, for the entry points that return the factors
-// (qpms_hip_zgetrf_dev and the ABI factorisation built on it): the pivots of
-// zgetrf (zgetf2's column loop, scatsystem.c:2214): pivot j is the first row
-// of largest |re| + |im| in column j at or below the diagonal, taken in full
-// double (or float) precision. One launch per column (k_pp_step): every
-// workgroup applies the previous column's interchange and elimination to its
-// rows of the strip (the pivot row and the old top row come from copies in the
-// workspace, so no workgroup reads a row another one rewrites), then reduces
-// the next column's candidates; the last workgroup to finish (an atomic
-// count after a device-scope release) combines the partial maxima, records
-// the pivot and copies the pivot row and the top row for the next launch.
-// k_pp_finish then writes the strip's slot (L11\U11, the moved-row list,
-// L11^{-1}, U11^{-1}) as the tournament's last level does, so the rest of the
-// LU is shared. L21 is left in place by the elimination.
+// Partial-pivoting strips (k_strip), for the entry points that return the
+// factors (qpms_hip_zgetrf_dev and the ABI factorisation built on it): the
+// pivots of zgetrf (zgetf2's column loop, scatsystem.c:2214): pivot j is the
+// first row of largest |re| + |im| in column j at or below the diagonal, taken
+// in full double (or float) precision. One launch factors a whole strip: the
+// workgroups hold its rows in registers for all of its columns and agree on
+// each pivot through memory. k_pp_finish then writes the strip's slot (L11\U11,
+// the moved-row list, L11^{-1}, U11^{-1}) as the tournament's last level does,
+// so the rest of the LU is shared. L21 is left in place by the elimination.
+//
+// Layout. A wave holds RT tiles of 16 rows; lane (rq, cq) = (lane % 16,
+// lane / 16) holds row rq of each tile and columns 4 i + cq, i = 0..7: the
+// accumulator layout of the 16 x 16 x 4 matrix instructions for the transposed
+// tile. Four columns (a chunk, register i) are factored with a row per lane: a
+// 4 x 4 transposition by lane swaps gives lane (rq, cq) row rq of tile cq and
+// its four entries y. Transposed back, register i is, as it stands, the right
+// operand of the rank-4 update of the columns beyond, whose left operand is the
+// chunk's U rows: four products per tile of 16 x 16. So a column step touches
+// four columns only. With a row per lane throughout and rank-1 updates of the
+// whole row, a column took 2.2 us beside its exchange (each wave took the whole
+// pivot row from LDS, and the row's owner wrote it there one lane wide).
+//
+// Exchange. Every word carries the column's tag beside its payload (a
+// candidate is two words: magnitude and position; a row is its entries' 32-bit
+// halves), so a reader needs no flag and no fence: it reads a word until the
+// tag is the column's. Words are relaxed agent-scope atomics, which pass the
+// XCDs' own L2s: about 1.3 us per column for 2 to 32 workgroups. One wave of a
+// workgroup reads them (every wave reading them took three times as long: the
+// words of a column lie in a few lines that all workgroups ask for). Sets of
+// words alternate between columns (candidates) and chunks (rows): a workgroup
+// writes a set again only after it has seen every workgroup's candidate of a
+// later column, hence after all of them have read the set. k_strip_init clears
+// the words before a factorisation; within one, neighbouring columns' tags
+// differ. One launch per column instead, with the strip read and written by
+// each, took 11.9 us per column at order 2190 and 18.9 us at 9216.
+//
+// Waiting. A workgroup may wait for another one only when all of them are on
+// the device. They announce themselves first: whoever has seen everybody moves
+// the strip's state word from 0 to GO, whoever has waited longer than the limit
+// moves it from 0 to ALONE, and the word's value after the attempt decides for
+// everybody. After GO every workgroup has started and none ends before the
+// last column, so every later wait ends. After
+// ALONE the workgroup that set it factors the strip by itself in memory and
+// the others leave without having written to the matrix.
 // ---------------------------------------------------------------------------
-constexpr int PP_ROWS = 64;   // rows per workgroup: 8 passes of 8 rows x 32 columns
-// per-matrix workspace layout (in the tournament's candidate area, unused here)
-constexpr long PP_CNT = 0, PP_PROW = 256, PP_TROW = 768, PP_PIV = 1280, PP_NZ = 1408, PP_PART = 1536;
-__host__ __device__ constexpr long pp_part_row_off(int G) { return PP_PART + ((long)G * 8 + 255) / 256 * 256; }
-__host__ __device__ constexpr long pp_ws_bytes(int n) {
-  return pp_part_row_off((n + PP_ROWS - 1) / PP_ROWS) + ((long)((n + PP_ROWS - 1) / PP_ROWS) * 4 + 255) / 256 * 256;
+constexpr int ST_GO = 1, ST_ALONE = 2;
+constexpr int ST_RT = 4;   // row tiles per wave
+// waves per workgroup: FP64 one per SIMD, FP32 two
+template <class T> constexpr int st_w() { return sizeof(T) == 8 ? 4 : 8; }
+template <class T> constexpr int st_rows() { return st_w<T>() * 16 * ST_RT; }   // 256 (FP64), 512 rows per workgroup
+typedef unsigned long long st_u64;
+constexpr st_u64 ST_LIMIT = 10000000ull;   // ticks of the 100 MHz clock (0.1 s) to wait for everybody
+// words of one row: the reciprocal of its pivot, then its entries
+template <class T> constexpr int st_ew() { return (int)sizeof(typename C2<T>::t) / 4; }
+template <class T> constexpr int st_words() { return (1 + PW_) * st_ew<T>(); }
+// Per-matrix workspace of the strips (in the tournament's candidate area,
+// unused here): the strip's pivots, a state word per strip, two sets of
+// candidates, the announcements, two sets of four rows per workgroup.
+constexpr long ST_PIV = 0, ST_STATE = 256;
+constexpr long st_cand_off(int n) { return ST_STATE + ((long)((n + PW_ - 1) / PW_) * 4 + 255) / 256 * 256; }
+template <class T> constexpr int st_groups(int rows) { return (rows + st_rows<T>() - 1) / st_rows<T>(); }
+template <class T> constexpr long st_meet_off(int n) { return st_cand_off(n) + 2L * st_groups<T>(n) * 2 * 8; }
+template <class T> constexpr long st_row_off(int n) { return st_meet_off<T>(n) + (long)st_groups<T>(n) * 8; }
+template <class T> constexpr long st_ws_bytes(int n) { return st_row_off<T>(n) + 8L * st_groups<T>(n) * st_words<T>() * 8; }
+
+__global__ __launch_bounds__(256) void k_strip_init(char *ws, long sW, long bytes) {
+  st_u64 *p = reinterpret_cast<st_u64 *>(ws + (long)blockIdx.z * sW);
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < bytes / 8; i += (long)gridDim.x * 256) p[i] = 0;
 }
 
-__global__ void k_pp_init(char *ws, long sW) { *reinterpret_cast<int *>(ws + (long)blockIdx.x * sW + PP_CNT) = 0; }
-
-// (magnitude, row) pairs: larger magnitude first, then the smaller row
-__device__ __forceinline__ void pp_better(double &m, int &r, double m2, int r2) {
-  if (m2 > m || (m2 == m && r2 < r)) { m = m2; r = r2; }
+__device__ __forceinline__ st_u64 st_load(const st_u64 *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void pp_reduce_wg(double &m, int &r, double *sm, int *sr) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const double m2 = __shfl_xor(m, off);
-    const int r2 = __shfl_xor(r, off);
-    pp_better(m, r, m2, r2);
+__device__ __forceinline__ void st_store(st_u64 *p, st_u64 v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A candidate's two words: 21 bits of tag above 43 bits of the rank, and above
+// its other 21 bits and 22 bits of the position.
+__device__ __forceinline__ void st_pack(unsigned tag, st_u64 rank, int pos, st_u64 &a, st_u64 &b) {
+  a = ((st_u64)tag << 43) | (rank >> 21);
+  b = ((st_u64)tag << 43) | ((rank & 0x1fffffull) << 22) | (unsigned)pos;
+}
+__device__ __forceinline__ bool st_unpack(unsigned tag, st_u64 a, st_u64 b, st_u64 &rank, int &pos) {
+  rank = (a << 21) | ((b >> 22) & 0x1fffffull);
+  pos = (int)(b & 0x3fffffull);
+  return (a >> 43) == tag && (b >> 43) == tag;
+}
+// A row's rank in the pivot search: the bits of |x|_1 (non-negative floating
+// values order as their bits) plus two, 1 where that is no number, 0 for no row.
+__device__ __forceinline__ st_u64 st_bits(double a) { return (st_u64)__double_as_longlong(a); }
+__device__ __forceinline__ st_u64 st_bits(float a) { return (st_u64)__float_as_uint(a); }
+template <class T> __device__ __forceinline__ st_u64 st_rank(bool live, typename C2<T>::t x) {
+  const T a = fabs(x.x) + fabs(x.y);
+  return live ? ((a == a) ? st_bits(a) + 2 : 1) : 0;
+}
+__device__ __forceinline__ bool st_before(st_u64 r, int p, st_u64 r2, int p2) { return r > r2 || (r == r2 && p < p2); }
+template <int CTRL, int RM>
+__device__ __forceinline__ unsigned st_dmax(unsigned v) {   // lanes without a source keep their own value
+  const unsigned o = (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, RM, 0xF, false);
+  return o > v ? o : v;
+}
+// The lane of a wave with the largest rank, the smallest position among equal
+// ones; rank and pos become that lane's. One DPP chain on the ranks' leading 32
+// bits (FP32: all of them); lanes that tie there are compared one by one.
+template <bool WIDE>
+__device__ __forceinline__ int st_wave_best(st_u64 &rank, int &pos) {
+  const unsigned own = WIDE ? (unsigned)(rank >> 32) : (unsigned)rank;
+  unsigned v = own;
+  v = st_dmax<0xB1, 0xF>(v);    // quad_perm [1,0,3,2]
+  v = st_dmax<0x4E, 0xF>(v);    // quad_perm [2,3,0,1]
+  v = st_dmax<0x124, 0xF>(v);   // row_ror 4
+  v = st_dmax<0x128, 0xF>(v);   // row_ror 8
+  v = st_dmax<0x142, 0xA>(v);   // row_bcast 15
+  v = st_dmax<0x143, 0xC>(v);   // row_bcast 31
+  const unsigned m = (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+  st_u64 eq = __ballot(own == m && rank != 0);
+  if (eq == 0) {   // no row in the wave
+    rank = 0;
+    return 0;
   }
-  const int t = threadIdx.x, wave = t >> 6;
-  if ((t & 63) == 0) { sm[wave] = m; sr[wave] = r; }
-  __syncthreads();
-  m = sm[0];
-  r = sr[0];
-  for (int q = 1; q < (int)(blockDim.x >> 6); ++q) pp_better(m, r, sm[q], sr[q]);
+  int l = __ffsll((long long)eq) - 1;
+  const int lo = (int)(unsigned)rank, hi = (int)(rank >> 32);
+  auto rank_of = [&](int i) {
+    return ((st_u64)(unsigned)__builtin_amdgcn_readlane(hi, i) << 32) | (unsigned)__builtin_amdgcn_readlane(lo, i);
+  };
+  st_u64 r = rank_of(l);
+  int p = __builtin_amdgcn_readlane(pos, l);
+  for (eq &= eq - 1; eq; eq &= eq - 1) {   // uniform
+    const int l2 = __ffsll((long long)eq) - 1, p2 = __builtin_amdgcn_readlane(pos, l2);
+    const st_u64 r2 = rank_of(l2);
+    if (st_before(r2, p2, r, p)) { r = r2; p = p2; l = l2; }
+  }
+  rank = r;
+  pos = p;
+  return l;
 }
 
 template <class T>
-__global__ __launch_bounds__(256) void k_pp_step(int n, int c0, int w, int j, typename C2<T>::t *A, long lda, long sA,
-                                                 char *ws, long sW, int *ipiv, long sP, int *info) {
+struct StShared {
   typedef typename C2<T>::t cT;
-  const int z = blockIdx.z, g = blockIdx.x, G = gridDim.x, t = threadIdx.x, k = t & 31, rr = t >> 5;
+  // rows in rotated order (entry 4 q + c is register q's column c: the chunk's
+  // four entries first): the workgroup's candidate on its way to memory, the
+  // chunk's pivot rows as they were when chosen, and their pivots' reciprocals
+  __align__(16) cT own[PW_], urow[4][PW_], rcp[4], orcp;
+  st_u64 rank[2][st_w<T>()];
+  int pos[2][st_w<T>()];
+  st_u64 prank;
+  int ppos;
+  int from[4];                     // the workgroups that had the chunk's pivots
+  int piv[PW_], nz[PW_];
+  int state;
+};
+
+// The strip's pivots (strip rows piv, nz[i] = 0 for a zero one) to the
+// workspace, ipiv and info.
+__device__ __forceinline__ void st_pivots(int c0, int w, const int *piv, const int *nz, char *wz, int *ipiv, int *info) {
+  int *out = reinterpret_cast<int *>(wz + ST_PIV);
+  for (int i = 0; i < w; ++i) {
+    out[i] = c0 + piv[i];
+    ipiv[c0 + i] = c0 + piv[i] + 1;
+    if (!nz[i] && *info == 0) *info = c0 + i + 1;
+  }
+}
+
+// The strip's rows (S = row c0, column c0; m of them) factored in memory by one
+// workgroup, after ALONE: a plain column loop.
+template <class T>
+__device__ __noinline__ void st_alone(int m, int w, typename C2<T>::t *S, long lda, StShared<T> &sh) {
+  typedef typename C2<T>::t cT;
+  constexpr bool WIDE = sizeof(T) == 8;
+  const int t = threadIdx.x, nt = st_w<T>() * 64, lane = t & 63, wave = t >> 6;
+  for (int j = 0; j < w; ++j) {
+    st_u64 rank = 0;
+    int pos = 0x3fffff;
+    for (int i = j + t; i < m; i += nt) {
+      const st_u64 r = st_rank<T>(true, S[(long)i * lda + j]);
+      if (r > rank) { rank = r; pos = i; }   // a thread's rows come in rising order
+    }
+    (void)st_wave_best<WIDE>(rank, pos);
+    if (lane == 0) { sh.rank[0][wave] = rank; sh.pos[0][wave] = pos; }
+    __syncthreads();
+    for (int q = 0; q < st_w<T>(); ++q)
+      if (q == 0 || st_before(sh.rank[0][q], sh.pos[0][q], rank, pos)) { rank = sh.rank[0][q]; pos = sh.pos[0][q]; }
+    if (t == 0) { sh.piv[j] = pos; sh.nz[j] = rank > 2; }
+    if (t < w) {   // the interchange
+      const cT a = S[(long)j * lda + t], b = S[(long)pos * lda + t];
+      S[(long)j * lda + t] = b;
+      if (pos != j) S[(long)pos * lda + t] = a;
+    }
+    __syncthreads();
+    if (rank > 2) {
+      const cT rcp = ts_crcp<T>(S[(long)j * lda + j]);
+      for (int i = j + 1 + t; i < m; i += nt) {
+        const cT l = cmul<T>(S[(long)i * lda + j], rcp);
+        S[(long)i * lda + j] = l;
+        for (int c = j + 1; c < w; ++c) {
+          const cT u = S[(long)j * lda + c], y = S[(long)i * lda + c];
+          S[(long)i * lda + c] = cT{fma(-l.x, u.x, fma(l.y, u.y, y.x)), fma(-l.x, u.y, fma(-l.y, u.x, y.y))};
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Everybody here? (one wave) Announces workgroup g with `tag` in the words `at`
+// and waits for the others; returns 1 (go on), 0 (leave) or -1 (do the strip
+// alone).
+__device__ __forceinline__ int st_rendezvous(int g, int G, unsigned tag, st_u64 *at, int *state, st_u64 limit) {
+  const int lane = threadIdx.x & 63;
+  if (lane == 0) st_store(at + g, tag);
+  const st_u64 t0 = wall_clock64();
+  bool late = false;
+  for (int c = lane; c < G; c += 64)
+    while (!late && st_load(at + c) != tag) late = wall_clock64() - t0 > limit;
+  const bool stop = __ballot(late) != 0;
+  int seen = 0;
+  if (lane == 0 && __hip_atomic_compare_exchange_strong(state, &seen, stop ? ST_ALONE : ST_GO, __ATOMIC_RELAXED,
+                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    seen = stop ? -1 : ST_GO;
+  seen = __builtin_amdgcn_readfirstlane(seen);
+  return seen == ST_ALONE ? 0 : seen;
+}
+
+// One column's exchange (one wave, all lanes; its candidate's words are on
+// their way): the reciprocal and row `own` to memory, everybody's candidates, and
+// the reciprocal and the chunk's entries of the winner's row to rcp and prow;
+// rank, p and the result become the winner's rank, position and workgroup.
+template <class T>
+__device__ __forceinline__ int st_exchange(int g, int G, unsigned tag, const st_u64 *cw, st_u64 *rw,
+                                           const typename C2<T>::t &orcp, const typename C2<T>::t *own,
+                                           typename C2<T>::t &rcp, typename C2<T>::t *prow, st_u64 &rank, int &p) {
+  constexpr int NW = st_words<T>(), EW = st_ew<T>();
+  const int lane = threadIdx.x & 63;
+  const st_u64 hi = (st_u64)tag << 32;
+  // reciprocal and chunk first
+  if (lane < EW) st_store(rw + g * NW + lane, hi | reinterpret_cast<const unsigned *>(&orcp)[lane]);
+#pragma unroll
+  for (int e = 0; e < PW_ * EW / 64; ++e)
+    st_store(rw + g * NW + EW + 64 * e + lane, hi | reinterpret_cast<const unsigned *>(own)[64 * e + lane]);
+  st_u64 best = 0;
+  int bp = 0x3fffff, bg = 0;
+  for (int c = lane; c < G; c += 64) {
+    st_u64 r2;
+    int p2;
+    while (!st_unpack(tag, st_load(cw + 2 * c), st_load(cw + 2 * c + 1), r2, p2)) {}
+    if (st_before(r2, p2, best, bp)) { best = r2; bp = p2; bg = c; }
+  }
+  const int bl = st_wave_best<sizeof(T) == 8>(best, bp);
+  bg = __builtin_amdgcn_readlane(bg, bl);
+  if (lane < 5 * EW) {
+    st_u64 v;
+    do v = st_load(rw + bg * NW + lane); while ((unsigned)(v >> 32) != tag);
+    unsigned *to = lane < EW ? reinterpret_cast<unsigned *>(&rcp) + lane : reinterpret_cast<unsigned *>(prow) + lane - EW;
+    *to = (unsigned)v;
+  }
+  rank = best;
+  p = bp;
+  return bg;
+}
+
+// Transposes four registers against the four rows of 16 lanes: v[a] of lane
+// (rq, b) becomes v[b] of lane (rq, a).
+__device__ __forceinline__ void st_transpose(unsigned (&v)[4]) {
+  const auto a = __builtin_amdgcn_permlane16_swap(v[0], v[1], false, false);   // odd rows of the first <-> even of the second
+  const auto b = __builtin_amdgcn_permlane16_swap(v[2], v[3], false, false);
+  const auto c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);   // upper half of the first <-> lower of the second
+  const auto d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+  v[0] = c[0];
+  v[1] = d[0];
+  v[2] = c[1];
+  v[3] = d[1];
+}
+__device__ __forceinline__ void st_transpose(float (&v)[4]) {
+  unsigned u[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) u[c] = __float_as_uint(v[c]);
+  st_transpose(u);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) v[c] = __uint_as_float(u[c]);
+}
+__device__ __forceinline__ void st_transpose(double (&v)[4]) {
+  unsigned lo[4], hi[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const st_u64 b = (st_u64)__double_as_longlong(v[c]);
+    lo[c] = (unsigned)b;
+    hi[c] = (unsigned)(b >> 32);
+  }
+  st_transpose(lo);
+  st_transpose(hi);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) v[c] = __longlong_as_double((long long)(((st_u64)hi[c] << 32) | lo[c]));
+}
+// of four values, the lane's own
+template <class T> __device__ __forceinline__ T st_own4(int cq, T a, T b, T c, T d) {
+  const T e = (cq & 1) ? b : a, f = (cq & 1) ? d : c;
+  return (cq & 2) ? f : e;
+}
+
+// Rows never move: each thread follows its row's position (the interchanges of
+// zgetrf as integers) and the rows are stored there at the end.
+template <class T>
+__global__ __launch_bounds__(st_w<T>() * 64, 2) void k_strip(int n, int c0, int w, typename C2<T>::t *A, long lda,
+                                                             long sA, char *ws, long sW, st_u64 limit, int *ipiv,
+                                                             long sP, int *info) {
+  typedef typename C2<T>::t cT;
+  typedef typename MF<T>::acc acc_t;
+  constexpr bool WIDE = sizeof(T) == 8;
+  constexpr int RT = ST_RT, NW = st_words<T>(), W = st_w<T>();
+  static_assert(RT == 4, "a tile per row of lanes in a chunk");
+  __shared__ StShared<T> sh;
+  const int z = blockIdx.z, g = blockIdx.x, G = gridDim.x, t = threadIdx.x, lane = t & 63, rq = lane & 15, cq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   A += (long)z * sA;
   char *wz = ws + (long)z * sW;
-  ipiv += (long)z * sP;
-  info += z;
-  cT *prow = reinterpret_cast<cT *>(wz + PP_PROW), *trow = reinterpret_cast<cT *>(wz + PP_TROW);
-  int *piv = reinterpret_cast<int *>(wz + PP_PIV), *nz = reinterpret_cast<int *>(wz + PP_NZ);
-  double *part_m = reinterpret_cast<double *>(wz + PP_PART);
-  int *part_r = reinterpret_cast<int *>(wz + pp_part_row_off(G));
-  int *cnt = reinterpret_cast<int *>(wz + PP_CNT);
-  const int s = j - 1, r = c0 + s;
-  int p = -1;
-  bool pnz = false;
-  cT pk = cT{0, 0}, tk = cT{0, 0}, rcp = cT{0, 0};
-  if (j > 0) {
-    p = piv[s];
-    pnz = nz[s] != 0;
-    if (k < w) { pk = prow[k]; tk = trow[k]; }
-    if (pnz) rcp = cdiv<T>(cT{1, 0}, prow[s]);
+  st_u64 *gcand = reinterpret_cast<st_u64 *>(wz + st_cand_off(n)), *grow = reinterpret_cast<st_u64 *>(wz + st_row_off<T>(n));
+  const int m = n - c0, row0 = g * st_rows<T>() + wave * 16 * RT;
+  int pos = row0 + lane;             // of row rq of tile cq
+  bool live = pos < m;
+  unsigned el = 0;                   // the chunk's steps that eliminated the row
+  // register q at chunk i is column 4 ((i + q) % 8) + cq: rotated by one per chunk,
+  // so that all indices are compile-time and one body serves every chunk
+  acc_t xr[RT][2], xi[RT][2];
+#pragma unroll
+  for (int T_ = 0; T_ < RT; ++T_) {
+    // rows past the last and columns past the strip repeat the last one (never chosen, never stored)
+    const cT *row = A + (long)(c0 + min(row0 + 16 * T_ + rq, m - 1)) * lda + c0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const cT v = row[min(4 * i + cq, w - 1)];
+      xr[T_][i / 4][i % 4] = v.x;
+      xi[T_][i / 4][i % 4] = v.y;
+    }
   }
-  double best = -1.0;
-  int bestrow = 0x7fffffff;
-  for (int q = 0; q < PP_ROWS / 8; ++q) {
-    const int i = c0 + g * PP_ROWS + q * 8 + rr;   // uniform per 32-lane group
-    const bool inrow = i < n;
-    cT x = (inrow && k < w) ? A[(long)i * lda + c0 + k] : cT{0, 0};
-    if (j > 0) {
-      if (i == r) x = pk;            // the pivot row moves to the top
-      else if (i == p) x = tk;       // the old top row takes its place
-      const T xs_re = __shfl(x.x, s, 32), xs_im = __shfl(x.y, s, 32);
-      if (i > r && pnz) {
-        const cT l = cmul<T>(cT{xs_re, xs_im}, rcp);
-        if (k == s) x = l;
-        else if (k > s) x = cT{x.x - (l.x * pk.x - l.y * pk.y), x.y - (l.x * pk.y + l.y * pk.x)};
+  if (G > 1) {
+    if (wave == 0)
+      sh.state = st_rendezvous(g, G, (unsigned)c0 + 1u, reinterpret_cast<st_u64 *>(wz + st_meet_off<T>(n)),
+                               reinterpret_cast<int *>(wz + ST_STATE) + c0 / PW_, limit);
+    __syncthreads();
+    const int st = sh.state;
+    if (st != ST_GO) {
+      if (st == -1) {
+        st_alone<T>(m, w, A + (long)c0 * lda + c0, lda, sh);
+        if (t == 0) st_pivots(c0, w, sh.piv, sh.nz, wz, ipiv + (long)z * sP, info + z);
       }
-      if (inrow && k < w && i >= r) A[(long)i * lda + c0 + k] = x;
+      return;
     }
-    if (j < w && inrow && k == j && i >= c0 + j) pp_better(best, bestrow, (double)(fabs(x.x) + fabs(x.y)), i);
   }
-  __shared__ double sm[4];
-  __shared__ int sr[4];
-  __shared__ int last;
-  pp_reduce_wg(best, bestrow, sm, sr);
-  if (t == 0) { part_m[g] = best; part_r[g] = bestrow; }
-  __threadfence();   // release: this workgroup's rows and partial maximum
-  if (t == 0) last = (atomicAdd(cnt, 1) == G - 1);
-  __syncthreads();
-  if (!last) return;
-  __threadfence();   // acquire: every other workgroup's rows and partial maxima
-  if (j < w) {
-    best = -1.0;
-    bestrow = 0x7fffffff;
-    for (int q = t; q < G; q += blockDim.x) pp_better(best, bestrow, part_m[q], part_r[q]);
-    __syncthreads();   // sm/sr reused
-    pp_reduce_wg(best, bestrow, sm, sr);
-    if (bestrow < c0 + j || bestrow >= n) { bestrow = c0 + j; best = 0.0; }   // no comparable candidate (NaN column)
-    if (t == 0) {
-      piv[j] = bestrow;
-      nz[j] = best > 0.0;
-      ipiv[c0 + j] = bestrow + 1;
-      if (!(best > 0.0) && *info == 0) *info = c0 + j + 1;
+  T ya[4], yb[4];   // the row's entries in the chunk: column 4 i + (k + c) % 4 in [c] at step k
+#pragma unroll 1
+  for (int j = 0; j < PW_; ++j) {
+    const int k = j & 3, i = j >> 2;
+    if (k == 0) {   // a new chunk
+      el = 0;
+#pragma unroll
+      for (int T_ = 0; T_ < RT; ++T_) { ya[T_] = xr[T_][0][0]; yb[T_] = xi[T_][0][0]; }
+      st_transpose(ya);
+      st_transpose(yb);
     }
-    if (t < w) prow[t] = A[(long)bestrow * lda + c0 + t];
-    else if (t >= 32 && t - 32 < w) trow[t - 32] = A[(long)(c0 + j) * lda + c0 + t - 32];
+    const int open = 4 - k;   // [0..open-1] are columns j.. of the chunk
+    bool nz = false;
+    cT P[4], rcp = cT{0, 0};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) P[c] = cT{0, 0};
+    if (j < w) {   // uniform
+      const int par = j & 1;
+      st_u64 rank = st_rank<T>(live, cT{ya[0], yb[0]});
+      int p = pos;
+      const int wl = st_wave_best<WIDE>(rank, p);
+      if (lane == 0) { sh.rank[par][wave] = rank; sh.pos[par][wave] = p; }
+      // each row's reciprocal, in case it is chosen: made while the waves meet
+      const bool some = ya[0] != 0 || yb[0] != 0;
+      const cT own_rcp = some ? ts_crcp<T>(cT{ya[0], yb[0]}) : cT{0, 0};
+      __syncthreads();
+      int bw = 0;   // the waves' best
+      rank = sh.rank[par][0];
+      p = sh.pos[par][0];
+#pragma unroll
+      for (int v = 1; v < W; ++v)
+        if (st_before(sh.rank[par][v], sh.pos[par][v], rank, p)) { rank = sh.rank[par][v]; p = sh.pos[par][v]; bw = v; }
+      const bool mine = wave == __builtin_amdgcn_readfirstlane(bw);
+      // the row beyond the chunk (needed at the chunk's end only)
+      auto hand_rest = [&](cT *own) {
+        if (rq == (wl & 15)) {
+#pragma unroll
+          for (int T_ = 0; T_ < RT; ++T_)
+            if (T_ == (wl >> 4)) {   // uniform
+#pragma unroll
+              for (int q = 1; q < 8; ++q) own[4 * q + cq] = cT{xr[T_][q / 4][q % 4], xi[T_][q / 4][q % 4]};
+            }
+        }
+      };
+      if (mine) {   // its wave hands it on
+        const unsigned tag = (unsigned)((c0 + j) % 0x1fffff) + 1u;
+        st_u64 *cw = gcand + par * G * 2;
+        if (G > 1) {
+          st_u64 wa, wb;
+          st_pack(tag, rank, p, wa, wb);
+          if (lane < 2) st_store(cw + 2 * g + lane, lane ? wb : wa);
+        }
+        cT *own = G > 1 ? sh.own : sh.urow[k];
+        if (lane == wl) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) own[(k + c) & 3] = cT{ya[c], yb[c]};
+          if (G > 1) sh.orcp = own_rcp;
+          else sh.rcp[k] = own_rcp;
+        }
+        if (G > 1) {
+          hand_rest(own);
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the row, across the wave's lanes
+          __builtin_amdgcn_wave_barrier();
+          const int from = st_exchange<T>(g, G, tag, cw, grow + ((i & 1) * 4 + k) * G * NW, sh.orcp, sh.own, sh.rcp[k],
+                                          sh.urow[k], rank, p);
+          if (lane == 0) { sh.prank = rank; sh.ppos = p; sh.from[k] = from; }
+        }
+      }
+      __syncthreads();
+      if (G == 1 && mine) hand_rest(sh.urow[k]);
+      if (G > 1) {
+        rank = sh.prank;
+        p = sh.ppos;
+      }
+      nz = rank > 2;   // uniform
+      if (t == 0) { sh.piv[j] = p; sh.nz[j] = nz; }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) P[c] = sh.urow[k][(k + c) & 3];
+      rcp = sh.rcp[k];
+      const bool chosen = live && pos == p;
+      if (live && pos == j) pos = p;   // the top row takes the pivot's place
+      if (chosen) { live = false; pos = j; }
+    }
+    {   // the step in the chunk, as a rotation by one
+      const bool e = live && nz;
+      const T a0 = ya[0], b0 = yb[0];
+      const cT l = cmul<T>(cT{a0, b0}, rcp);
+#pragma unroll
+      for (int c = 1; c < 4; ++c) {
+        const T fa = fma(-l.x, P[c].x, fma(l.y, P[c].y, ya[c])), fb = fma(-l.x, P[c].y, fma(-l.y, P[c].x, yb[c]));
+        ya[c - 1] = (e && c < open) ? fa : ya[c];
+        yb[c - 1] = (e && c < open) ? fb : yb[c];
+      }
+      ya[3] = e ? l.x : a0;
+      yb[3] = e ? l.y : b0;
+      if (e) el |= 1u << k;
+    }
+    if (k == 3) {
+      T ma[4], mb[4];   // the row's multipliers, zero where it was not eliminated; then the lane's operands
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        ma[c] = ((el >> c) & 1) ? ya[c] : T(0);
+        mb[c] = ((el >> c) & 1) ? yb[c] : T(0);
+      }
+      st_transpose(ya);
+      st_transpose(yb);
+      if (j + 1 < w) {   // the columns beyond: x -= (multipliers) (U rows)
+        if (__ballot(el != 15u) == 0) {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) { ma[c] = ya[c]; mb[c] = yb[c]; }
+        } else {
+          st_transpose(ma);
+          st_transpose(mb);
+        }
+        if (G > 1 && wave < 4) {
+          const unsigned tag = (unsigned)((c0 + 4 * i + wave) % 0x1fffff) + 1u;
+          const st_u64 *src = grow + (((i & 1) * 4 + wave) * G + sh.from[wave]) * NW + st_ew<T>();
+#pragma unroll
+          for (int e = 0; e < PW_ * st_ew<T>() / 64; ++e) {
+            st_u64 v;
+            do v = st_load(src + 64 * e + lane); while ((unsigned)(v >> 32) != tag);
+            reinterpret_cast<unsigned *>(sh.urow[wave])[64 * e + lane] = (unsigned)v;
+          }
+        }
+        __syncthreads();
+        // U rows by substitution with the pivot rows' multipliers, each lane for
+        // one column of each half and one row (cq)
+        cT L[6];
+#pragma unroll
+        for (int s = 0, e = 0; s < 3; ++s)
+#pragma unroll
+          for (int r = s + 1; r < 4; ++r, ++e) {
+            const cT v = sh.urow[r][s];
+            L[e] = sh.nz[4 * i + s] ? v : cT{0, 0};   // (1,0) (2,0) (3,0) (2,1) (3,1) (3,2)
+          }
+        // the lane's operand row rq of a product: register rq / 4 of lanes with cq =
+        // rq % 4 (FP64), register rq % 4 of lanes with cq = rq / 4 (FP32)
+        const int oq = WIDE ? rq >> 2 : rq & 3, oc = WIDE ? rq & 3 : rq >> 2;
+        T ur[2], ui[2];
+        bool odd = false;   // a value that is no finite number takes part
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) {
+          cT u[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) u[r] = sh.urow[r][4 * (4 * ct + oq) + oc];
+          auto sub = [](cT a, cT l, cT b) {
+            return cT{fma(-l.x, b.x, fma(l.y, b.y, a.x)), fma(-l.x, b.y, fma(-l.y, b.x, a.y))};
+          };
+          u[1] = sub(u[1], L[0], u[0]);
+          u[2] = sub(sub(u[2], L[1], u[0]), L[3], u[1]);
+          u[3] = sub(sub(sub(u[3], L[2], u[0]), L[4], u[1]), L[5], u[2]);
+          const bool use = 4 * ct + oq > 0 && i + 4 * ct + oq < 8 && sh.nz[4 * i + cq];   // an open column
+          ur[ct] = use ? st_own4(cq, u[0].x, u[1].x, u[2].x, u[3].x) : T(0);
+          ui[ct] = use ? st_own4(cq, u[0].y, u[1].y, u[2].y, u[3].y) : T(0);
+          odd |= !(fabs(ur[ct]) + fabs(ui[ct]) < T(INFINITY));
+        }
+#pragma unroll
+        for (int T_ = 0; T_ < RT; ++T_) odd |= !(fabs(ma[T_]) + fabs(mb[T_]) < T(INFINITY));
+        if (__ballot(odd)) {
+          // With an infinity or NaN about, a product with zero is not nothing: such
+          // factors become zero, and NaN goes to the entries they reach, which a
+          // product of zeros and ones finds (a step that eliminates the row, times a
+          // bad U entry; a bad multiplier, times an open column).
+          unsigned es[4] = {el & 1u, (el >> 1) & 1u, (el >> 2) & 1u, (el >> 3) & 1u};
+          st_transpose(es);
+#pragma unroll
+          for (int ct = 0; ct < 2; ++ct) {
+            const bool bad = !(fabs(ur[ct]) + fabs(ui[ct]) < T(INFINITY));
+            const T one = (4 * ct + oq > 0 && i + 4 * ct + oq < 8) ? T(1) : T(0);
+#pragma unroll
+            for (int T_ = 0; T_ < RT; ++T_) {
+              const bool badl = !(fabs(ma[T_]) + fabs(mb[T_]) < T(INFINITY));
+              acc_t hit = acc_t{0, 0, 0, 0};
+              hit = MF<T>::mma(bad ? T(1) : T(0), es[T_] ? T(1) : T(0), hit);
+              hit = MF<T>::mma(one, badl ? T(1) : T(0), hit);
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if (hit[e] > 0) xr[T_][ct][e] = xi[T_][ct][e] = T(NAN);
+            }
+            if (bad) ur[ct] = ui[ct] = 0;
+          }
+#pragma unroll
+          for (int T_ = 0; T_ < RT; ++T_)
+            if (!(fabs(ma[T_]) + fabs(mb[T_]) < T(INFINITY))) ma[T_] = mb[T_] = 0;
+        }
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct) {
+          if (ct == 1 && i >= 4) continue;   // finished columns (uniform)
+#pragma unroll
+          for (int T_ = 0; T_ < RT; ++T_) {
+            xr[T_][ct] = MF<T>::mma(-ur[ct], ma[T_], xr[T_][ct]);
+            xi[T_][ct] = MF<T>::mma(-ui[ct], ma[T_], xi[T_][ct]);
+          }
+#pragma unroll
+          for (int T_ = 0; T_ < RT; ++T_) {
+            xr[T_][ct] = MF<T>::mma(ui[ct], mb[T_], xr[T_][ct]);
+            xi[T_][ct] = MF<T>::mma(-ur[ct], mb[T_], xi[T_][ct]);
+          }
+        }
+      }
+      // the finished chunk goes behind the others; the pins keep the rotation in
+      // place (as a parallel move it took a second set of registers)
+#pragma unroll
+      for (int T_ = 0; T_ < RT; ++T_) {
+#pragma unroll
+        for (int q = 0; q < 7; ++q) {
+          xr[T_][q / 4][q % 4] = xr[T_][(q + 1) / 4][(q + 1) % 4];
+          xi[T_][q / 4][q % 4] = xi[T_][(q + 1) / 4][(q + 1) % 4];
+        }
+        xr[T_][1][3] = ya[T_];
+        xi[T_][1][3] = yb[T_];
+        asm("" : "+v"(xr[T_][0]), "+v"(xr[T_][1]), "+v"(xi[T_][0]), "+v"(xi[T_][1]));
+      }
+    }
   }
-  if (t == 0) *cnt = 0;
+  unsigned at[4] = {(unsigned)pos, (unsigned)pos, (unsigned)pos, (unsigned)pos};
+  st_transpose(at);   // [T] = the position of row rq of tile T
+#pragma unroll
+  for (int T_ = 0; T_ < RT; ++T_)
+    if (row0 + 16 * T_ + rq < m) {
+      cT *row = A + (long)(c0 + (int)at[T_]) * lda + c0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (4 * i + cq < w) row[4 * i + cq] = cT{xr[T_][i / 4][i % 4], xi[T_][i / 4][i % 4]};
+    }
+  if (g == 0 && t == 0) st_pivots(c0, w, sh.piv, sh.nz, wz, ipiv + (long)z * sP, info + z);
 }
 
 template <class T>
@@ -871,7 +1332,7 @@ __global__ __launch_bounds__(256) void k_pp_finish(int n, int c0, int w, const t
   A += (long)z * sA;
   char *wz = ws + (long)z * sW;
   char *fin = wz + finoff;
-  const int *piv = reinterpret_cast<const int *>(wz + PP_PIV);
+  const int *piv = reinterpret_cast<const int *>(wz + ST_PIV);
   cT *lu = reinterpret_cast<cT *>(fin);
   int *lfrom = reinterpret_cast<int *>(fin + PW_ * PW_ * sizeof(cT));
   int *lto = lfrom + 2 * PW_;
@@ -1285,7 +1746,7 @@ static size_t whole_cu_lds(const void *fn) {
 }
 template <class T>
 struct WholeCu {   // dynamic-LDS requests of the strip kernels for whole-CU launches
-  size_t local, merge, apply, gemm_assign, gemm_sub;
+  size_t local, merge, apply, gemm_assign, gemm_sub, strip;
 };
 template <class T>
 static const WholeCu<T> &whole_cu() {
@@ -1297,6 +1758,7 @@ static const WholeCu<T> &whole_cu() {
     w.apply = whole_cu_lds((const void *)k_ts_apply<T>);
     w.gemm_assign = std::max(whole_cu_lds((const void *)k_gemm_cu<T, true>), gcu_lds<T>());
     w.gemm_sub = std::max(whole_cu_lds((const void *)k_gemm_cu<T, false>), gcu_lds<T>());
+    w.strip = whole_cu_lds((const void *)k_strip<T>);
   });
   return w;
 }
@@ -1344,7 +1806,7 @@ static size_t getrf_ws_bytes(int n, int batch) {
 template <class T>
 static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long sA, int *ipiv, long sP,
                           int *perm, int *dinfo, hipStream_t s, char *ws = nullptr, bool lookahead = true,
-                          bool own_gemm = false, bool pp = false) {
+                          bool own_gemm = false, bool pp = false, st_u64 wait = ST_LIMIT) {
   typedef typename C2<T>::t cT;
   constexpr int PW = PanelW<T>::W;
   const dim3 b256(256);
@@ -1373,14 +1835,15 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
   // The strips of the outer block [k0, k0 + nb): tournament, interchanges on
   // the block's own columns, L21, then the block's remaining columns by TRSM
   // and the rank-w update. Touches only the block's columns (rows >= k0).
-  if (pp && pp_ws_bytes(n) > 2 * (long)Gmax * setb)
+  if (pp && st_ws_bytes<T>(n) > 2 * (long)Gmax * setb)
     qpms_hip_die(__FILE__, __LINE__, __func__, "partial-pivoting workspace does not fit (order %d)", n);
-  if (pp) QH_LAUNCH(k_pp_init, dim3(batch), dim3(1), 0, s, ws, sW);
-  // partial pivoting: the strip in place, column by column, then its slot
-  auto pp_strip = [&](int c0, int w, hipStream_t st) {
-    const int G = (n - c0 + PP_ROWS - 1) / PP_ROWS;
-    for (int j = 0; j <= w; ++j)
-      QH_LAUNCH(k_pp_step<T>, dim3(G, 1, batch), b256, 0, st, n, c0, w, j, A, lda, sA, ws, sW, ipiv, sP, dinfo);
+  if (pp)
+    QH_LAUNCH(k_strip_init, dim3((unsigned)std::min((st_ws_bytes<T>(n) / 8 + 255) / 256, 1024L), 1, batch), b256, 0, s,
+              ws, sW, st_ws_bytes<T>(n));
+  // partial pivoting: the strip in place, then its slot
+  auto pp_strip = [&](int c0, int w, hipStream_t st, bool wcu) {
+    QH_LAUNCH(k_strip<T>, dim3(st_groups<T>(n - c0), 1, batch), dim3(st_w<T>() * 64), wcu ? whole_cu<T>().strip : 0, st, n,
+              c0, w, A, lda, sA, ws, sW, wait, ipiv, sP, dinfo);
     QH_LAUNCH(k_pp_finish<T>, dim3(1, 1, batch), b256, PP_FIN_LDS, st, n, c0, w, A, lda, sA, ws, sW,
               (long)(fin0 - ws) + (long)((c0 % LU_NB) / PW) * finb, perm, sP);
   };
@@ -1393,7 +1856,7 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
       const int w = min(PW, nb - j0), c0 = k0 + j0;
       char *fin = fin0 + (long)(j0 / PW) * finb;
       if (pp) {   // the strip factored in place (L21 included); interchanges on the block's other columns
-        pp_strip(c0, w, st);
+        pp_strip(c0, w, st, wcu);
         if (c0 > k0)
           QH_LAUNCH(k_ts_apply<T>, dim3((c0 - k0 + AP_COLS - 1) / AP_COLS, 1, batch), b256, l_apply, st, n, c0, w, A,
                     lda, sA, fin, sW, k0, c0);
@@ -1488,7 +1951,10 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
       const int nb1 = min(LU_NB, nr);
       trailing_gemm<T>(nr, nb1, nb, batch, A + (long)(k0 + nb) * lda + k0, lda, sA, A + (long)k0 * lda + k0 + nb, lda,
                        sA, A + (long)(k0 + nb) * lda + k0 + nb, lda, sA, s, own_gemm);
-      const bool split = la && nr > nb1;
+      // A strip's workgroups wait for each other, so each needs one of the CUs kept
+      // free for it: beside the update on a shared CU the slowest held all of them up
+      // (order 9216: 1.8 ms for the first strip of a block, 0.1 ms alone).
+      const bool split = la && nr > nb1 && !(pp && st_groups<T>(nr) > lu_reserve_cus());
       if (nr > nb1) {
         hipStream_t sg = split ? side : s;
         if (split) {
@@ -1836,6 +2302,20 @@ extern "C" int qpms_hip_zgetrf_dev(size_t n, _Complex double *A_dev, int *ipiv_d
   HIPCHK(hipStreamSynchronize(s));
   qh_dfree(dinfo);
   return info;
+}
+
+// The partial-pivoting LU of one FP64 or FP32 (prec 64, 32) matrix with the
+// strips' wait for their workgroups as an argument (clock ticks; 0: a strip of
+// several workgroups is left to the first one that does not see the others at
+// once). info: a device word. Tests reach both ways through a strip with it.
+extern "C" int qh_getrf_pp(int prec, int n, double *A, int *ipiv, int *info, unsigned long long wait, void *stream) {
+  hipStream_t s = (hipStream_t)qh_stream(stream);
+  qh_zero(info, sizeof(int), s);
+  if (prec == 32)
+    getrf_batched<float>(n, 1, (v2f *)A, n, 0, ipiv, 0, nullptr, info, s, nullptr, true, false, true, wait);
+  else
+    getrf_batched<double>(n, 1, (v2d *)A, n, 0, ipiv, 0, nullptr, info, s, nullptr, true, false, true, wait);
+  return 0;
 }
 
 // ---------------------------------------------------------------------------
