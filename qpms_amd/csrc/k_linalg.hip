@@ -29,6 +29,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <algorithm>
+#include <type_traits>
 #include <mutex>
 #include <rocblas/rocblas.h>
 #include "qpms_internal.h"
@@ -357,11 +358,12 @@ constexpr int TS_SLOTS = 8;   // strips per outer block (LU_NB / PW)
 template <class T>
 struct PanelWS {
   static size_t set_bytes() { return ((size_t)PW_ * 4 + (size_t)PW_ * PW_ * sizeof(typename C2<T>::t) + 255) / 256 * 256; }
-  // slot: L11\U11, moved-row lists, then L11^{-1} and U11^{-1} (PW x PW each)
-  __host__ __device__ static constexpr size_t fin_inv_off() { return ((size_t)PW_ * PW_ * sizeof(typename C2<T>::t) + 4 * PW_ * 4 + 16 + 255) / 256 * 256; }
-  static size_t fin_bytes() { return fin_inv_off() + 2 * (size_t)PW_ * PW_ * sizeof(typename C2<T>::t); }
+  // slot of a strip: its interchanges (src[i], the strip row that ends as row i of
+  // the top PW; to[i], where row i of the top went), then (tournament) L11\U11 and
+  // U11^{-1}, PW x PW each
+  static constexpr size_t LU_OFF = 2 * PW_ * 4, UINV_OFF = LU_OFF + (size_t)PW_ * PW_ * sizeof(typename C2<T>::t);
+  static size_t fin_bytes() { return UINV_OFF + (size_t)PW_ * PW_ * sizeof(typename C2<T>::t); }
   static int sets(int n) { return (n + TsRows<T>::R - 1) / TsRows<T>::R; }
-  static size_t bytes(int n) { return (2 * (size_t)sets(n) * set_bytes() + TS_SLOTS * fin_bytes() + 255) / 256 * 256; }
 };
 
 // Workgroup state of the elimination: each wave's packed winner and winning
@@ -521,25 +523,23 @@ __device__ __forceinline__ int ts_gepp(typename C2<T>::t *X, int key, int w, TsS
   return ns;
 }
 
-// L11^{-1} (unit lower) and U11^{-1} (upper) of a strip's PW x PW L\U into
-// out (two PW x PW blocks, row-major), for the strip's L21 and U12 updates as
-// products. v: entries e = t + TS_THREADS q of L\U. PW right-looking steps
-// over both inverses at once (forward for L, backward for U), each entry
-// owned by one thread, one barrier per step, in the LDS of X (whose rows are
-// no longer needed). A zero diagonal entry of U is taken as one: the row's
-// L21 entry is then kept, as a zero pivot leaves it.
+// U11^{-1} of a strip's PW x PW L\U into out (row-major), for the strip's L21 as
+// a product. v: entries e = t + TS_THREADS q of L\U. PW backward right-looking
+// steps, each entry owned by one thread, one barrier per step, in the LDS of X
+// (whose rows are no longer needed). A zero diagonal entry of U is taken as one:
+// the row's L21 entry is then kept, as a zero pivot leaves it.
 template <class T>
-__device__ __forceinline__ void ts_tri_inverses(typename C2<T>::t *X, const typename C2<T>::t *v, char *out) {
+__device__ __forceinline__ void ts_u_inverse(typename C2<T>::t *X, const typename C2<T>::t *v, char *out) {
   typedef typename C2<T>::t cT;
-  constexpr int NE = PW_ * PW_ / TS_THREADS, PP = PW_ * PW_;
+  constexpr int PP = PW_ * PW_, NE = PP / TS_THREADS;
   const int t = threadIdx.x;
-  cT *LU = X, *Z = X + PP, *dinv = X + 3 * PP;   // Z: L^{-1}, then U^{-1} with unscaled rows
+  cT *LU = X, *Z = X + PP, *dinv = X + 2 * PP;   // Z: U^{-1} with unscaled rows
   __syncthreads();   // every read of X's rows is done
 #pragma unroll
   for (int q = 0; q < NE; ++q) {
-    const int e = t + TS_THREADS * q, i = e / PW_, c = e % PW_;
+    const int e = t + TS_THREADS * q;
     LU[e] = v[q];
-    Z[e] = Z[PP + e] = (i == c) ? cT{1, 0} : cT{0, 0};
+    Z[e] = (e / PW_ == e % PW_) ? cT{1, 0} : cT{0, 0};
   }
   __syncthreads();
   if (t < PW_) {
@@ -547,38 +547,28 @@ __device__ __forceinline__ void ts_tri_inverses(typename C2<T>::t *X, const type
     dinv[t] = (d.x == 0 && d.y == 0) ? cT{1, 0} : cdiv<T>(cT{1, 0}, d);
   }
   __syncthreads();
-  for (int s = 0; s < PW_; ++s) {
-    const int su = PW_ - 1 - s;
+  for (int s = PW_ - 1; s >= 0; --s) {   // rows above s take row s divided by its diagonal
 #pragma unroll
-    for (int q = 0; q < 2 * NE; ++q) {
-      const int e = t + TS_THREADS * q;
-      if (e < PP) {   // L: rows below s take row s
-        const int i = e / PW_, c = e % PW_;
-        if (i > s) {
-          const cT l = LU[i * PW_ + s], z = Z[s * PW_ + c];
-          Z[e] = cT{Z[e].x - (l.x * z.x - l.y * z.y), Z[e].y - (l.x * z.y + l.y * z.x)};
-        }
-      } else {        // U: rows above su take row su divided by its diagonal
-        const int f = e - PP, i = f / PW_, c = f % PW_;
-        if (i < su) {
-          const cT u = cmul<T>(LU[i * PW_ + su], dinv[su]), z = Z[PP + su * PW_ + c];
-          Z[e] = cT{Z[e].x - (u.x * z.x - u.y * z.y), Z[e].y - (u.x * z.y + u.y * z.x)};
-        }
+    for (int q = 0; q < NE; ++q) {
+      const int e = t + TS_THREADS * q, i = e / PW_, c = e % PW_;
+      if (i < s) {
+        const cT u = cmul<T>(LU[i * PW_ + s], dinv[s]), z = Z[s * PW_ + c];
+        Z[e] = cT{Z[e].x - (u.x * z.x - u.y * z.y), Z[e].y - (u.x * z.y + u.y * z.x)};
       }
     }
     __syncthreads();
   }
   cT *o = reinterpret_cast<cT *>(out);
 #pragma unroll
-  for (int q = 0; q < 2 * NE; ++q) {
+  for (int q = 0; q < NE; ++q) {
     const int e = t + TS_THREADS * q;
-    o[e] = (e < PP) ? Z[e] : cmul<T>(Z[e], dinv[(e - PP) / PW_]);
+    o[e] = cmul<T>(Z[e], dinv[e / PW_]);
   }
 }
 
 // Output of the last tournament level: L11\U11 rows, ipiv (1-based, matrix
-// rows), perm, info, and the compacted list of (from, to) strip rows the
-// interchanges move. The list starts as the w top rows; each interchange
+// rows), perm, info, U11^{-1}, and where the interchanges take rows from and
+// to, from a list of the rows they touch. The list starts as the w top rows; each interchange
 // i <-> p is applied to it with wave ballots (a row not yet listed sits at
 // its own index).
 template <class T>
@@ -587,10 +577,8 @@ __device__ __forceinline__ void ts_finish(typename C2<T>::t *X, int ns, int w, i
   typedef typename C2<T>::t cT;
   constexpr int XS = TsStride<T>::XS, NE = PW_ * PW_ / TS_THREADS;
   const int t = threadIdx.x;
-  cT *lu = reinterpret_cast<cT *>(fin);
-  int *lfrom = reinterpret_cast<int *>(fin + PW_ * PW_ * sizeof(cT));
-  int *lto = lfrom + 2 * PW_;
-  int *lcount = lto + 2 * PW_;
+  cT *lu = reinterpret_cast<cT *>(fin + PanelWS<T>::LU_OFF);
+  int *src = reinterpret_cast<int *>(fin), *to = src + PW_;
   cT v[NE];   // entries t + TS_THREADS q of L11\U11
 #pragma unroll
   for (int q = 0; q < NE; ++q) {
@@ -624,17 +612,15 @@ __device__ __forceinline__ void ts_finish(typename C2<T>::t *X, int ns, int w, i
         if (sh.sval[i] == 0) z0 = c0 + i + 1;
       if (z0 && *info == 0) *info = z0;
     }
+    if (t < nlist && pos < w) src[pos] = id;
+    if (t < nlist && id < w) to[id] = pos;
     const bool mv = (t < nlist) && id != pos;
-    const unsigned long long mm = __ballot(mv);
-    const int slot = __popcll(mm & ((1ull << t) - 1ull));
-    if (mv) { lfrom[slot] = id; lto[slot] = pos; }
-    if (t == 0) *lcount = __popcll(mm);
     if (perm) {   // the moved rows as one gather: every lane loads before any stores
       const int pv = mv ? perm[c0 + id] : 0;
       if (mv) perm[c0 + pos] = pv;
     }
   }
-  ts_tri_inverses<T>(X, v, fin + PanelWS<T>::fin_inv_off());
+  ts_u_inverse<T>(X, v, fin + PanelWS<T>::UINV_OFF);
 }
 
 template <class T>
@@ -750,9 +736,7 @@ __global__ __launch_bounds__(TS_THREADS) void k_ts_merge(int c0, int w, int nin,
 // first row of largest |re| + |im| in column j at or below the diagonal, taken
 // in full double (or float) precision. One launch factors a whole strip: the
 // workgroups hold its rows in registers for all of its columns and agree on
-// each pivot through memory. k_pp_finish then writes the strip's slot (L11\U11,
-// the moved-row list, L11^{-1}, U11^{-1}) as the tournament's last level does,
-// so the rest of the LU is shared. L21 is left in place by the elimination.
+// each pivot through memory. L21 is left in place by the elimination.
 //
 // Layout. A wave holds RT tiles of 16 rows; lane (rq, cq) = (lane % 16,
 // lane / 16) holds row rq of each tile and columns 4 i + cq, i = 0..7: the
@@ -799,10 +783,9 @@ constexpr st_u64 ST_LIMIT = 10000000ull;   // ticks of the 100 MHz clock (0.1 s)
 // words of one row: the reciprocal of its pivot, then its entries
 template <class T> constexpr int st_ew() { return (int)sizeof(typename C2<T>::t) / 4; }
 template <class T> constexpr int st_words() { return (1 + PW_) * st_ew<T>(); }
-// Per-matrix workspace of the strips (in the tournament's candidate area,
-// unused here): the strip's pivots, a state word per strip, two sets of
+// Per-matrix workspace of the strips: a state word per strip, two sets of
 // candidates, the announcements, two sets of four rows per workgroup.
-constexpr long ST_PIV = 0, ST_STATE = 256;
+constexpr long ST_STATE = 0;
 constexpr long st_cand_off(int n) { return ST_STATE + ((long)((n + PW_ - 1) / PW_) * 4 + 255) / 256 * 256; }
 template <class T> constexpr int st_groups(int rows) { return (rows + st_rows<T>() - 1) / st_rows<T>(); }
 template <class T> constexpr long st_meet_off(int n) { return st_cand_off(n) + 2L * st_groups<T>(n) * 2 * 8; }
@@ -845,39 +828,42 @@ __device__ __forceinline__ unsigned st_dmax(unsigned v) {   // lanes without a s
   const unsigned o = (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, RM, 0xF, false);
   return o > v ? o : v;
 }
-// The lane of a wave with the largest rank, the smallest position among equal
-// ones; rank and pos become that lane's. One DPP chain on the ranks' leading 32
-// bits (FP32: all of them); lanes that tie there are compared one by one.
-template <bool WIDE>
-__device__ __forceinline__ int st_wave_best(st_u64 &rank, int &pos) {
-  const unsigned own = WIDE ? (unsigned)(rank >> 32) : (unsigned)rank;
-  unsigned v = own;
+__device__ __forceinline__ unsigned st_wave_max(unsigned v) {
   v = st_dmax<0xB1, 0xF>(v);    // quad_perm [1,0,3,2]
   v = st_dmax<0x4E, 0xF>(v);    // quad_perm [2,3,0,1]
   v = st_dmax<0x124, 0xF>(v);   // row_ror 4
   v = st_dmax<0x128, 0xF>(v);   // row_ror 8
   v = st_dmax<0x142, 0xA>(v);   // row_bcast 15
   v = st_dmax<0x143, 0xC>(v);   // row_bcast 31
-  const unsigned m = (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+// The lane of a wave with the largest rank, the smallest position among equal
+// ones; rank and pos become that lane's. One DPP chain on the ranks' leading 32
+// bits (FP32: all of them); only where lanes tie, one more for the other bits
+// and one for the positions (a flat cluster's matrix has many entries that are
+// exactly zero: taken one by one, their ties made a column three times as long).
+template <bool WIDE>
+__device__ __forceinline__ int st_wave_best(st_u64 &rank, int &pos) {
+  const unsigned lo = (unsigned)rank, hi = (unsigned)(rank >> 32), own = WIDE ? hi : lo;
+  const unsigned m = st_wave_max(own);
   st_u64 eq = __ballot(own == m && rank != 0);
   if (eq == 0) {   // no row in the wave
     rank = 0;
     return 0;
   }
-  int l = __ffsll((long long)eq) - 1;
-  const int lo = (int)(unsigned)rank, hi = (int)(rank >> 32);
-  auto rank_of = [&](int i) {
-    return ((st_u64)(unsigned)__builtin_amdgcn_readlane(hi, i) << 32) | (unsigned)__builtin_amdgcn_readlane(lo, i);
-  };
-  st_u64 r = rank_of(l);
-  int p = __builtin_amdgcn_readlane(pos, l);
-  for (eq &= eq - 1; eq; eq &= eq - 1) {   // uniform
-    const int l2 = __ffsll((long long)eq) - 1, p2 = __builtin_amdgcn_readlane(pos, l2);
-    const st_u64 r2 = rank_of(l2);
-    if (st_before(r2, p2, r, p)) { r = r2; p = p2; l = l2; }
+  bool in = own == m && rank != 0;
+  if (WIDE && (eq & (eq - 1))) {   // uniform
+    const unsigned m2 = st_wave_max(in ? lo : 0u);
+    in = in && lo == m2;
+    eq = __ballot(in);
   }
-  rank = r;
-  pos = p;
+  if (eq & (eq - 1)) {
+    const unsigned m3 = st_wave_max(in ? 0x7fffffffu - (unsigned)pos : 0u);
+    eq = __ballot(in && 0x7fffffffu - (unsigned)pos == m3);
+  }
+  const int l = __ffsll((long long)eq) - 1;
+  rank = ((st_u64)(unsigned)__builtin_amdgcn_readlane((int)hi, l) << 32) | (unsigned)__builtin_amdgcn_readlane((int)lo, l);
+  pos = __builtin_amdgcn_readlane(pos, l);
   return l;
 }
 
@@ -897,12 +883,9 @@ struct StShared {
   int state;
 };
 
-// The strip's pivots (strip rows piv, nz[i] = 0 for a zero one) to the
-// workspace, ipiv and info.
-__device__ __forceinline__ void st_pivots(int c0, int w, const int *piv, const int *nz, char *wz, int *ipiv, int *info) {
-  int *out = reinterpret_cast<int *>(wz + ST_PIV);
+// The strip's pivots (strip rows piv, nz[i] = 0 for a zero one) to ipiv and info.
+__device__ __forceinline__ void st_pivots(int c0, int w, const int *piv, const int *nz, int *ipiv, int *info) {
   for (int i = 0; i < w; ++i) {
-    out[i] = c0 + piv[i];
     ipiv[c0 + i] = c0 + piv[i] + 1;
     if (!nz[i] && *info == 0) *info = c0 + i + 1;
   }
@@ -1048,8 +1031,8 @@ template <class T> __device__ __forceinline__ T st_own4(int cq, T a, T b, T c, T
 // zgetrf as integers) and the rows are stored there at the end.
 template <class T>
 __global__ __launch_bounds__(st_w<T>() * 64, 2) void k_strip(int n, int c0, int w, typename C2<T>::t *A, long lda,
-                                                             long sA, char *ws, long sW, st_u64 limit, int *ipiv,
-                                                             long sP, int *info) {
+                                                             long sA, char *ws, long sW, long finoff, st_u64 limit,
+                                                             int *ipiv, long sP, int *info) {
   typedef typename C2<T>::t cT;
   typedef typename MF<T>::acc acc_t;
   constexpr bool WIDE = sizeof(T) == 8;
@@ -1060,10 +1043,12 @@ __global__ __launch_bounds__(st_w<T>() * 64, 2) void k_strip(int n, int c0, int 
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   A += (long)z * sA;
   char *wz = ws + (long)z * sW;
+  int *src = reinterpret_cast<int *>(wz + finoff), *moved_to = src + PW_;   // PanelWS's slot
   st_u64 *gcand = reinterpret_cast<st_u64 *>(wz + st_cand_off(n)), *grow = reinterpret_cast<st_u64 *>(wz + st_row_off<T>(n));
   const int m = n - c0, row0 = g * st_rows<T>() + wave * 16 * RT;
   int pos = row0 + lane;             // of row rq of tile cq
-  bool live = pos < m;
+  const bool live_row = pos < m;
+  bool live = live_row;
   unsigned el = 0;                   // the chunk's steps that eliminated the row
   // register q at chunk i is column 4 ((i + q) % 8) + cq: rotated by one per chunk,
   // so that all indices are compile-time and one body serves every chunk
@@ -1088,7 +1073,14 @@ __global__ __launch_bounds__(st_w<T>() * 64, 2) void k_strip(int n, int c0, int 
     if (st != ST_GO) {
       if (st == -1) {
         st_alone<T>(m, w, A + (long)c0 * lda + c0, lda, sh);
-        if (t == 0) st_pivots(c0, w, sh.piv, sh.nz, wz, ipiv + (long)z * sP, info + z);
+        if (t < w) {   // the interchanges followed forth from row t and back from place t
+          int f = t, b = sh.piv[t];
+          for (int i = 0; i < w; ++i) f = f == i ? sh.piv[i] : f == sh.piv[i] ? i : f;
+          for (int i = t - 1; i >= 0; --i) b = b == i ? sh.piv[i] : b == sh.piv[i] ? i : b;
+          moved_to[t] = f;
+          src[t] = b;
+        }
+        if (t == 0) st_pivots(c0, w, sh.piv, sh.nz, ipiv + (long)z * sP, info + z);
       }
       return;
     }
@@ -1318,77 +1310,35 @@ __global__ __launch_bounds__(st_w<T>() * 64, 2) void k_strip(int n, int c0, int 
       for (int i = 0; i < 8; ++i)
         if (4 * i + cq < w) row[4 * i + cq] = cT{xr[T_][i / 4][i % 4], xi[T_][i / 4][i % 4]};
     }
-  if (g == 0 && t == 0) st_pivots(c0, w, sh.piv, sh.nz, wz, ipiv + (long)z * sP, info + z);
+  if (live_row && pos < w) src[pos] = row0 + lane;
+  if (live_row && row0 + lane < w) moved_to[row0 + lane] = pos;
+  if (g == 0 && t == 0) st_pivots(c0, w, sh.piv, sh.nz, ipiv + (long)z * sP, info + z);
 }
-
-template <class T>
-__global__ __launch_bounds__(256) void k_pp_finish(int n, int c0, int w, const typename C2<T>::t *A, long lda,
-                                                   long sA, char *ws, long sW, long finoff, int *perm, long sP) {
-  typedef typename C2<T>::t cT;
-  constexpr int NE = PW_ * PW_ / 256;
-  extern __shared__ __align__(16) char smem_raw[];
-  cT *X = reinterpret_cast<cT *>(smem_raw);
-  const int z = blockIdx.z, t = threadIdx.x;
-  A += (long)z * sA;
-  char *wz = ws + (long)z * sW;
-  char *fin = wz + finoff;
-  const int *piv = reinterpret_cast<const int *>(wz + ST_PIV);
-  cT *lu = reinterpret_cast<cT *>(fin);
-  int *lfrom = reinterpret_cast<int *>(fin + PW_ * PW_ * sizeof(cT));
-  int *lto = lfrom + 2 * PW_;
-  int *lcount = lto + 2 * PW_;
-  cT v[NE];
-#pragma unroll
-  for (int q = 0; q < NE; ++q) {
-    const int e = t + 256 * q, i = e / PW_, c = e % PW_;
-    v[q] = (i < w && c < w) ? A[(long)(c0 + i) * lda + c0 + c] : cT{0, 0};
-    lu[e] = v[q];
-  }
-  if (t < 64) {   // the interchanges as a list of moved rows: lane entry (original strip row, current row)
-    int id = -1, pos = -1, nlist = 0;
-    for (int i = 0; i < w; ++i) {
-      const int pr = piv[i] - c0;
-      if (pr == i) continue;
-      if (!__ballot(pos == i)) { if (t == nlist) { id = i; pos = i; } ++nlist; }
-      if (!__ballot(pos == pr)) { if (t == nlist) { id = pr; pos = pr; } ++nlist; }
-      const bool at_i = pos == i, at_p = pos == pr;
-      if (at_i) pos = pr;
-      else if (at_p) pos = i;
-    }
-    const bool mv = (t < nlist) && id != pos;
-    const unsigned long long mm = __ballot(mv);
-    const int slot = __popcll(mm & ((1ull << t) - 1ull));
-    if (mv) { lfrom[slot] = id; lto[slot] = pos; }
-    if (t == 0) *lcount = __popcll(mm);
-    if (perm) {   // every lane loads before any stores
-      int *pz = perm + (long)z * sP;
-      const int pv = mv ? pz[c0 + id] : 0;
-      if (mv) pz[c0 + pos] = pv;
-    }
-  }
-  ts_tri_inverses<T>(X, v, fin + PanelWS<T>::fin_inv_off());
-}
-constexpr size_t PP_FIN_LDS = (size_t)(3 * PW_ * PW_ + PW_) * 16;   // ts_tri_inverses' area (FP64 size)
 
 // Row interchanges of strips as gathers A[c0 + to] = A[c0 + from] over their
 // moved rows, per block of AP_COLS columns: every moved entry is loaded into
 // registers, then (after a barrier) stored.
-//   k_ts_apply:  one strip (its slot `fin`), columns [col_lo, col_hi), then
-//                L11\U11 into the strip's top block;
+//   k_ts_apply:  a tournament strip on its own columns, then its L11\U11;
 //   k_ts_apply_defer: the strips of an outer block (slots 0..nslots-1, strip
 //                c0 = K0 + PW slot, in order) on every column outside
 //                [skip_lo, skip_hi).
 constexpr int AP_COLS = 32;
 template <class T>
 __device__ __forceinline__ void ts_gather(int n, int c0, const char *fin, typename C2<T>::t *A, long lda, int j0,
-                                          int *from, int *to, bool colok) {
+                                          int *from, int *to, int *count, bool colok) {
   typedef typename C2<T>::t cT;
   const int t = threadIdx.x;
-  const int *lfrom = reinterpret_cast<const int *>(fin + PW_ * PW_ * sizeof(cT));
-  const int *lto = lfrom + 2 * PW_;
-  const int k = lto[2 * PW_];
-  if (t < k) { from[t] = lfrom[t]; to[t] = lto[t]; }
+  if (t < 64) {   // lanes 0..31: what comes to the top; 32..63: what leaves it
+    const int *src = reinterpret_cast<const int *>(fin), *dst = src + PW_, w = min(PW_, n - c0), i = t & (PW_ - 1);
+    const int f = t < PW_ ? (i < w ? src[i] : i) : i, d = t < PW_ ? i : (i < w ? dst[i] : i);
+    const bool mv = t < PW_ ? f != d : d >= w && i < w;
+    const unsigned long long mm = __ballot(mv);
+    const int slot = __popcll(mm & ((1ull << t) - 1ull));
+    if (mv) { from[slot] = f; to[slot] = d; }
+    if (t == 0) *count = __popcll(mm);
+  }
   __syncthreads();
+  const int k = *count;
   const int c = t % AP_COLS, r4 = t / AP_COLS;
   constexpr int RP = 256 / AP_COLS, NQ = 2 * PW_ / RP;   // rows per pass; passes over the longest list
   cT v[NQ];
@@ -1407,33 +1357,203 @@ __device__ __forceinline__ void ts_gather(int n, int c0, const char *fin, typena
 }
 
 template <class T>
-__global__ __launch_bounds__(256) void k_ts_apply(int n, int c0, int w, typename C2<T>::t *A, long lda, long sA,
-                                                  const char *fin, long sW, int col_lo, int col_hi) {
+__global__ __launch_bounds__(256) void k_ts_apply(int n, int c0, int w, typename C2<T>::t *A, long lda, const char *fin) {
   typedef typename C2<T>::t cT;
-  __shared__ int from[2 * PW_], to[2 * PW_];
-  const int z = blockIdx.z, t = threadIdx.x, j0 = col_lo + blockIdx.x * AP_COLS;
-  A += (long)z * sA;
-  fin += (long)z * sW;
-  const int c = t % AP_COLS, r4 = t / AP_COLS;
-  const bool colok = j0 + c < col_hi;
-  ts_gather<T>(n, c0, fin, A, lda, j0, from, to, colok);
-  const cT *lu = reinterpret_cast<const cT *>(fin);
-  if (colok && j0 + c >= c0 && j0 + c < c0 + w)
-    for (int i = r4; i < w; i += 256 / AP_COLS) A[(long)(c0 + i) * lda + j0 + c] = lu[i * PW_ + (j0 + c - c0)];
+  __shared__ int from[2 * PW_], to[2 * PW_], count;
+  const int t = threadIdx.x, c = t % AP_COLS, r4 = t / AP_COLS;
+  const bool colok = c < w;
+  ts_gather<T>(n, c0, fin, A, lda, c0, from, to, &count, colok);
+  const cT *lu = reinterpret_cast<const cT *>(fin + PanelWS<T>::LU_OFF);
+  if (colok)
+    for (int i = r4; i < w; i += 256 / AP_COLS) A[(long)(c0 + i) * lda + c0 + c] = lu[i * PW_ + c];
 }
 
 template <class T>
 __global__ __launch_bounds__(256) void k_ts_apply_defer(int n, int K0, int nslots, typename C2<T>::t *A, long lda,
                                                         long sA, const char *fin0, long finb, long sW, int skip_lo,
                                                         int skip_hi) {
-  __shared__ int from[2 * PW_], to[2 * PW_];
+  __shared__ int from[2 * PW_], to[2 * PW_], count;
   const int z = blockIdx.z, j0 = blockIdx.x * AP_COLS;
   if (j0 >= skip_lo && j0 + AP_COLS <= skip_hi) return;   // whole block inside the skipped columns (uniform)
   A += (long)z * sA;
   fin0 += (long)z * sW;
   const int c = threadIdx.x % AP_COLS;
   const bool colok = j0 + c < n && (j0 + c < skip_lo || j0 + c >= skip_hi);
-  for (int q = 0; q < nslots; ++q) ts_gather<T>(n, K0 + PW_ * q, fin0 + q * finb, A, lda, j0, from, to, colok);
+  for (int q = 0; q < nslots; ++q) ts_gather<T>(n, K0 + PW_ * q, fin0 + q * finb, A, lda, j0, from, to, &count, colok);
+}
+
+// Forward substitution with a unit lower 32 x 32 block for the 16 columns of a
+// wave, four lanes per column (lane = 4 column + class): x[q] is row 4 q + class.
+// Each step's solved entry goes round its four lanes by DPP. The rolled loop
+// over groups of four rows keeps the group at hand in x[0] and hands it to
+// out(kb, value) when it is done. A thread per column instead has 496 dependent
+// updates in a row; a product with the inverse needs the inverse (26 us for the
+// launch that made it).
+// lane class K's value
+template <int K> __device__ __forceinline__ unsigned su_dpp(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, K * 0x55, 0xF, 0xF, true);
+}
+template <int K> __device__ __forceinline__ float su_bc(float v) { return __uint_as_float(su_dpp<K>(__float_as_uint(v))); }
+template <int K> __device__ __forceinline__ double su_bc(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = su_dpp<K>((unsigned)b), hi = su_dpp<K>((unsigned)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+constexpr int SU_LS = PW_ + 1;   // LDS row stride of the lower block
+template <class T, class Out>
+__device__ __forceinline__ void su_solve(const typename C2<T>::t *L, int cls, typename C2<T>::t (&x)[8], Out out) {
+  typedef typename C2<T>::t cT;
+#pragma unroll 1
+  for (int kb = 0; kb < 8; ++kb) {
+    auto step = [&](auto kc) {
+      constexpr int K = decltype(kc)::value;
+      const cT v = cT{su_bc<K>(x[0].x), su_bc<K>(x[0].y)};
+      const int k = 4 * kb + K;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        if (q >= 8 - kb) continue;   // rows beyond the block (uniform)
+        const cT l = L[(4 * (kb + q) + cls) * SU_LS + k];
+        const cT y = cT{fma(-l.x, v.x, fma(l.y, v.y, x[q].x)), fma(-l.x, v.y, fma(-l.y, v.x, x[q].y))};
+        if (q > 0 || cls > K) x[q] = y;
+      }
+    };
+    step(std::integral_constant<int, 0>{});
+    step(std::integral_constant<int, 1>{});
+    step(std::integral_constant<int, 2>{});
+    step(std::integral_constant<int, 3>{});
+    out(kb, x[0]);
+#pragma unroll
+    for (int q = 0; q < 7; ++q) x[q] = x[q + 1];
+  }
+}
+
+// A strip's interchanges on the block's other columns [lo, hi), and U = L11^{-1}
+// A12 on those behind the strip: 64 columns per workgroup, 16 per wave. The
+// first nl workgroups take the columns before the strip, the others those
+// behind; workgroup 0 also brings perm up to date.
+template <class T>
+__global__ __launch_bounds__(256) void k_swap_u(int n, int c0, int w, typename C2<T>::t *A, long lda, long sA,
+                                                const char *fin, long sW, int lo, int hi, int nl, int *perm, long sP) {
+  typedef typename C2<T>::t cT;
+  __shared__ __align__(16) cT L[PW_ * SU_LS];
+  const int z = blockIdx.z, b = blockIdx.x, t = threadIdx.x, lane = t & 63, cls = lane & 3;
+  A += (long)z * sA;
+  fin += (long)z * sW;
+  const int *src = reinterpret_cast<const int *>(fin), *to = src + PW_;
+  if (b == 0 && perm && t < 2 * PW_) {
+    int *pz = perm + (long)z * sP + c0;
+    const int i = t & (PW_ - 1);
+    const bool mv = i < w && (t < PW_ || to[i] >= w);
+    const int f = mv ? (t < PW_ ? src[i] : i) : 0, d = mv ? (t < PW_ ? i : to[i]) : 0;
+    const int v = mv ? pz[f] : 0;   // one wave: every lane loads before any stores
+    __builtin_amdgcn_s_waitcnt(0);
+    if (mv) pz[d] = v;
+  }
+  const bool behind = b >= nl;
+  const int col = (behind ? c0 + w + (b - nl) * 64 : lo + b * 64) + (t >> 6) * 16 + (lane >> 2);
+  const bool ok = col < (behind ? hi : c0);
+  if (behind)
+    for (int e = t; e < PW_ * PW_; e += 256) {
+      const int i = e / PW_, k = e % PW_;
+      L[i * SU_LS + k] = (i < w && k < i) ? A[(long)(c0 + i) * lda + c0 + k] : cT{0, 0};
+    }
+  cT x[8], y[8];   // rows 4 q + cls of the new top, and of the old top where they leave it
+  int d[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int i = 4 * q + cls;
+    const bool in = ok && i < w;
+    const int s = in ? src[i] : 0;
+    d[q] = in ? to[i] : 0;
+    x[q] = in ? A[(long)(c0 + s) * lda + col] : cT{0, 0};
+    y[q] = in && d[q] >= w ? A[(long)(c0 + i) * lda + col] : cT{0, 0};
+  }
+  __builtin_amdgcn_s_waitcnt(0);   // the four lanes of a column read each other's rows: all loads are done
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (ok && d[q] >= w) A[(long)(c0 + d[q]) * lda + col] = y[q];
+  auto put = [&](int q, cT v) {
+    const int i = 4 * q + cls;
+    if (ok && i < w) A[(long)(c0 + i) * lda + col] = v;
+  };
+  if (behind) {
+    su_solve<T>(L, cls, x, put);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) put(q, x[q]);
+  }
+}
+
+// U12 = L11^{-1} A12 of an outer block (nb <= 256 rows at A, unit lower L in the
+// columns before them) for 16 columns per workgroup, held in LDS for the whole
+// solve: per 32 rows one wave substitutes (su_solve), then the four waves
+// subtract L21 times the solved rows from the rows below with matrix
+// instructions, L read as operands straight from the matrix (all workgroups
+// read the same 512 KB). As eight products with inverses and seven updates it
+// was 15 dependent launches, about 200 us per block.
+constexpr int U12_C = 16, U12_XS = U12_C + 1;
+template <class T> constexpr size_t u12_lds() { return (size_t)(256 * U12_XS + PW_ * SU_LS) * sizeof(typename C2<T>::t); }
+template <class T>
+__global__ __launch_bounds__(256) void k_u12(int nb, int ncols, const typename C2<T>::t *Lm, long lda, long sA,
+                                             typename C2<T>::t *B) {
+  typedef typename C2<T>::t cT;
+  typedef typename MF<T>::acc acc_t;
+  extern __shared__ __align__(16) char smem_raw[];
+  cT *X = reinterpret_cast<cT *>(smem_raw), *L = X + 256 * U12_XS;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, j0 = blockIdx.x * U12_C, nc = min(U12_C, ncols - j0);
+  Lm += (long)blockIdx.z * sA;
+  B += (long)blockIdx.z * sA + j0;
+  {
+    const int c = t % U12_C, r = t / U12_C;
+    cT v[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = (c < nc && r + 16 * q < nb) ? B[(long)(r + 16 * q) * lda + c] : cT{0, 0};
+#pragma unroll
+    for (int q = 0; q < 16; ++q) X[(r + 16 * q) * U12_XS + c] = v[q];
+  }
+  const int lr = lane & 15, lk = lane >> 4;
+  for (int s = 0; s < nb; s += PW_) {
+    const int w = min(PW_, nb - s);
+#pragma unroll
+    for (int e = t; e < PW_ * PW_; e += 256) {
+      const int i = e / PW_, k = e % PW_;
+      L[i * SU_LS + k] = (i < w && k < i) ? Lm[(long)(s + i) * lda + s + k] : cT{0, 0};
+    }
+    __syncthreads();
+    if (wave == 0) {
+      const int cls = lane & 3, c = lane >> 2;
+      cT x[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) x[q] = X[(s + 4 * q + cls) * U12_XS + c];
+      su_solve<T>(L, cls, x, [&](int q, cT v) { X[(s + 4 * q + cls) * U12_XS + c] = v; });
+    }
+    __syncthreads();
+    for (int r0 = s + PW_ + 16 * wave; r0 < nb; r0 += 64) {   // 16 rows at a time
+      cT a[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        a[q] = (r0 + lr < nb) ? Lm[(long)(r0 + lr) * lda + s + 4 * q + lk] : cT{0, 0};
+      acc_t pr = acc_t{0, 0, 0, 0}, pi = acc_t{0, 0, 0, 0};
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const cT b = X[(s + 4 * q + lk) * U12_XS + lr];
+        pr = MF<T>::mma(a[q].x, b.x, pr);
+        pi = MF<T>::mma(a[q].x, b.y, pi);
+        pr = MF<T>::mma(-a[q].y, b.y, pr);
+        pi = MF<T>::mma(a[q].y, b.x, pi);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        cT &x = X[(r0 + MF<T>::row(lk, e)) * U12_XS + lr];
+        x = cT{x.x - pr[e], x.y - pi[e]};
+      }
+    }
+    __syncthreads();
+  }
+  const int c = t % U12_C;
+  for (int r = t / U12_C; r < nb; r += 16)
+    if (c < nc) B[(long)r * lda + c] = X[r * U12_XS + c];
 }
 
 // ---------------------------------------------------------------------------
@@ -1746,7 +1866,7 @@ static size_t whole_cu_lds(const void *fn) {
 }
 template <class T>
 struct WholeCu {   // dynamic-LDS requests of the strip kernels for whole-CU launches
-  size_t local, merge, apply, gemm_assign, gemm_sub, strip;
+  size_t local, merge, apply, gemm_assign, gemm_sub, strip, swap_u;
 };
 template <class T>
 static const WholeCu<T> &whole_cu() {
@@ -1759,6 +1879,7 @@ static const WholeCu<T> &whole_cu() {
     w.gemm_assign = std::max(whole_cu_lds((const void *)k_gemm_cu<T, true>), gcu_lds<T>());
     w.gemm_sub = std::max(whole_cu_lds((const void *)k_gemm_cu<T, false>), gcu_lds<T>());
     w.strip = whole_cu_lds((const void *)k_strip<T>);
+    w.swap_u = whole_cu_lds((const void *)k_swap_u<T>);
   });
   return w;
 }
@@ -1773,6 +1894,10 @@ static void ts_prepare() {
     HIPCHK(hipFuncSetAttribute((const void *)k_ts_merge<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ts_lds<T>()));
   });
   (void)whole_cu<T>();   // raises the limits further for whole-CU launches
+  static std::once_flag u12;
+  std::call_once(u12, [] {
+    HIPCHK(hipFuncSetAttribute((const void *)k_u12<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)u12_lds<T>()));
+  });
 }
 
 extern "C" void qh_cgemm3m_prepare(void);
@@ -1787,10 +1912,33 @@ extern "C" void qh_lu_prepare(void) {
   qh_cgemm3m_prepare();
 }
 
+// Whether a factorisation may use the tournament for some of its blocks (see
+// getrf_batched): single matrices with strips of more workgroups than CUs are
+// kept free beside the trailing update.
+template <class T>
+static bool may_tournament(int n, int batch, bool pp) {
+  return !pp && batch == 1 && use_lookahead() && st_groups<T>(n) > lu_reserve_cus();
+}
+// Workspace of one matrix: the strips' words, the tournament's two candidate
+// buffers (the second holds the first merge level's output, a set per workgroup
+// of fan-in sets) where it may be used, the output slots.
+template <class T>
+struct LuWS {
+  size_t strip, buf_a, buf_b, fin, bytes;   // offsets, total
+  LuWS(int n, int batch, bool pp) {
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t sets = may_tournament<T>(n, batch, pp) ? (size_t)PanelWS<T>::sets(n) : 0;
+    strip = 0;
+    buf_a = up((size_t)st_ws_bytes<T>(n));
+    buf_b = buf_a + sets * PanelWS<T>::set_bytes();
+    fin = buf_b + (sets + ts_fan<T>() - 1) / ts_fan<T>() * PanelWS<T>::set_bytes();
+    bytes = fin + up(TS_SLOTS * PanelWS<T>::fin_bytes());
+  }
+};
 // Workspace bytes for getrf_batched<T>(n, batch).
 template <class T>
 static size_t getrf_ws_bytes(int n, int batch) {
-  return (size_t)batch * PanelWS<T>::bytes(n);
+  return (size_t)batch * LuWS<T>(n, batch, false).bytes;
 }
 
 // Blocked right-looking LU with tournament-pivoted panels of `batch` n x n
@@ -1812,10 +1960,9 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
   const dim3 b256(256);
   if (n <= 0 || batch <= 0) return;
   if (n >= (1 << 22)) qpms_hip_die(__FILE__, __LINE__, __func__, "order %d above the pivot search's 2^22 rows", n);
-  const int Gmax = PanelWS<T>::sets(n);
-  const long sW = (long)PanelWS<T>::bytes(n);
+  const LuWS<T> lay(n, batch, pp);
+  const long sW = (long)lay.bytes;
   const long setb = (long)PanelWS<T>::set_bytes();
-  const long sWc = sW / (long)sizeof(cT);   // the workspace stride in complex entries
   if (!ws) {
     static char *own = nullptr;
     static size_t own_bytes = 0;
@@ -1829,88 +1976,69 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
   }
   const dim3 bts(TS_THREADS);
   ts_prepare<T>();
-  char *bufA = ws, *bufB = ws + (long)Gmax * setb;   // two candidate buffers per matrix
-  char *fin0 = ws + 2 * (long)Gmax * setb;           // per-strip slots of the last level's output
+  char *bufA = ws + lay.buf_a, *bufB = ws + lay.buf_b, *fin0 = ws + lay.fin;
   const long finb = (long)PanelWS<T>::fin_bytes();
-  // The strips of the outer block [k0, k0 + nb): tournament, interchanges on
-  // the block's own columns, L21, then the block's remaining columns by TRSM
-  // and the rank-w update. Touches only the block's columns (rows >= k0).
-  if (pp && st_ws_bytes<T>(n) > 2 * (long)Gmax * setb)
-    qpms_hip_die(__FILE__, __LINE__, __func__, "partial-pivoting workspace does not fit (order %d)", n);
-  if (pp)
-    QH_LAUNCH(k_strip_init, dim3((unsigned)std::min((st_ws_bytes<T>(n) / 8 + 255) / 256, 1024L), 1, batch), b256, 0, s,
-              ws, sW, st_ws_bytes<T>(n));
-  // partial pivoting: the strip in place, then its slot
-  auto pp_strip = [&](int c0, int w, hipStream_t st, bool wcu) {
-    QH_LAUNCH(k_strip<T>, dim3(st_groups<T>(n - c0), 1, batch), dim3(st_w<T>() * 64), wcu ? whole_cu<T>().strip : 0, st, n,
-              c0, w, A, lda, sA, ws, sW, wait, ipiv, sP, dinfo);
-    QH_LAUNCH(k_pp_finish<T>, dim3(1, 1, batch), b256, PP_FIN_LDS, st, n, c0, w, A, lda, sA, ws, sW,
-              (long)(fin0 - ws) + (long)((c0 % LU_NB) / PW) * finb, perm, sP);
-  };
+  QH_LAUNCH(k_strip_init, dim3((unsigned)std::min((st_ws_bytes<T>(n) / 8 + 255) / 256, 1024L), 1, batch), b256, 0, s, ws,
+            sW, st_ws_bytes<T>(n));
+  // The strips of the outer block [k0, k0 + nb): pivots, interchanges on the
+  // block's own columns, L21, then the block's remaining columns by TRSM and the
+  // rank-w update. Touches only the block's columns (rows >= k0). wcu: beside a
+  // trailing update, as whole-CU workgroups; strips of more workgroups than CUs
+  // are free then go by tournament, whose workgroups do not wait for each other.
   auto block_strips = [&](int k0, int nb, hipStream_t st, bool wcu) {
     constexpr int F = ts_fan<T>();
+    const bool tour = wcu && st_groups<T>(n - k0) > lu_reserve_cus();
     const WholeCu<T> &W = whole_cu<T>();
-    const size_t l_local = wcu ? W.local : ts_lds<T>(), l_merge = wcu ? W.merge : ts_lds<T>();
-    const size_t l_apply = wcu ? W.apply : 0, l_asg = wcu ? W.gemm_assign : 0, l_sub = wcu ? W.gemm_sub : 0;
+    const size_t l_asg = W.gemm_assign, l_sub = W.gemm_sub;
     for (int j0 = 0; j0 < nb; j0 += PW) {
       const int w = min(PW, nb - j0), c0 = k0 + j0;
       char *fin = fin0 + (long)(j0 / PW) * finb;
-      if (pp) {   // the strip factored in place (L21 included); interchanges on the block's other columns
-        pp_strip(c0, w, st, wcu);
-        if (c0 > k0)
-          QH_LAUNCH(k_ts_apply<T>, dim3((c0 - k0 + AP_COLS - 1) / AP_COLS, 1, batch), b256, l_apply, st, n, c0, w, A,
-                    lda, sA, fin, sW, k0, c0);
-        if (k0 + nb > c0 + w)
-          QH_LAUNCH(k_ts_apply<T>, dim3((k0 + nb - c0 - w + AP_COLS - 1) / AP_COLS, 1, batch), b256, l_apply, st, n,
-                    c0, w, A, lda, sA, fin, sW, c0 + w, k0 + nb);
-      } else {
-      const int G = (n - c0 + TsRows<T>::R - 1) / TsRows<T>::R;
-      QH_LAUNCH(k_ts_local<T>, dim3(G, 1, batch), bts, l_local, st, n, c0, w, A, lda, sA, ws, sW, setb,
-                         (long)(fin - ws), G == 1 ? 1 : 0, ipiv, sP, perm, dinfo);
-      char *cur = bufA, *nxt = bufB;
-      for (int nsets = G; nsets > 1; nsets = (nsets + F - 1) / F) {
-        const int nout = (nsets + F - 1) / F;
-        QH_LAUNCH(k_ts_merge<T>, dim3(nout, 1, batch), bts, l_merge, st, c0, w, nsets, cur, nxt, sW,
-                           setb, fin, nout == 1 ? 1 : 0, ipiv, sP, perm, dinfo);
-        char *tmp = cur; cur = nxt; nxt = tmp;
-      }
-      QH_LAUNCH(k_ts_apply<T>, dim3((nb + AP_COLS - 1) / AP_COLS, 1, batch), b256, l_apply, st, n, c0, w, A,
-                lda, sA, fin, sW, k0, k0 + nb);
-      }
-      const cT *linv = reinterpret_cast<const cT *>(fin + PanelWS<T>::fin_inv_off()), *uinv = linv + PW * PW;
-      const int mr = n - c0 - w;
       const int rest = k0 + nb - (c0 + w);
+      if (!tour) {   // the strip factored in place (L21 included), its interchanges and U on the block's other columns
+        QH_LAUNCH(k_strip<T>, dim3(st_groups<T>(n - c0), 1, batch), dim3(st_w<T>() * 64), wcu ? W.strip : 0, st, n, c0, w,
+                  A, lda, sA, ws, sW, (long)(fin - ws), wait, ipiv, sP, dinfo);
+        const int nl = (c0 - k0 + 63) / 64, nu = (rest + 63) / 64;
+        if (nl + nu > 0 || perm)
+          QH_LAUNCH(k_swap_u<T>, dim3(std::max(nl + nu, 1), 1, batch), b256, wcu ? W.swap_u : 0, st, n, c0, w, A, lda, sA,
+                    fin, sW, k0, k0 + nb, nl, perm, sP);
+      } else {
+        const int G = (n - c0 + TsRows<T>::R - 1) / TsRows<T>::R;
+        QH_LAUNCH(k_ts_local<T>, dim3(G), bts, W.local, st, n, c0, w, A, lda, sA, bufA, sW, setb, (long)(fin - bufA),
+                  G == 1 ? 1 : 0, ipiv, sP, perm, dinfo);
+        char *cur = bufA, *nxt = bufB;
+        for (int nsets = G; nsets > 1; nsets = (nsets + F - 1) / F) {
+          const int nout = (nsets + F - 1) / F;
+          QH_LAUNCH(k_ts_merge<T>, dim3(nout), bts, W.merge, st, c0, w, nsets, cur, nxt, sW, setb, fin,
+                    nout == 1 ? 1 : 0, ipiv, sP, perm, dinfo);
+          std::swap(cur, nxt);
+        }
+        const int nl = (c0 - k0 + 63) / 64, nu = (rest + 63) / 64;
+        QH_LAUNCH(k_ts_apply<T>, dim3(1), b256, W.apply, st, n, c0, w, A, lda, fin);
+        if (nl + nu > 0)
+          QH_LAUNCH(k_swap_u<T>, dim3(nl + nu), b256, W.swap_u, st, n, c0, w, A, lda, sA, fin, sW, k0, k0 + nb, nl,
+                    (int *)nullptr, sP);
+      }
+      const int mr = n - c0 - w;
       if (wcu) {   // single matrix, whole-CU launches (k_gemm_cu: several tiles per CU, K <= PW)
         const dim3 bcu(gcu_q<T>() * 256);
         auto gcu_grid = [](int M, int N) {
           const int nt = ((M + GT - 1) / GT) * ((N + GT - 1) / GT);
           return dim3(std::min((nt + gcu_q<T>() - 1) / gcu_q<T>(), 4096));
         };
-        if (mr > 0 && !pp)   // L21 = A21 U11^{-1}
+        if (mr > 0 && tour)   // L21 = A21 U11^{-1}
           QH_LAUNCH((k_gemm_cu<T, true>), gcu_grid(mr, w), bcu, l_asg, st, mr, w, w, A + (long)(c0 + w) * lda + c0,
-                    lda, uinv, (long)PW, A + (long)(c0 + w) * lda + c0, lda);
-        if (rest > 0) {   // the block's next columns: U = L11^{-1} A12, then A22 -= L21 U
-          QH_LAUNCH((k_gemm_cu<T, true>), gcu_grid(w, rest), bcu, l_asg, st, w, rest, w, linv, (long)PW,
-                    A + (long)c0 * lda + c0 + w, lda, A + (long)c0 * lda + c0 + w, lda);
-          if (mr > 0)
-            QH_LAUNCH((k_gemm_cu<T, false>), gcu_grid(mr, rest), bcu, l_sub, st, mr, rest, w,
-                      A + (long)(c0 + w) * lda + c0, lda, A + (long)c0 * lda + c0 + w, lda,
-                      A + (long)(c0 + w) * lda + c0 + w, lda);
-        }
+                    lda, reinterpret_cast<const cT *>(fin + PanelWS<T>::UINV_OFF), (long)PW,
+                    A + (long)(c0 + w) * lda + c0, lda);
+        if (rest > 0 && mr > 0)   // the block's next columns: A22 -= L21 U
+          QH_LAUNCH((k_gemm_cu<T, false>), gcu_grid(mr, rest), bcu, l_sub, st, mr, rest, w,
+                    A + (long)(c0 + w) * lda + c0, lda, A + (long)c0 * lda + c0 + w, lda,
+                    A + (long)(c0 + w) * lda + c0 + w, lda);
         continue;
       }
-      if (mr > 0 && !pp)   // L21 = A21 U11^{-1}
-        QH_LAUNCH((k_gemm_sub<T, true>), dim3(1, (mr + GT - 1) / GT, batch), b256, l_asg, st, mr, w, w,
-                  A + (long)(c0 + w) * lda + c0, lda, sA, uinv, (long)PW, sWc, A + (long)(c0 + w) * lda + c0, lda,
-                  sA);
-      if (rest > 0) {   // the block's next columns: U = L11^{-1} A12, then A22 -= L21 U
-        QH_LAUNCH((k_gemm_sub<T, true>), dim3((rest + GT - 1) / GT, 1, batch), b256, l_asg, st, w, rest, w, linv,
-                  (long)PW, sWc, A + (long)c0 * lda + c0 + w, lda, sA, A + (long)c0 * lda + c0 + w, lda, sA);
-        if (mr > 0)
-          QH_LAUNCH(k_gemm_sub<T>, dim3((rest + GT - 1) / GT, (mr + GT - 1) / GT, batch), b256, l_sub, st, mr,
-                             rest, w, A + (long)(c0 + w) * lda + c0, lda, sA, A + (long)c0 * lda + c0 + w, lda, sA,
-                             A + (long)(c0 + w) * lda + c0 + w, lda, sA);
-      }
+      if (rest > 0 && mr > 0)   // the block's next columns: A22 -= L21 U
+        QH_LAUNCH(k_gemm_sub<T>, dim3((rest + GT - 1) / GT, (mr + GT - 1) / GT, batch), b256, 0, st, mr, rest, w,
+                  A + (long)(c0 + w) * lda + c0, lda, sA, A + (long)c0 * lda + c0 + w, lda, sA,
+                  A + (long)(c0 + w) * lda + c0 + w, lda, sA);
     }
   };
   // Lookahead: once the trailing update has reached block k+1's columns, the
@@ -1935,18 +2063,8 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
                          (nb + PW - 1) / PW, A, lda, sA, fin0, finb, sW, k0, k0 + nb);
     const int nr = n - k0 - nb;
     if (nr > 0) {
-      // U12 = L11^{-1} A12, PW rows at a time (each strip's L^{-1} from its slot)
-      for (int j0 = 0; j0 < nb; j0 += PW) {
-        const int w = min(PW, nb - j0), c0 = k0 + j0;
-        const cT *linv = reinterpret_cast<const cT *>(fin0 + (long)(j0 / PW) * finb + PanelWS<T>::fin_inv_off());
-        QH_LAUNCH((k_gemm_sub<T, true>), dim3((nr + GT - 1) / GT, 1, batch), b256, 0, s, w, nr, w, linv, (long)PW,
-                  sWc, A + (long)c0 * lda + k0 + nb, lda, sA, A + (long)c0 * lda + k0 + nb, lda, sA);
-        const int below = nb - j0 - w;
-        if (below > 0)
-          QH_LAUNCH(k_gemm_sub<T>, dim3((nr + GT - 1) / GT, (below + GT - 1) / GT, batch), b256, 0, s, below,
-                             nr, w, A + (long)(c0 + w) * lda + c0, lda, sA, A + (long)c0 * lda + k0 + nb, lda, sA,
-                             A + (long)(c0 + w) * lda + k0 + nb, lda, sA);
-      }
+      QH_LAUNCH(k_u12<T>, dim3((nr + U12_C - 1) / U12_C, 1, batch), b256, u12_lds<T>(), s, nb, nr,
+                (const cT *)(A + (long)k0 * lda + k0), lda, sA, A + (long)k0 * lda + k0 + nb);
       // A22 -= L21 U12: the next block's columns first, then the rest and the next block's strips
       const int nb1 = min(LU_NB, nr);
       trailing_gemm<T>(nr, nb1, nb, batch, A + (long)(k0 + nb) * lda + k0, lda, sA, A + (long)k0 * lda + k0 + nb, lda,
@@ -2429,27 +2547,25 @@ extern "C" void qh_noalloc_scratch_init(void) {
   g_scratch_ptr[dev] = (char *)p;
 }
 
-// Largest order the scratch array takes (FP64 tournament workspace after a
-// 256-byte info slot).
-extern "C" size_t qpms_hip_zgetrf_noalloc_max_n(void) {
-  size_t n = 256;
-  while (256 + PanelWS<double>::bytes((int)(n + 256)) <= NOALLOC_SCRATCH_BYTES) n += 256;
-  return n;
-}
+// Largest order the entry point takes (its strips' words and slots, after a
+// 256-byte info word, fit the scratch array).
+constexpr int NOALLOC_MAX_N = 125952;
+extern "C" size_t qpms_hip_zgetrf_noalloc_max_n(void) { return NOALLOC_MAX_N; }
 
 extern "C" int qpms_hip_zgetrf_dev_noalloc(size_t n, _Complex double *A_dev, int *ipiv_dev, void *stream) {
   hipStream_t s = (hipStream_t)qh_stream(stream);
   if (n == 0) return 0;
-  const size_t need = 256 + PanelWS<double>::bytes((int)(n < (1u << 22) ? n : (1u << 22)));
-  if (n >= (1u << 22) || need > NOALLOC_SCRATCH_BYTES) {
-    fprintf(stderr, "qpms_hip_zgetrf_dev_noalloc: order %zu needs %zu bytes of scratch, above the %zu-byte array "
-            "(largest order %zu)\n", n, need, NOALLOC_SCRATCH_BYTES, qpms_hip_zgetrf_noalloc_max_n());
+  if (n > (size_t)NOALLOC_MAX_N) {
+    fprintf(stderr, "qpms_hip_zgetrf_dev_noalloc: order %zu is above the largest order %d of the %zu-byte scratch "
+            "array\n", n, NOALLOC_MAX_N, NOALLOC_SCRATCH_BYTES);
     return -1;
   }
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
   char *base = (dev >= 0 && dev < NOALLOC_MAX_DEV) ? g_scratch_ptr[dev] : nullptr;
   if (!base) qpms_hip_die(__FILE__, __LINE__, __func__, "scratch of device %d not initialised", dev);
+  if (256 + LuWS<double>((int)n, 1, true).bytes > NOALLOC_SCRATCH_BYTES)
+    qpms_hip_die(__FILE__, __LINE__, __func__, "scratch too small for order %zu", n);
   int *dinfo = (int *)base;
   qh_zero(dinfo, 256, s);   // a kernel: the info word must start at zero on every call
   getrf_batched<double>((int)n, 1, (v2d *)A_dev, (long)n, 0, ipiv_dev, 0, nullptr, dinfo, s, base + 256,

@@ -89,3 +89,38 @@ def test_strip_non_finite(gpu, where):
     assert np.max(np.abs(LU[fin] - ref[fin])) < 1e-11 * np.max(np.abs(ref[fin]))
     ok = int(np.argmin(np.append(fin.all(axis=0), False)))   # columns before the first that is touched
     assert np.array_equal(piv[:ok], rp[:ok])
+
+
+@pytest.mark.parametrize("prec, n", [(64, 32), (64, 64), (64, 512), (32, 64), (32, 1024)])
+def test_strip_ties(gpu, prec, n):
+    """A Hadamard matrix: every pivot search is a tie of many rows, and every
+    value a power of two, so that the first row has to win each time."""
+    H = np.ones((1, 1))
+    while len(H) < n:
+        H = np.block([[H, H], [H, -H]])
+    LU, piv, info = getrf_pp(H + 0j, prec, 10 ** 7)
+    ref, rp = eliminate(H + 0j)
+    assert info == 0 and np.array_equal(piv, rp) and np.array_equal(LU, ref)
+
+
+def test_blocks_by_tournament(gpu):
+    """Blocks of more rows than the strips' workgroups find CUs for beside the
+    trailing update (FP64: 8192) go by tournament, the others by k_strip."""
+    import qpms_amd
+    from test_gpu_lu import check_plu
+    L = qpms_amd.lib()
+    n = 8800
+    rng = np.random.default_rng(5)
+    A = np.empty((n, n), np.complex128)
+    A.real = rng.random((n, n), np.float32) - 0.5
+    A.imag = rng.random((n, n), np.float32) - 0.5
+    dA = qpms_amd.DeviceBuffer.from_array(A)
+    dp, dq, di = qpms_amd.DeviceBuffer(4 * n), qpms_amd.DeviceBuffer(4 * n), qpms_amd.DeviceBuffer.from_array(
+        np.zeros(1, np.int32))
+    L.qh_getrf_batched_f64.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p,
+                                       ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+    L.qh_getrf_batched_f64(n, 1, dA.ptr, n * n, dp.ptr, dq.ptr, di.ptr, None)
+    L.qpms_hip_sync()
+    assert int(di.to_array(np.int32, (1,))[0]) == 0
+    # rows of a random matrix: |L| <= 2 or so per level of the tournament, errors of n products
+    check_plu(A, dA.to_array(np.complex128, (n, n)), dp.to_array(np.int32, (n,)), 1e-13)
