@@ -303,14 +303,14 @@ beyn_result_t *beyn_solve_v(size_t m, size_t l, beyn_function_M_t M, beyn_functi
 	qh_h2d(dV, Vhat, ml * sizeof(complex double), NULL);
 	complex double *Mh = NULL, *dM = NULL, *Xh = NULL;
 	int *dpiv = NULL, *dperm = NULL, *dinfo = NULL;
-	complex double *dwork = NULL;
+	void *dwork = NULL;
 	if (!M_inv_Vhat) {
 		QH_MALLOC(Mh, m * m * sizeof(complex double));
 		dM = qh_dmalloc(m * m * sizeof(complex double));
 		dpiv = qh_dmalloc(m * sizeof(int));
 		dperm = qh_dmalloc(m * sizeof(int));
 		dinfo = qh_dmalloc(sizeof(int));
-		dwork = qh_dmalloc(ml * sizeof(complex double));
+		dwork = qh_dmalloc(qh_getrs_ws_bytes(64, (int)m, (int)l, 1));
 	} else {
 		QH_MALLOC(Xh, ml * sizeof(complex double));
 	}
@@ -328,8 +328,7 @@ beyn_result_t *beyn_solve_v(size_t m, size_t l, beyn_function_M_t M, beyn_functi
 				qh_memset(dinfo, 0, sizeof(int), NULL);
 				qh_getrf_batched_f64((int)m, 1, (double *)dM, 0, dpiv, dperm, dinfo, NULL);
 				qh_copy_c64((long)ml, (const double *)dV, (double *)dX, NULL);
-				qh_getrs_batched_f64((int)m, (int)l, 1, (const double *)dM, 0, dperm, (double *)dX, 0,
-					(double *)dwork, NULL);
+				qh_getrs_ws_f64((int)m, (int)l, 1, (const double *)dM, 0, dperm, (double *)dX, 0, dwork, NULL);
 			}
 		}
 		const complex double w = z - z0;

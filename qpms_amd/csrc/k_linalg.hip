@@ -185,40 +185,24 @@ __global__ void k_iota(int n, int *p, long sP) {
   if (i < n) p[i] = i;
 }
 
-// Y[i][:] = X[perm[i]][:]
-template <class T>
-__global__ void k_gather_rows(int n, int ncols, const int *perm, long sP, const typename C2<T>::t *X, long ldx,
-                              long sX, typename C2<T>::t *Y, long ldy, long sY) {
-  perm += (long)blockIdx.z * sP;
-  X += (long)blockIdx.z * sX;
-  Y += (long)blockIdx.z * sY;
-  for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < (long)n * ncols; e += (long)gridDim.x * 256) {
-    const int i = (int)(e / ncols), c = (int)(e % ncols);
-    Y[(long)i * ldy + c] = X[(long)perm[i] * ldx + c];
+// perm from LAPACK-style pivots (where a caller hands in pivots without the
+// permutation): each lane follows one row through the interchanges, the same for
+// all, 64 of them loaded at a time while the ones before are gone through; a wave
+// ends when its rows' places lie behind it. One thread making the interchanges
+// one by one took 0.11 us each (1.0 ms at order 9216).
+__global__ __launch_bounds__(64) void k_perm_from_ipiv(int n, const int *__restrict__ ipiv, int *__restrict__ perm) {
+  const int lane = threadIdx.x, t = blockIdx.x * 64 + lane;
+  int pos = t, next = ipiv[min(lane, n - 1)] - 1;
+  for (int i0 = 0; i0 < n && __ballot(pos >= i0 && t < n); i0 += 64) {
+    const int own = i0 + lane < n ? next : i0 + lane;   // behind the end: stays where it is
+    next = ipiv[min(i0 + 64 + lane, n - 1)] - 1;
+#pragma unroll 16
+    for (int q = 0; q < 64; ++q) {
+      const int i = i0 + q, p = __builtin_amdgcn_readlane(own, q);
+      pos = pos == i ? p : pos == p ? i : pos;
+    }
   }
-}
-
-// Y[i][:] = X[i][:] for n rows of ncols (batched, per-matrix strides)
-template <class T>
-__global__ void k_copy_rows(int n, int ncols, const typename C2<T>::t *X, long ldx, long sX, typename C2<T>::t *Y,
-                            long ldy, long sY) {
-  X += (long)blockIdx.z * sX;
-  Y += (long)blockIdx.z * sY;
-  for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < (long)n * ncols; e += (long)gridDim.x * 256) {
-    const int i = (int)(e / ncols), c = (int)(e % ncols);
-    Y[(long)i * ldy + c] = X[(long)i * ldx + c];
-  }
-}
-
-// perm from LAPACK-style pivots (single thread per matrix; used only when a
-// caller hands in pivots without the permutation).
-__global__ void k_perm_from_ipiv(int n, const int *ipiv, int *perm) {
-  if (threadIdx.x != 0) return;
-  for (int i = 0; i < n; ++i) perm[i] = i;
-  for (int i = 0; i < n; ++i) {
-    const int p = ipiv[i] - 1;
-    if (p != i) { int a = perm[i]; perm[i] = perm[p]; perm[p] = a; }
-  }
+  if (t < n) perm[pos] = t;
 }
 
 // C[:, 0:NR] -= A B for few right-hand sides (NR <= 4), FP64 complex: one
@@ -1903,12 +1887,12 @@ static void ts_prepare() {
 extern "C" void qh_cgemm3m_prepare(void);
 // Every kernel attribute the LU paths set, set now (the serving loop calls
 // this at creation, before it captures any launch sequence into a graph).
-template <class T> static void tsb_prepare();
+template <class T> static void tr_prepare();
 extern "C" void qh_lu_prepare(void) {
   ts_prepare<float>();
   ts_prepare<double>();
-  tsb_prepare<float>();
-  tsb_prepare<double>();
+  tr_prepare<float>();
+  tr_prepare<double>();
   qh_cgemm3m_prepare();
 }
 
@@ -2091,321 +2075,359 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
   HIPCHK(hipGetLastError());
 }
 
-// Triangular solves with few right-hand sides (nrhs <= TRV_R), in blocks of
-// TRV_W rows, on the permuted right-hand side W (n x nrhs, row-major):
-//   k_trsv_wave: one wave per matrix solves the w x w (w <= 64) diagonal
-//                block (unit lower, forward; or upper, backward), lane i
-//                owning row r0 + i, with no barrier per step: step s
-//                finalises x_j (j = s forward, w - 1 - s backward, where it
-//                takes the diagonal's reciprocal computed up front), every
-//                lane reads it with readlane, and the rows still open
-//                subtract their column entry times it; the block sits in LDS
-//                column-major (lane i reads entry (i, j) at j TRV_W + i, no
-//                bank conflict) and each lane loads its entries PF steps
-//                ahead;
-//   k_trsv_update: the rows outside the block (below it forward, above it
-//                backward) subtract the block's columns times its solution,
-//                one thread per row walking its row contiguously.
-constexpr int TRV_R = 4, TRV_W = 64;
-__device__ __forceinline__ float trv_readlane(float v, int j) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
+// ---------------------------------------------------------------------------
+// Both triangular solves with a factorisation, one launch (k_tri): workgroup g
+// of G owns the 64-row blocks g, g + G, ... of 16 right-hand-side columns. For a
+// block it subtracts the products with the blocks solved before (each wave a
+// quarter of their columns, by matrix instructions, the sums added in a fixed
+// order), multiplies with the inverse of its diagonal block, which it made while
+// others were solving, and publishes the result; backward the same from below.
+//
+// What bounds it: the chain of blocks, 6.3 us each in FP64 and 4.1 in FP32 (the
+// words' way to the next workgroup, then 64 matrix instructions in a row for the
+// last block's columns and up to 64 for the inverse). As launches per 64-row block
+// (a wave substituting, 18-22 us, then an update, 17 us) an FP64 solve of order
+// 9216 took 10.5 ms, now 2.0; per 256-row block (130 us + 70 us) an FP32 one of
+// order 9990 with 32 right-hand sides 16 ms, now 1.8. Loading the next product's
+// operands or words ahead gained nothing.
+//
+// Published values carry a tag (1 forward, 2 backward) beside each 32 bits, as
+// the strips' words do, so a reader needs no flag. Forward values are all read
+// before the last block is solved forward, hence before any backward one
+// replaces them. The workgroups of a slab announce themselves first
+// (st_rendezvous); where they do not all get onto the device in time, one of
+// them takes all blocks and the others leave.
+// ---------------------------------------------------------------------------
+constexpr int TR_B = 64, TR_C = 16, TR_VS = TR_B + 1, TR_XS = TR_C + 1;
+constexpr int TR_MEET = 256;   // most workgroups of a slab
+template <class T> constexpr size_t tr_lds() {   // diagonal block, the waves' sums, the diagonal's reciprocals
+  return (size_t)(TR_B * TR_VS + 4 * TR_B * TR_XS + TR_B) * sizeof(typename C2<T>::t);
 }
-__device__ __forceinline__ double trv_readlane(double v, int j) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), j), hi = __builtin_amdgcn_readlane((int)(b >> 32), j);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+template <class T> constexpr size_t tr_slab_bytes(int n, int nrhs) {
+  return 256 + TR_MEET * 8 + (size_t)((n + TR_B - 1) / TR_B) * TR_B * (nrhs < TR_C ? nrhs : TR_C) * st_ew<T>() * 8;
 }
-template <class T, bool FWD>
-__global__ __launch_bounds__(TRV_W) void k_trsv_wave(int r0, int w, int nrhs, const typename C2<T>::t *LU, long lda,
-                                                     long sA, typename C2<T>::t *W, long sW) {
+template <class T> constexpr size_t tr_ws_bytes(int n, int nrhs) {
+  return (size_t)((nrhs + TR_C - 1) / TR_C) * ((tr_slab_bytes<T>(n, nrhs) + 255) / 256 * 256);
+}
+
+template <class F, int... K>
+__device__ __forceinline__ void tr_each(F f, std::integer_sequence<int, K...>) {
+  (f(std::integral_constant<int, K>{}), ...);
+}
+
+// The 64 x 64 triangular block V (LDS, row stride TR_VS; UPPER: with dinv its
+// diagonal's reciprocals; zeros in the other triangle) is replaced by its inverse,
+// all 256 threads. W: scratch. UPPER works on the block turned
+// round (row and column i for 63 - i), where it is lower triangular. The four
+// 16 x 16 diagonal blocks by substitution, one per wave, four lanes per column;
+// then [A 0; B C] of twice the size, whose inverse's corner is -C^-1 (B A^-1), by
+// matrix instructions, twice. Substitution with the whole block (64 steps in a
+// row, each waiting for LDS) took 35 us, this way 5. The solutions' errors in FP64
+// (80-bit reference, orders 64 to 1024) are 1.3 to 2 times those of
+// substitution throughout, 4e-16 for systems near the identity; a residual
+// correction per block brought 1.0 to 1.4 times for twice the chain.
+template <class T, bool UPPER>
+__device__ __forceinline__ void tr_invert(typename C2<T>::t *V, const typename C2<T>::t *dinv, typename C2<T>::t *W,
+                                          int wave, int lane) {
   typedef typename C2<T>::t cT;
-  constexpr int PF = 4;
-  __shared__ cT sL[TRV_W * TRV_W];   // sL[j TRV_W + i] = LU(r0 + i, r0 + j)
-  LU += (long)blockIdx.z * sA;
-  W += (long)blockIdx.z * sW;
-  const int i = threadIdx.x;
-  const bool mine = i < w;
-  if (mine) {
-    const cT *row = LU + (long)(r0 + i) * lda + r0;
-    for (int j = 0; j < w; ++j) sL[j * TRV_W + i] = row[j];
-  }
-  cT y[TRV_R];
+  typedef typename MF<T>::acc acc_t;
+  auto at = [&](int r, int c) -> cT & { return V[UPPER ? (TR_B - 1 - r) * TR_VS + TR_B - 1 - c : r * TR_VS + c]; };
+  const int cls = lane & 3, col = lane >> 2, o = 16 * wave, lr = lane & 15, lk = lane >> 4;
+  {
+    cT x[4];
 #pragma unroll
-  for (int c = 0; c < TRV_R; ++c) y[c] = (mine && c < nrhs) ? W[(long)(r0 + i) * nrhs + c] : cT{0, 0};
+    for (int q = 0; q < 4; ++q) x[q] = cT{4 * q + cls == col ? T(1) : T(0), 0};
+    auto step = [&](auto kc) {
+      constexpr int K = decltype(kc)::value;
+      cT v = cT{su_bc<(K & 3)>(x[K / 4].x), su_bc<(K & 3)>(x[K / 4].y)};
+      if (UPPER) {
+        v = cmul<T>(v, dinv[TR_B - 1 - o - K]);
+        if (cls == (K & 3)) x[K / 4] = v;
+      }
+#pragma unroll
+      for (int q = K / 4; q < 4; ++q) {
+        const cT l = at(o + 4 * q + cls, o + K);
+        const cT y = cT{fma(-l.x, v.x, fma(l.y, v.y, x[q].x)), fma(-l.x, v.y, fma(-l.y, v.x, x[q].y))};
+        if (q > K / 4 || cls > (K & 3)) x[q] = y;
+      }
+    };
+    tr_each(step, std::make_integer_sequence<int, 16>{});
+    // only this wave reads its block
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      at(o + 4 * q + cls, o + col) = x[q];
+  }
   __syncthreads();
-  const cT dinv = (!FWD && mine) ? cdiv<T>(cT{1, 0}, sL[i * TRV_W + i]) : cT{1, 0};
-  auto col = [&](int s) { return FWD ? s : w - 1 - s; };
-  cT buf[PF];
+  // 32 x 32: wave w the real (even) or imaginary (odd) parts for pair w / 2
+  const int pair = wave >> 1, part = wave & 1, a0 = 32 * pair, c0 = a0 + 16;
+  T *Wt = reinterpret_cast<T *>(W);
+  auto corner = [&](auto &&A, auto &&X) {
+    acc_t p = acc_t{0, 0, 0, 0};
 #pragma unroll
-  for (int k = 0; k < PF; ++k) buf[k] = (mine && k < w) ? sL[col(k) * TRV_W + i] : cT{0, 0};
-  for (int s0 = 0; s0 < w; s0 += PF) {
-#pragma unroll
-    for (int k = 0; k < PF; ++k) {
-      const int s = s0 + k;
-      if (s >= w) continue;   // uniform
-      const int j = col(s);
-      const cT l = buf[k];
-      buf[k] = (mine && s + PF < w) ? sL[col(s + PF) * TRV_W + i] : cT{0, 0};
-      if (!FWD && i == j) {
-#pragma unroll
-        for (int c = 0; c < TRV_R; ++c) y[c] = cmul<T>(y[c], dinv);
-      }
-      cT x[TRV_R];
-#pragma unroll
-      for (int c = 0; c < TRV_R; ++c) x[c] = cT{trv_readlane(y[c].x, j), trv_readlane(y[c].y, j)};
-      if (mine && (FWD ? i > j : i < j)) {
-#pragma unroll
-        for (int c = 0; c < TRV_R; ++c)
-          y[c] = cT{y[c].x - (l.x * x[c].x - l.y * x[c].y), y[c].y - (l.x * x[c].y + l.y * x[c].x)};
-      }
+    for (int ks = 0; ks < 4; ++ks) {
+      const cT a = A(lr, 4 * ks + lk), x = X(4 * ks + lk, lr);
+      p = MF<T>::mma(part ? a.y : a.x, x.x, p);
+      p = MF<T>::mma(part ? a.x : -a.y, x.y, p);
     }
-  }
-  if (mine)
+    return p;
+  };
+  {
+    const acc_t p = corner([&](int r, int k) { return at(c0 + r, a0 + k); }, [&](int k, int c) { return at(a0 + k, a0 + c); });
 #pragma unroll
-    for (int c = 0; c < TRV_R; ++c)
-      if (c < nrhs) W[(long)(r0 + i) * nrhs + c] = y[c];
+    for (int e = 0; e < 4; ++e) Wt[2 * ((16 * pair + MF<T>::row(lk, e)) * TR_XS + lr) + part] = p[e];
+  }
+  __syncthreads();
+  {
+    const acc_t p = corner([&](int r, int k) { return at(c0 + r, c0 + k); }, [&](int k, int c) { return W[(16 * pair + k) * TR_XS + c]; });
+#pragma unroll
+    for (int e = 0; e < 4; ++e) reinterpret_cast<T *>(&at(c0 + MF<T>::row(lk, e), a0 + lr))[part] = -p[e];
+  }
+  __syncthreads();
+  // 64 x 64: a 16 x 16 tile of the corner per wave, without the triangles' zero tiles
+  const int ti = wave >> 1, tj = wave & 1;
+  auto product = [&](int k0, int k1, auto &&A, auto &&X, acc_t &re, acc_t &im) {
+    re = im = acc_t{0, 0, 0, 0};
+#pragma unroll 4
+    for (int ks = k0; ks < k1; ++ks) {
+      const cT a = A(16 * ti + lr, 4 * ks + lk), x = X(4 * ks + lk, 16 * tj + lr);
+      re = MF<T>::mma(a.x, x.x, re);
+      im = MF<T>::mma(a.x, x.y, im);
+      re = MF<T>::mma(-a.y, x.y, re);
+      im = MF<T>::mma(a.y, x.x, im);
+    }
+  };
+  acc_t re, im;
+  product(4 * tj, 8, [&](int r, int k) { return at(32 + r, k); }, [&](int k, int c) { return at(k, c); }, re, im);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) W[(16 * ti + MF<T>::row(lk, e)) * TR_VS + 16 * tj + lr] = cT{re[e], im[e]};
+  __syncthreads();
+  product(0, 4 * ti + 4, [&](int r, int k) { return at(32 + r, 32 + k); }, [&](int k, int c) { return W[k * TR_VS + c]; }, re, im);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) at(32 + 16 * ti + MF<T>::row(lk, e), 16 * tj + lr) = cT{-re[e], -im[e]};
+  __syncthreads();
 }
 
 template <class T>
-__global__ __launch_bounds__(64) void k_trsv_update(int i0, int nrows, int r0, int w, int nrhs,
-                                                    const typename C2<T>::t *LU, long lda, long sA,
-                                                    typename C2<T>::t *W, long sW) {
-  typedef typename C2<T>::t cT;
-  __shared__ cT sx[TRV_W * TRV_R];
-  LU += (long)blockIdx.z * sA;
-  W += (long)blockIdx.z * sW;
-  for (int e = threadIdx.x; e < w * nrhs; e += 64) sx[(e / nrhs) * TRV_R + e % nrhs] = W[(long)r0 * nrhs + e];
-  __syncthreads();
-  const int r = blockIdx.x * 64 + threadIdx.x;
-  if (r >= nrows) return;
-  const int i = i0 + r;
-  const cT *row = LU + (long)i * lda + r0;
-  cT acc[TRV_R];
-#pragma unroll
-  for (int c = 0; c < TRV_R; ++c) acc[c] = cT{0, 0};
-  for (int j = 0; j < w; ++j) {
-    const cT l = row[j];
-#pragma unroll
-    for (int c = 0; c < TRV_R; ++c) {
-      const cT x = sx[j * TRV_R + c];
-      acc[c] = cT{acc[c].x + (l.x * x.x - l.y * x.y), acc[c].y + (l.x * x.y + l.y * x.x)};
-    }
+__device__ __forceinline__ typename C2<T>::t tr_value(const st_u64 (&w)[sizeof(T) == 8 ? 4 : 2]) {
+  if constexpr (sizeof(T) == 8)
+    return v2d{__longlong_as_double((long long)((w[1] << 32) | (unsigned)w[0])),
+               __longlong_as_double((long long)((w[3] << 32) | (unsigned)w[2]))};
+  else
+    return v2f{__uint_as_float((unsigned)w[0]), __uint_as_float((unsigned)w[1])};
+}
+template <class T>
+__device__ __forceinline__ void tr_publish(st_u64 *at, unsigned tag, typename C2<T>::t v) {
+  const st_u64 hi = (st_u64)tag << 32;
+  if constexpr (sizeof(T) == 8) {
+    const st_u64 a = (st_u64)__double_as_longlong(v.x), b = (st_u64)__double_as_longlong(v.y);
+    st_store(at, hi | (unsigned)a);
+    st_store(at + 1, hi | (unsigned)(a >> 32));
+    st_store(at + 2, hi | (unsigned)b);
+    st_store(at + 3, hi | (unsigned)(b >> 32));
+  } else {
+    st_store(at, hi | __float_as_uint(v.x));
+    st_store(at + 1, hi | __float_as_uint(v.y));
   }
-#pragma unroll
-  for (int c = 0; c < TRV_R; ++c)
-    if (c < nrhs) {
-      cT &y = W[(long)i * nrhs + c];
-      y = cT{y.x - acc[c].x, y.y - acc[c].y};
-    }
 }
 
-// Many right-hand sides: the triangle in diagonal blocks of TsbRows rows
-// (256 FP32, 128 FP64), each solved by one launch of k_trsm_blk, and the rows
-// beyond the block updated by one GEMM with K = the block height: an eighth
-// (a quarter) of the dependent launches of 32-row blocks. k_trsm_blk takes a
-// slab of 32 right-hand-side columns per workgroup into LDS and walks the
-// block's 32-row sub-blocks: the sub-block's triangle and the panel of the
-// triangle beside it (the block's other rows, those columns) are staged in
-// LDS, every load issued before the substitution, which runs in registers,
-// one thread per column; then all threads subtract the panel times the
-// solved rows from the other rows, reading only LDS.
-template <class T> struct TsbRows;
-template <> struct TsbRows<float> { static constexpr int R = 256; };
-template <> struct TsbRows<double> { static constexpr int R = 128; };
-constexpr int TSB_SS = 33, TSB_THREADS = 512;   // LDS row stride of the triangle's columns; workgroup size
-constexpr int TSB_SW = 8, TSB_BS = TSB_SW + 1;  // right-hand-side columns per workgroup; slab row stride
-template <class T> constexpr size_t tsb_lds() {
-  return (size_t)(TsbRows<T>::R * (TSB_BS + TSB_SS)) * sizeof(typename C2<T>::t);   // slab + (sub-block and panel)
-}
-template <class T, bool LOWER>
-__global__ __launch_bounds__(TSB_THREADS) void k_trsm_blk(int w, int ncols, const typename C2<T>::t *L, long ldl,
-                                                          long sL, typename C2<T>::t *B, long ldb, long sB) {
+template <class T>
+__global__ __launch_bounds__(256, 1) void k_tri(int n, int nrhs, const typename C2<T>::t *LU, long lda, long sA,
+                                                const int *perm, long sP, typename C2<T>::t *B, long ldb, long sB,
+                                                char *ws, long sW, long slabb, st_u64 limit) {
   typedef typename C2<T>::t cT;
-  constexpr int TB = TsbRows<T>::R, NPL = TB * 32 / TSB_THREADS;   // staged triangle entries per thread
+  typedef typename MF<T>::acc acc_t;
+  constexpr int EW = st_ew<T>();
   extern __shared__ __align__(16) char smem_raw[];
-  cT *sb = reinterpret_cast<cT *>(smem_raw);   // [TB][TSB_BS] the slab
-  cT *sp = sb + TB * TSB_BS;                    // [TB][TSB_SS] rows of the triangle, columns of the sub-block
-  L += (long)blockIdx.z * sL;
-  B += (long)blockIdx.z * sB;
-  const int t = threadIdx.x, c0 = blockIdx.x * TSB_SW, nc = min(TSB_SW, ncols - c0);
-  for (int e = t; e < w * TSB_SW; e += TSB_THREADS) {
-    const int r = e / TSB_SW, c = e % TSB_SW;
-    sb[r * TSB_BS + c] = (c < nc) ? B[(long)r * ldb + c0 + c] : cT{0, 0};
-  }
-  const int nsub = (w + 31) / 32;
-  for (int q = 0; q < nsub; ++q) {
-    const int j0 = (LOWER ? q : nsub - 1 - q) * 32, jw = min(32, w - j0);
-    // columns j0..j0+jw of every row of the block (the sub-block's triangle
-    // and the panel), loads first
-    {
-      cT v[NPL];
-#pragma unroll
-      for (int u = 0; u < NPL; ++u) {
-        const int e = t + TSB_THREADS * u, r = e >> 5, k = e & 31;
-        v[u] = (r < w && k < jw) ? L[(long)r * ldl + j0 + k] : cT{0, 0};
-      }
-      __syncthreads();   // the previous sub-block's reads of sp are done
-#pragma unroll
-      for (int u = 0; u < NPL; ++u) {
-        const int e = t + TSB_THREADS * u;
-        sp[(e >> 5) * TSB_SS + (e & 31)] = v[u];
-      }
-    }
+  cT *V = reinterpret_cast<cT *>(smem_raw);   // the diagonal block, then its inverse
+  cT *S = V + TR_B * TR_VS, *dinv = S + 4 * TR_B * TR_XS;
+  __shared__ int go;
+  const int z = blockIdx.z, t = threadIdx.x, lane = t & 63, lr = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  int g = blockIdx.x, G = gridDim.x;
+  const int j0 = blockIdx.y * TR_C, nc = min(TR_C, nrhs - j0), cs = min(TR_C, nrhs);   // columns, words' column stride
+  LU += (long)z * sA;
+  perm += (long)z * sP;
+  B += (long)z * sB + j0;
+  char *wz = ws + (long)z * sW + (long)blockIdx.y * slabb;
+  st_u64 *X = reinterpret_cast<st_u64 *>(wz + 256 + TR_MEET * 8);
+  if (G > 1) {
+    if (wave == 0) go = st_rendezvous(g, G, 1u, reinterpret_cast<st_u64 *>(wz + 256), reinterpret_cast<int *>(wz), limit);
     __syncthreads();
-    if (t < TSB_SW) {   // substitution on column t of the slab, in registers
-      cT x[32];
+    if (go == 0) return;
+    if (go < 0) { g = 0; G = 1; }
+  }
+  const int nblk = (n + TR_B - 1) / TR_B;
+  auto sweep = [&](auto up) {
+    constexpr bool UPPER = decltype(up)::value;
+    constexpr unsigned tag = UPPER ? 2u : 1u;
+    const int mine = (nblk - 1 - g) / G + 1;   // blocks of this workgroup
+    for (int b = 0; b < mine; ++b) {
+      const int i = g + G * (UPPER ? mine - 1 - b : b), r0 = i * TR_B;
+      // the diagonal block and its inverse
+      {
+        cT v[16];
 #pragma unroll
-      for (int r = 0; r < 32; ++r) x[r] = (r < jw) ? sb[(j0 + r) * TSB_BS + t] : cT{0, 0};
-      // each row's sum in four interleaved partial sums (shorter dependent chains)
-      if (LOWER) {
-#pragma unroll
-        for (int r = 1; r < 32; ++r) {
-          if (r < jw) {
-            cT a[4] = {cT{0, 0}, cT{0, 0}, cT{0, 0}, cT{0, 0}};
-#pragma unroll
-            for (int k = 0; k < r; ++k) {
-              const cT l = sp[(j0 + r) * TSB_SS + k];
-              a[k & 3] = cT{a[k & 3].x + (l.x * x[k].x - l.y * x[k].y), a[k & 3].y + (l.x * x[k].y + l.y * x[k].x)};
-            }
-            x[r] = cT{x[r].x - ((a[0].x + a[1].x) + (a[2].x + a[3].x)), x[r].y - ((a[0].y + a[1].y) + (a[2].y + a[3].y))};
-          }
+        for (int q = 0; q < 16; ++q) {
+          const int e = t + 256 * q, r = e >> 6, c = e & 63;
+          const bool in = r0 + r < n && r0 + c < n && (UPPER ? c >= r : c < r);
+          v[q] = in ? LU[(long)(r0 + r) * lda + r0 + c] : cT{r == c ? T(1) : T(0), 0};
         }
-      } else {
 #pragma unroll
-        for (int r = 31; r >= 0; --r) {
-          if (r < jw) {
-            cT a[4] = {cT{0, 0}, cT{0, 0}, cT{0, 0}, cT{0, 0}};
-#pragma unroll
-            for (int k = r + 1; k < 32; ++k) {
-              const cT u = sp[(j0 + r) * TSB_SS + k];
-              a[k & 3] = cT{a[k & 3].x + (u.x * x[k].x - u.y * x[k].y), a[k & 3].y + (u.x * x[k].y + u.y * x[k].x)};
-            }
-            const cT v = cT{x[r].x - ((a[0].x + a[1].x) + (a[2].x + a[3].x)), x[r].y - ((a[0].y + a[1].y) + (a[2].y + a[3].y))};
-            x[r] = cdiv<T>(v, sp[(j0 + r) * TSB_SS + r]);
-          }
+        for (int q = 0; q < 16; ++q) {
+          const int e = t + 256 * q, r = e >> 6, c = e & 63;
+          V[r * TR_VS + c] = v[q];
         }
+        __syncthreads();
+        if (UPPER) {
+          if (t < TR_B) dinv[t] = cdiv<T>(cT{1, 0}, V[t * TR_VS + t]);
+          __syncthreads();
+        }
+        tr_invert<T, UPPER>(V, dinv, S, wave, lane);
+      }
+      // this wave's 16 rows of the right-hand side, as results of matrix
+      // instructions: rows of P B, or what the forward sweep left
+      const int rw = r0 + 16 * wave;
+      acc_t rr, ri;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = rw + MF<T>::row(lk, e);
+        cT v = cT{0, 0};
+        if (UPPER) {
+          if (lr < cs) {
+            st_u64 w[EW];
+            bool ok;
+            do {
+              ok = true;
+#pragma unroll
+              for (int k = 0; k < EW; ++k) { w[k] = st_load(X + ((long)r * cs + lr) * EW + k); ok &= (w[k] >> 32) == 1u; }
+            } while (!ok);
+            v = tr_value<T>(w);
+          }
+        } else if (r < n && lr < nc) {
+          v = B[(long)perm[r] * ldb + lr];
+        }
+        rr[e] = v.x;
+        ri[e] = v.y;
+      }
+      // less the products with the blocks solved before, a quarter of their columns per wave
+      acc_t pr[4], pi[4];
+#pragma unroll
+      for (int T_ = 0; T_ < 4; ++T_) { pr[T_] = acc_t{0, 0, 0, 0}; pi[T_] = acc_t{0, 0, 0, 0}; }
+      const int nb = UPPER ? nblk - 1 - i : i;
+      for (int q = 0; q < nb; ++q) {
+        const int k0 = (UPPER ? nblk - 1 - q : q) * TR_B + 16 * wave + lk;
+        cT a[4][4], x[4];
+#pragma unroll
+        for (int T_ = 0; T_ < 4; ++T_)
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) {
+            const int r = r0 + 16 * T_ + lr, c = k0 + 4 * ks;
+            a[T_][ks] = (r < n && c < n) ? LU[(long)r * lda + c] : cT{0, 0};
+          }
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) x[ks] = cT{0, 0};
+        if (lr < cs) {
+          st_u64 w[4][EW];
+          bool ok;
+          do {
+            ok = true;
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+              for (int k = 0; k < EW; ++k) {
+                w[ks][k] = st_load(X + ((long)(k0 + 4 * ks) * cs + lr) * EW + k);
+                ok &= (w[ks][k] >> 32) == tag;
+              }
+          } while (!ok);
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) x[ks] = tr_value<T>(w[ks]);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+          for (int T_ = 0; T_ < 4; ++T_) {
+            pr[T_] = MF<T>::mma(a[T_][ks].x, x[ks].x, pr[T_]);
+            pi[T_] = MF<T>::mma(a[T_][ks].x, x[ks].y, pi[T_]);
+            pr[T_] = MF<T>::mma(-a[T_][ks].y, x[ks].y, pr[T_]);
+            pi[T_] = MF<T>::mma(a[T_][ks].y, x[ks].x, pi[T_]);
+          }
       }
 #pragma unroll
-      for (int r = 0; r < 32; ++r)
-        if (r < jw) sb[(j0 + r) * TSB_BS + t] = x[r];
-    }
-    __syncthreads();
-    // the block's other rows: below the sub-block (L), above it (U)
-    const int u0 = LOWER ? j0 + jw : 0, u1 = LOWER ? w : j0, c = t % TSB_SW;
-    if (u1 > u0) {
-      cT x[32];
+      for (int T_ = 0; T_ < 4; ++T_)
 #pragma unroll
-      for (int k = 0; k < 32; ++k) x[k] = (k < jw) ? sb[(j0 + k) * TSB_BS + c] : cT{0, 0};
-      if constexpr (sizeof(T) == 4) {
-        // two rows per step, each in two partial sums
-        constexpr int RS = TSB_THREADS / TSB_SW;
-        for (int r = u0 + t / TSB_SW; r < u1; r += 2 * RS) {
-          const int r2 = r + RS;
-          const bool two = r2 < u1;
-          cT a0 = cT{0, 0}, a1 = cT{0, 0}, b0 = cT{0, 0}, b1 = cT{0, 0};
+        for (int e = 0; e < 4; ++e)
+          S[(wave * TR_B + 16 * T_ + MF<T>::row(lk, e)) * TR_XS + lr] = cT{pr[T_][e], pi[T_][e]};
+      __syncthreads();
 #pragma unroll
-          for (int k = 0; k < 32; k += 2) {
-            const cT l0 = sp[r * TSB_SS + k], l1 = sp[r * TSB_SS + k + 1];
-            const cT m0 = two ? sp[r2 * TSB_SS + k] : cT{0, 0}, m1 = two ? sp[r2 * TSB_SS + k + 1] : cT{0, 0};
-            a0 = cT{a0.x + (l0.x * x[k].x - l0.y * x[k].y), a0.y + (l0.x * x[k].y + l0.y * x[k].x)};
-            a1 = cT{a1.x + (l1.x * x[k + 1].x - l1.y * x[k + 1].y), a1.y + (l1.x * x[k + 1].y + l1.y * x[k + 1].x)};
-            b0 = cT{b0.x + (m0.x * x[k].x - m0.y * x[k].y), b0.y + (m0.x * x[k].y + m0.y * x[k].x)};
-            b1 = cT{b1.x + (m1.x * x[k + 1].x - m1.y * x[k + 1].y), b1.y + (m1.x * x[k + 1].y + m1.y * x[k + 1].x)};
-          }
-          cT &y = sb[r * TSB_BS + c];
-          y = cT{y.x - (a0.x + a1.x), y.y - (a0.y + a1.y)};
-          if (two) {
-            cT &y2 = sb[r2 * TSB_BS + c];
-            y2 = cT{y2.x - (b0.x + b1.x), y2.y - (b0.y + b1.y)};
-          }
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const cT v = S[(k * TR_B + 16 * wave + MF<T>::row(lk, e)) * TR_XS + lr];
+          rr[e] -= v.x;
+          ri[e] -= v.y;
         }
-      } else {   // FP64: one row per step (the two-row form exceeds the registers)
-        for (int r = u0 + t / TSB_SW; r < u1; r += TSB_THREADS / TSB_SW) {
-          cT acc = cT{0, 0};
+      // times the inverse, 16 rows per wave, the triangle's columns only; shared in
+      // sums that no other wave reads
+      auto shared = [&](int r) { return S + (long)((r >> 4) * TR_B + r) * TR_XS + lr; };
 #pragma unroll
-          for (int k = 0; k < 32; ++k) {
-            const cT l = sp[r * TSB_SS + k];
-            acc = cT{acc.x + (l.x * x[k].x - l.y * x[k].y), acc.y + (l.x * x[k].y + l.y * x[k].x)};
-          }
-          cT &y = sb[r * TSB_BS + c];
-          y = cT{y.x - acc.x, y.y - acc.y};
+      for (int e = 0; e < 4; ++e) *shared(16 * wave + MF<T>::row(lk, e)) = cT{rr[e], ri[e]};
+      __syncthreads();
+      acc_t yr = acc_t{0, 0, 0, 0}, yi = acc_t{0, 0, 0, 0};
+#pragma unroll 4
+      for (int ks = UPPER ? 4 * wave : 0; ks < (UPPER ? 16 : 4 * wave + 4); ++ks) {
+        const cT a = V[(16 * wave + lr) * TR_VS + 4 * ks + lk], x = *shared(4 * ks + lk);
+        yr = MF<T>::mma(a.x, x.x, yr);
+        yi = MF<T>::mma(a.x, x.y, yi);
+        yr = MF<T>::mma(-a.y, x.y, yr);
+        yi = MF<T>::mma(a.y, x.x, yi);
+      }
+      if (lr < cs) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = rw + MF<T>::row(lk, e);
+          const cT v = cT{yr[e], yi[e]};
+          tr_publish<T>(X + ((long)r * cs + lr) * EW, tag, v);
+          if (UPPER && r < n && lr < nc) B[(long)r * ldb + lr] = v;
         }
       }
+      __syncthreads();
     }
-  }
-  __syncthreads();
-  for (int e = t; e < w * TSB_SW; e += TSB_THREADS) {
-    const int r = e / TSB_SW, c = e % TSB_SW;
-    if (c < nc) B[(long)r * ldb + c0 + c] = sb[r * TSB_BS + c];
-  }
+  };
+  sweep(std::false_type{});
+  sweep(std::true_type{});
 }
 template <class T>
-static void tsb_prepare() {
+static void tr_prepare() {
   static std::once_flag once;
   std::call_once(once, [] {
-    HIPCHK(hipFuncSetAttribute((const void *)k_trsm_blk<T, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)tsb_lds<T>()));
-    HIPCHK(hipFuncSetAttribute((const void *)k_trsm_blk<T, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)tsb_lds<T>()));
+    HIPCHK(hipFuncSetAttribute((const void *)k_tri<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)tr_lds<T>()));
   });
 }
+template <class T> static size_t getrs_ws_bytes(int n, int nrhs, int batch) {
+  return (size_t)batch * tr_ws_bytes<T>(n, nrhs);
+}
 
-// B (n x nrhs, ldb) <- A^{-1} B given LU and the row permutation.
+// B (n x nrhs, ldb) <- A^{-1} B given LU and the row permutation. ws:
+// getrs_ws_bytes<T>(n, nrhs, batch) bytes.
 template <class T>
 static void getrs_batched(int n, int nrhs, int batch, const typename C2<T>::t *LU, long lda, long sA,
-                          const int *perm, long sP, typename C2<T>::t *B, long ldb, long sB,
-                          typename C2<T>::t *work, long sW, hipStream_t s) {
-  typedef typename C2<T>::t cT;
-  const dim3 b256(256);
-  const long tot = (long)n * nrhs;
-  // work <- P B, then forward / backward substitution in place on work, copy back.
-  QH_LAUNCH(k_gather_rows<T>, dim3(qh_stride_blocks(tot), 1, batch), b256, 0, s, n, nrhs, perm, sP,
-                     (const cT *)B, ldb, sB, work, (long)nrhs, sW);
-  if (nrhs <= TRV_R) {
-    const int nblk = (n + TRV_W - 1) / TRV_W;
-    for (int bi = 0; bi < nblk; ++bi) {
-      const int r0 = bi * TRV_W, w = min(TRV_W, n - r0), rem = n - r0 - w;
-      QH_LAUNCH((k_trsv_wave<T, true>), dim3(1, 1, batch), dim3(TRV_W), 0, s, r0, w, nrhs, LU, lda, sA, work, sW);
-      if (rem > 0)
-        QH_LAUNCH(k_trsv_update<T>, dim3((rem + 63) / 64, 1, batch), dim3(64), 0, s, r0 + w, rem, r0, w, nrhs,
-                           LU, lda, sA, work, sW);
-    }
-    for (int bi = nblk - 1; bi >= 0; --bi) {
-      const int r0 = bi * TRV_W, w = min(TRV_W, n - r0);
-      QH_LAUNCH((k_trsv_wave<T, false>), dim3(1, 1, batch), dim3(TRV_W), 0, s, r0, w, nrhs, LU, lda, sA, work, sW);
-      if (r0 > 0)
-        QH_LAUNCH(k_trsv_update<T>, dim3((r0 + 63) / 64, 1, batch), dim3(64), 0, s, 0, r0, r0, w, nrhs, LU, lda,
-                           sA, work, sW);
-    }
-    QH_LAUNCH(k_copy_rows<T>, dim3(qh_stride_blocks(tot), 1, batch), b256, 0, s, n, nrhs,
-                       (const cT *)work, (long)nrhs, sW, B, ldb, sB);
-    HIPCHK(hipGetLastError());
-    return;
-  }
-  tsb_prepare<T>();
-  const dim3 gs((nrhs + TSB_SW - 1) / TSB_SW, 1, batch);
-  for (int r0 = 0; r0 < n; r0 += TsbRows<T>::R) {
-    const int w = min(TsbRows<T>::R, n - r0);
-    QH_LAUNCH((k_trsm_blk<T, true>), gs, dim3(TSB_THREADS), tsb_lds<T>(), s, w, nrhs, LU + (long)r0 * lda + r0, lda, sA,
-              work + (long)r0 * nrhs, (long)nrhs, sW);
-    const int rem = n - r0 - w;
-    if (rem > 0)
-      QH_LAUNCH(k_gemm_sub<T>, dim3((nrhs + GT - 1) / GT, (rem + GT - 1) / GT, batch), b256, 0, s, rem, nrhs, w,
-                         LU + (long)(r0 + w) * lda + r0, lda, sA, (const cT *)(work + (long)r0 * nrhs), (long)nrhs, sW,
-                         work + (long)(r0 + w) * nrhs, (long)nrhs, sW);
-  }
-  const int nblk = (n + TsbRows<T>::R - 1) / TsbRows<T>::R;
-  for (int bi = nblk - 1; bi >= 0; --bi) {
-    const int r0 = bi * TsbRows<T>::R, w = min(TsbRows<T>::R, n - r0);
-    QH_LAUNCH((k_trsm_blk<T, false>), gs, dim3(TSB_THREADS), tsb_lds<T>(), s, w, nrhs, LU + (long)r0 * lda + r0, lda, sA,
-              work + (long)r0 * nrhs, (long)nrhs, sW);
-    if (r0 > 0)
-      QH_LAUNCH(k_gemm_sub<T>, dim3((nrhs + GT - 1) / GT, (r0 + GT - 1) / GT, batch), b256, 0, s, r0, nrhs, w,
-                         LU + r0, lda, sA, (const cT *)(work + (long)r0 * nrhs), (long)nrhs, sW, work, (long)nrhs, sW);
-  }
-  // copy back (B may have a different leading dimension), one launch for the batch
-  QH_LAUNCH(k_copy_rows<T>, dim3(qh_stride_blocks(tot), 1, batch), b256, 0, s, n, nrhs,
-                     (const cT *)work, (long)nrhs, sW, B, ldb, sB);
+                          const int *perm, long sP, typename C2<T>::t *B, long ldb, long sB, void *ws, hipStream_t s,
+                          st_u64 wait = ST_LIMIT) {
+  if (n <= 0 || nrhs <= 0 || batch <= 0) return;
+  tr_prepare<T>();
+  const int nblk = (n + TR_B - 1) / TR_B, nslab = (nrhs + TR_C - 1) / TR_C;
+  const long slabb = (long)((tr_slab_bytes<T>(n, nrhs) + 255) / 256 * 256), sW = slabb * nslab;
+  qh_zero(ws, (size_t)batch * sW, s);
+  // A workgroup's next block, up to nblk products of 64 x 64 blocks (2 us each),
+  // has to be ready when the chain (4 to 7 us a block) gets there: nblk / 4 of
+  // them keep up. A quarter of those the device holds (256 in FP64, 512 in FP32)
+  // leaves room for the solves of other streams, whose workgroups wait for one
+  // another too, hence no more than that for small systems, in batches either.
+  const long quarter = sizeof(T) == 8 ? 64 : 128;
+  const long room = std::min((long)TR_MEET, std::max(quarter, (long)nslab * nblk / 4));
+  const int G = (int)std::max(1L, std::min((long)nblk, room / ((long)nslab * batch)));
+  QH_LAUNCH(k_tri<T>, dim3(G, nslab, batch), dim3(256), tr_lds<T>(), s, n, nrhs, LU, lda, sA, perm, sP, B, ldb, sB,
+            (char *)ws, sW, slabb, wait);
   HIPCHK(hipGetLastError());
 }
 
@@ -2579,14 +2601,14 @@ extern "C" int qpms_hip_zgetrf_dev_noalloc(size_t n, _Complex double *A_dev, int
 extern "C" int qpms_hip_zgetrs_dev(size_t n, size_t nrhs, const _Complex double *LU_dev, const int *ipiv_dev,
                                    _Complex double *B_dev, void *stream) {
   hipStream_t s = (hipStream_t)qh_stream(stream);
-  int *perm = (int *)qh_dmalloc(n * sizeof(int));
-  v2d *work = (v2d *)qh_dmalloc(n * nrhs * sizeof(v2d));
-  QH_LAUNCH(k_perm_from_ipiv, dim3(1), dim3(64), 0, s, (int)n, ipiv_dev, perm);
-  getrs_batched<double>((int)n, (int)nrhs, 1, (const v2d *)LU_dev, (long)n, 0, perm, 0, (v2d *)B_dev, (long)nrhs, 0,
-                        work, 0, s);
+  if (n == 0 || nrhs == 0) return 0;
+  const size_t wb = getrs_ws_bytes<double>((int)n, (int)nrhs, 1);
+  char *ws = (char *)qh_dmalloc(wb + n * sizeof(int));
+  int *perm = (int *)(ws + wb);
+  QH_LAUNCH(k_perm_from_ipiv, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, s, (int)n, ipiv_dev, perm);
+  getrs_batched<double>((int)n, (int)nrhs, 1, (const v2d *)LU_dev, (long)n, 0, perm, 0, (v2d *)B_dev, (long)nrhs, 0, ws, s);
   HIPCHK(hipStreamSynchronize(s));
-  qh_dfree(perm);
-  qh_dfree(work);
+  qh_dfree(ws);
   return 0;
 }
 
@@ -2640,10 +2662,48 @@ extern "C" int qh_getrf_batched_wsla_f64(int n, int batch, double *A, long sA, i
                         lookahead != 0);
   return 0;
 }
-extern "C" int qh_getrs_batched_f64(int n, int nrhs, int batch, const double *LU, long sA, const int *perm,
-                                    double *B, long sB, double *work, void *stream) {
-  getrs_batched<double>(n, nrhs, batch, (const v2d *)LU, n, sA, perm, n, (v2d *)B, nrhs, sB, (v2d *)work,
-                        (long)n * nrhs, (hipStream_t)qh_stream(stream));
+// Solves with batched factorisations. The workspace form neither allocates nor
+// waits.
+extern "C" size_t qh_getrs_ws_bytes(int prec, int n, int nrhs, int batch) {
+  return prec == 32 ? getrs_ws_bytes<float>(n, nrhs, batch) : getrs_ws_bytes<double>(n, nrhs, batch);
+}
+extern "C" int qh_getrs_ws_f64(int n, int nrhs, int batch, const double *LU, long sA, const int *perm, double *B,
+                               long sB, void *ws, void *stream) {
+  getrs_batched<double>(n, nrhs, batch, (const v2d *)LU, n, sA, perm, n, (v2d *)B, nrhs, sB, ws,
+                        (hipStream_t)qh_stream(stream));
+  return 0;
+}
+extern "C" int qh_getrs_ws_f32(int n, int nrhs, int batch, const float *LU, long sA, const int *perm, float *B, long sB,
+                               void *ws, void *stream) {
+  getrs_batched<float>(n, nrhs, batch, (const v2f *)LU, n, sA, perm, n, (v2f *)B, nrhs, sB, ws,
+                       (hipStream_t)qh_stream(stream));
+  return 0;
+}
+// The same for matrices one behind the other, with the limit of the slabs'
+// rendezvous (0: one workgroup takes the slab unless it sees the others at once).
+// Tests reach both ways through a solve with it.
+extern "C" int qh_getrs_wait(int prec, int n, int nrhs, int batch, const double *LU, const int *perm, double *B,
+                             unsigned long long wait, void *stream) {
+  hipStream_t s = (hipStream_t)qh_stream(stream);
+  void *ws = qh_dmalloc(qh_getrs_ws_bytes(prec, n, nrhs, batch));
+  const long sA = (long)n * n, sB = (long)n * nrhs;
+  if (prec == 32)
+    getrs_batched<float>(n, nrhs, batch, (const v2f *)LU, n, sA, perm, n, (v2f *)B, nrhs, sB, ws, s, wait);
+  else
+    getrs_batched<double>(n, nrhs, batch, (const v2d *)LU, n, sA, perm, n, (v2d *)B, nrhs, sB, ws, s, wait);
+  HIPCHK(hipStreamSynchronize(s));
+  qh_dfree(ws);
+  return 0;
+}
+// (work: n x nrhs x batch entries of scratch, as an earlier form of the solve
+// needed; its own words are allocated here)
+extern "C" int qh_getrs_batched_f64(int n, int nrhs, int batch, const double *LU, long sA, const int *perm, double *B, long sB,
+                                    double *work, void *stream) {
+  (void)work;
+  void *ws = qh_dmalloc(getrs_ws_bytes<double>(n, nrhs, batch));
+  qh_getrs_ws_f64(n, nrhs, batch, LU, sA, perm, B, sB, ws, stream);
+  HIPCHK(hipStreamSynchronize((hipStream_t)qh_stream(stream)));
+  qh_dfree(ws);
   return 0;
 }
 extern "C" int qh_getrf_batched_f32(int n, int batch, float *A, long sA, int *ipiv, int *perm, int *info,
@@ -2651,10 +2711,15 @@ extern "C" int qh_getrf_batched_f32(int n, int batch, float *A, long sA, int *ip
   getrf_batched<float>(n, batch, (v2f *)A, n, sA, ipiv, n, perm, info, (hipStream_t)qh_stream(stream));
   return 0;
 }
-extern "C" int qh_getrs_batched_f32(int n, int nrhs, int batch, const float *LU, long sA, const int *perm,
-                                    float *B, long sB, float *work, void *stream) {
-  getrs_batched<float>(n, nrhs, batch, (const v2f *)LU, n, sA, perm, n, (v2f *)B, nrhs, sB, (v2f *)work,
-                       (long)n * nrhs, (hipStream_t)qh_stream(stream));
+// (work: n x nrhs x batch entries of scratch, as an earlier form of the solve
+// needed; its own words are allocated here)
+extern "C" int qh_getrs_batched_f32(int n, int nrhs, int batch, const float *LU, long sA, const int *perm, float *B, long sB,
+                                    float *work, void *stream) {
+  (void)work;
+  void *ws = qh_dmalloc(getrs_ws_bytes<float>(n, nrhs, batch));
+  qh_getrs_ws_f32(n, nrhs, batch, LU, sA, perm, B, sB, ws, stream);
+  HIPCHK(hipStreamSynchronize((hipStream_t)qh_stream(stream)));
+  qh_dfree(ws);
   return 0;
 }
 // C -= A B (FP64 complex, batched, row-major, packed leading dimensions)
@@ -2732,7 +2797,7 @@ extern "C" int qpms_hip_solve_mixed_dev(size_t n_, size_t nrhs_, const _Complex 
   int *dinfo = (int *)qh_dmalloc(sizeof(int));
   double *R = (double *)qh_dmalloc(nb * sizeof(v2d));
   float *R32 = (float *)qh_dmalloc(nb * sizeof(v2f));
-  float *W32 = (float *)qh_dmalloc(nb * sizeof(v2f));
+  void *W32 = qh_dmalloc(getrs_ws_bytes<float>(n, nrhs, 1));
   HIPCHK(hipMemsetAsync(dinfo, 0, sizeof(int), s));
   qh_d2f(nn, (const double *)A_dev, A32, s);
   getrf_batched<float>(n, 1, (v2f *)A32, n, 0, ipiv, 0, perm, dinfo, s);
@@ -2744,7 +2809,7 @@ extern "C" int qpms_hip_solve_mixed_dev(size_t n_, size_t nrhs_, const _Complex 
   qh_copy_c64(nb, (const double *)B_dev, R, s);
   for (it = 0; it < maxit; ++it) {
     qh_d2f(nb, R, R32, s);
-    getrs_batched<float>(n, nrhs, 1, (const v2f *)A32, n, 0, perm, 0, (v2f *)R32, nrhs, 0, (v2f *)W32, 0, s);
+    getrs_batched<float>(n, nrhs, 1, (const v2f *)A32, n, 0, perm, 0, (v2f *)R32, nrhs, 0, W32, s);
     qh_f2d_add(nb, R32, (double *)X_dev, s);
     // R = B - A X
     qh_copy_c64(nb, (const double *)B_dev, R, s);
@@ -2767,12 +2832,12 @@ extern "C" int qpms_hip_solve_mixed_dev(size_t n_, size_t nrhs_, const _Complex 
   int *ip = (int *)qh_dmalloc(n * sizeof(int));
   int *pm = (int *)qh_dmalloc(n * sizeof(int));
   int *inf = (int *)qh_dmalloc(sizeof(int));
-  double *work = (double *)qh_dmalloc(nb * sizeof(v2d));
+  void *work = qh_dmalloc(getrs_ws_bytes<double>(n, nrhs, 1));
   HIPCHK(hipMemsetAsync(inf, 0, sizeof(int), s));
   qh_copy_c64(nn, (const double *)A_dev, A64, s);
   qh_copy_c64(nb, (const double *)B_dev, (double *)X_dev, s);
   getrf_batched<double>(n, 1, (v2d *)A64, n, 0, ip, 0, pm, inf, s);
-  getrs_batched<double>(n, nrhs, 1, (const v2d *)A64, n, 0, pm, 0, (v2d *)X_dev, nrhs, 0, (v2d *)work, 0, s);
+  getrs_batched<double>(n, nrhs, 1, (const v2d *)A64, n, 0, pm, 0, (v2d *)X_dev, nrhs, 0, work, s);
   HIPCHK(hipStreamSynchronize(s));
   qh_dfree(A64); qh_dfree(ip); qh_dfree(pm); qh_dfree(inf); qh_dfree(work);
   return -1;

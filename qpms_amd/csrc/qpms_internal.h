@@ -77,6 +77,12 @@ int qh_getrs_batched_f64(int n, int nrhs, int batch, const double *LU, long sA, 
 int qh_getrf_batched_f32(int n, int batch, float *A, long sA, int *ipiv, int *perm, int *info, void *stream);
 int qh_getrs_batched_f32(int n, int nrhs, int batch, const float *LU, long sA, const int *perm,
 		float *B, long sB, float *work, void *stream);
+/* The same with caller's scratch of qh_getrs_ws_bytes (prec 32, 64): no allocation, no wait. */
+size_t qh_getrs_ws_bytes(int prec, int n, int nrhs, int batch);
+int qh_getrs_ws_f64(int n, int nrhs, int batch, const double *LU, long sA, const int *perm,
+		double *B, long sB, void *ws, void *stream);
+int qh_getrs_ws_f32(int n, int nrhs, int batch, const float *LU, long sA, const int *perm,
+		float *B, long sB, void *ws, void *stream);
 int qh_gemm_sub_f64(int M, int N, int K, int batch, const double *A, long lda, long sA, const double *B,
 		long ldb, long sB, double *C, long ldc, long sC, void *stream);
 int qh_gemm_sub_f32(int M, int N, int K, int batch, const float *A, long lda, long sA, const float *B,

@@ -196,8 +196,9 @@ typedef struct {
 	 * node chunks are enqueued one at a time from the progress loop */
 	complex double *dA0, *dA1, *dA0c, *dA1c;
 	int chunk, next_node, cancelled;
-	double *bV, *bM, *bX, *bR, *bW, *btd, *bpos;
-	float *bM32, *bR32, *bW32;
+	double *bV, *bM, *bX, *bR, *btd, *bpos;
+	float *bM32, *bR32;
+	void *bW;
 	int *bipiv, *bperm, *binfo, *btt;
 	void *bws, *btail;
 	beyn_contour_t *bcont;
@@ -253,8 +254,9 @@ static size_t scatter_bytes(const qpms_hip_server_t *s, size_t npad, int batch, 
 	size_t b = 0;
 	b += align256(batch * nn * 16);                    /* M (FP64) */
 	if (s->o.mixed) b += align256(batch * nn * 8);     /* M (FP32) */
-	b += 5 * align256(batch * npad * 16);              /* a, b, x, r, work */
-	b += 2 * align256(batch * npad * 8);               /* r32, w32 */
+	b += 4 * align256(batch * npad * 16);              /* a, b, x, r */
+	if (s->o.mixed) b += align256(batch * npad * 8);   /* r32 */
+	b += align256(qh_getrs_ws_bytes(s->o.mixed ? 32 : 64, (int)npad, 1, batch));
 	b += 2 * align256(batch * npad * 4) + align256(batch * 4);
 	b += align256(qh_getrf_ws_bytes(s->o.mixed ? 32 : 64, (int)npad, batch));
 	b += align256(batch * QH_SUMSQ_PARTS * 8);         /* norm partial sums */
@@ -274,8 +276,8 @@ static size_t periodic_bytes(size_t L, size_t np, int nsc, size_t nR, size_t nK)
 }
 
 static size_t beyn_node_bytes(const qpms_hip_server_t *s, size_t L, size_t l) {
-	return align256(L * L * 16) + (s->o.mixed ? align256(L * L * 8) : 0) + 4 * align256(L * l * 16)
-		+ 2 * align256(L * l * 8) + 2 * align256(L * 4) + 1024;
+	return align256(L * L * 16) + (s->o.mixed ? align256(L * L * 8) + align256(L * l * 8) : 0) + 2 * align256(L * l * 16)
+		+ align256(qh_getrs_ws_bytes(s->o.mixed ? 32 : 64, (int)L, (int)l, 1)) + 2 * align256(L * 4) + 1024;
 }
 /* A contour of N nodes handled `chunk` nodes at a time: per-chunk matrices and
  * workspaces, the probe and moment blocks, and per-node Mie parameters and
@@ -526,8 +528,9 @@ static void launch_scatter(qpms_hip_server_t *s, qh_unit *u, hipStream_t st) {
 	double *M = bump(&bp, B * nn * 16);
 	float *M32 = s->o.mixed ? bump(&bp, B * nn * 8) : NULL;
 	double *a = bump(&bp, B * npad * 16), *b = bump(&bp, B * npad * 16), *x = bump(&bp, B * npad * 16);
-	double *r = bump(&bp, B * npad * 16), *work = bump(&bp, B * npad * 16);
-	float *r32 = bump(&bp, B * npad * 8), *w32 = bump(&bp, B * npad * 8);
+	double *r = bump(&bp, B * npad * 16);
+	float *r32 = s->o.mixed ? bump(&bp, B * npad * 8) : NULL;
+	void *work = bump(&bp, qh_getrs_ws_bytes(s->o.mixed ? 32 : 64, (int)npad, 1, B));
 	int *ipiv = bump(&bp, B * npad * 4), *perm = bump(&bp, B * npad * 4), *info = bump(&bp, B * 4);
 	void *ws = bump(&bp, qh_getrf_ws_bytes(s->o.mixed ? 32 : 64, (int)npad, B));
 	double *outs = bump(&bp, B * 8 * 8);   /* per job: dot, |r|^2, |x|^2, |M|^2, info */
@@ -577,7 +580,7 @@ static void launch_scatter(qpms_hip_server_t *s, qh_unit *u, hipStream_t st) {
 		qh_copy_c64((long)(B * npad), b, r, st);
 		for (int it = 0; it < s->o.refine_steps; ++it) {
 			qh_d2f((long)(B * npad), r, r32, st);
-			qh_getrs_batched_f32((int)npad, 1, B, M32, sM, perm, r32, sV, w32, st);
+			qh_getrs_ws_f32((int)npad, 1, B, M32, sM, perm, r32, sV, work, st);
 			qh_f2d_add((long)(B * npad), r32, x, st);
 			qh_copy_c64((long)(B * npad), b, r, st);
 			qh_gemm_sub_f64((int)npad, 1, (int)npad, B, M, (long)npad, sM, x, 1, sV, r, 1, sV, st);
@@ -587,7 +590,7 @@ static void launch_scatter(qpms_hip_server_t *s, qh_unit *u, hipStream_t st) {
 		 * so the residual uses the factors' reconstruction bound instead. */
 		qh_getrf_batched_wsla_f64((int)npad, B, M, sM, ipiv, perm, info, ws, npad >= SRV_LOOKAHEAD_MIN, st);
 		qh_copy_c64((long)(B * npad), b, x, st);
-		qh_getrs_batched_f64((int)npad, 1, B, M, sM, perm, x, sV, work, st);
+		qh_getrs_ws_f64((int)npad, 1, B, M, sM, perm, x, sV, work, st);
 		qh_zero(r, B * npad * 16, st);
 	}
 	qh_launch_sumsq_batched(B, (long)npad, r, sV, part, outs + B, st);
@@ -766,8 +769,9 @@ static void launch_beyn(qpms_hip_server_t *s, qh_unit *u, hipStream_t st, int ch
 	u->bws = bump(&bp, qh_getrf_ws_bytes(s->o.mixed ? 32 : 64, (int)L, chunk));
 	u->bM = bump(&bp, chunk * L * L * 16);
 	u->bM32 = s->o.mixed ? bump(&bp, chunk * L * L * 8) : NULL;
-	u->bX = bump(&bp, chunk * L * l * 16); u->bR = bump(&bp, chunk * L * l * 16); u->bW = bump(&bp, chunk * L * l * 16);
-	u->bR32 = bump(&bp, chunk * L * l * 8); u->bW32 = bump(&bp, chunk * L * l * 8);
+	u->bX = bump(&bp, chunk * L * l * 16); u->bR = bump(&bp, chunk * L * l * 16);
+	u->bR32 = s->o.mixed ? bump(&bp, chunk * L * l * 8) : NULL;
+	u->bW = bump(&bp, qh_getrs_ws_bytes(s->o.mixed ? 32 : 64, (int)L, (int)l, chunk));
 	u->bipiv = bump(&bp, chunk * L * 4); u->bperm = bump(&bp, chunk * L * 4); u->binfo = bump(&bp, chunk * 4);
 	u->btt = bump(&bp, np * 4);
 	double *dprm = bump(&bp, N * 9 * 8), *mie = bump(&bp, N * 2 * (lMax + 1) * 16);
@@ -833,7 +837,7 @@ static void beyn_chunk_body(qpms_hip_server_t *s, qh_unit *u, hipStream_t st, in
 		/* nodes near an eigenvalue make M ill-conditioned: twice the steps of a solve */
 		for (int it = 0; it < 2 * s->o.refine_steps; ++it) {
 			qh_d2f((long)(C * L * l), R, u->bR32, st);
-			qh_getrs_batched_f32((int)L, (int)l, C, u->bM32, sM, u->bperm, u->bR32, sV, u->bW32, st);
+			qh_getrs_ws_f32((int)L, (int)l, C, u->bM32, sM, u->bperm, u->bR32, sV, u->bW, st);
 			qh_f2d_add((long)(C * L * l), u->bR32, X, st);
 			for (int i = 0; i < C; ++i) qh_copy_c64((long)(L * l), u->bV, R + i * sV * 2, st);
 			qh_gemm_sub_f64((int)L, (int)l, (int)L, C, M, (long)L, sM, X, (long)l, sV, R, (long)l, sV, st);
@@ -841,7 +845,7 @@ static void beyn_chunk_body(qpms_hip_server_t *s, qh_unit *u, hipStream_t st, in
 	} else {
 		qh_getrf_batched_wsla_f64((int)L, C, M, sM, u->bipiv, u->bperm, u->binfo, u->bws, L >= SRV_LOOKAHEAD_MIN, st);
 		for (int i = 0; i < C; ++i) qh_copy_c64((long)(L * l), u->bV, X + i * sV * 2, st);
-		qh_getrs_batched_f64((int)L, (int)l, C, M, sM, u->bperm, X, sV, u->bW, st);
+		qh_getrs_ws_f64((int)L, (int)l, C, M, sM, u->bperm, X, sV, u->bW, st);
 	}
 	for (int i = 0; i < C; ++i)
 		qh_beyn_accum_node((long)(L * l), X + i * sV * 2, u->btab, u->bcur, i, (double *)u->dA0, (double *)u->dA1,
