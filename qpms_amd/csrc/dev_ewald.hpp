@@ -29,6 +29,75 @@ namespace qew {
 
 constexpr int WEID_N = 32;
 
+// exp, sin and cos, and a reciprocal, for loops whose registers are sums: the
+// library's keep their polynomials' coefficients in vector registers over the loop
+// (or in scratch, where those do not suffice), evaluate sin and cos apart, and
+// carry paths for every argument. Here the coefficients, those of the Taylor
+// series, come through scalar loads each time. Errors below 1.5 units in the last
+// place.
+struct Taylor {
+  double s[8], c[9], e[14];   // (-1)^i / (2i+3)!, (-1)^(i+1) / (2i+2)!, 1 / i!
+};
+constexpr Taylor taylor_table() {
+  Taylor t{};
+  double f = 1.0;   // i!: exact up to 18!
+  for (int i = 0; i <= 19; ++i) {
+    if (i > 0) f *= i;
+    if (i < 14) t.e[i] = 1.0 / f;
+    if (i >= 2 && i % 2 == 0) t.c[i / 2 - 1] = ((i / 2) % 2 ? -1.0 : 1.0) / f;
+    if (i >= 3 && i % 2 == 1 && (i - 3) / 2 < 8) t.s[(i - 3) / 2] = ((i - 1) / 2 % 2 ? -1.0 : 1.0) / f;
+  }
+  return t;
+}
+#if defined(__HIPCC__)
+__device__ constexpr Taylor g_taylor = taylor_table();
+__device__ __forceinline__ const Taylor *taylor() {
+  const Taylor *t = &g_taylor;
+  asm volatile("" : "+s"(t));   // read again each time
+  return t;
+}
+
+// x != 0, normal and not close to the limits of the range
+__device__ __forceinline__ double rcp_(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+
+__device__ __forceinline__ double exp_(double x) {
+  const Taylor *t = taylor();
+  x = x > 1100.0 ? 1100.0 : x < -1100.0 ? -1100.0 : x;   // inf and 0 by the scaling; NaN stays
+  const double n = rint(x * 1.4426950408889634074);
+  double r = fma(n, -6.9314718055994530942e-1, x);        // ln 2 to double
+  r = fma(n, -2.3190468138462995584e-17, r);              // and the rest of it
+  double p = t->e[13];
+#pragma unroll
+  for (int i = 12; i >= 0; --i) p = fma(p, r, t->e[i]);
+  return ldexp(p, (int)n);
+}
+
+// e^{i x}: x - n pi/2 by two fused steps (the first one is exact), |x| < 1e9, else
+// the library's.
+__device__ __forceinline__ cplx expi_(double x) {
+  if (__any(!(fabs(x) < 1e9))) return cexpi(x);
+  const Taylor *t = taylor();
+  const double n = rint(x * 0.63661977236758134308);
+  double r = fma(n, -1.5707963267948965580, x);           // pi/2 to double
+  r = fma(n, -6.1232339957367658861e-17, r);              // and the rest of it
+  const double z = r * r;
+  double s = t->s[7], c = t->c[8];
+#pragma unroll
+  for (int i = 6; i >= 0; --i) s = fma(s, z, t->s[i]);
+#pragma unroll
+  for (int i = 7; i >= 0; --i) c = fma(c, z, t->c[i]);
+  s = fma(s * z, r, r);
+  c = fma(c, z, 1.0);
+  const int q = (int)n;
+  const double a = q & 1 ? s : c, b = q & 1 ? c : s;   // cos, sin up to their signs
+  return mk((q + 1) & 2 ? -a : a, q & 2 ? -b : b);
+}
+#endif
+
 QPMS_HD inline cplx cexp2(cplx z) { return cexp_(z); }
 
 // Faddeeva w(z) for Im z >= 0 given the Weideman coefficients a[0..N-1] (a_1..a_N).
@@ -76,6 +145,39 @@ QPMS_HD inline void sr_integrals(double R, cplx k, double eta, const double *wa,
     etap *= eta * eta;
   }
 }
+
+// The same for real k, R > 0: with real kappa w(-kappa + i R eta) is the conjugate
+// of w(kappa + i R eta), so one expansion serves both and every I_n is real.
+#if defined(__HIPCC__)
+template <int NMAX>
+__device__ __forceinline__ void sr_integrals_real(double R, double k, double eta, const double *wa, double *out) {
+  const double kap = k / (2.0 * eta), Re = R * eta;
+  const double F = exp_(kap * kap - Re * Re);
+  const double L = 4.7568284600108841;                         // sqrt(32 / sqrt(2))
+  const double den = L + Re, f = rcp_(den * den + kap * kap);
+  const cplx inv = mk(den * f, kap * f);                       // 1 / (L - iz)
+  const cplx Z = mk(L - Re, kap) * inv;
+  cplx p = mk(wa[WEID_N - 1], 0.0);
+#pragma unroll
+  for (int m = WEID_N - 2; m >= 0; --m)
+    p = mk(fma(p.re, Z.re, fma(-p.im, Z.im, wa[m])), fma(p.re, Z.im, p.im * Z.re));
+  const cplx w = inv * (2.0 * (p * inv) + mk(0.56418958354775628695, 0.0));   // 1/sqrt(pi)
+  const double sqpi = 1.7724538509055160273;
+  const double Jm1 = sqpi * w.im / k, iR = rcp_(R), J0 = (0.5 * sqpi) * iR * w.re;
+  const double hk2 = 0.5 * (k * k), inv2R2 = 0.5 * iR * iR;
+  out[0] = F * J0;
+  double etap = eta;  // eta^{2n-1}
+  double Jn2 = Jm1, Jn1 = J0;
+#pragma unroll
+  for (int n = 1; n <= NMAX; ++n) {
+    const double Jn = fma((double)(2 * n - 1), Jn1, fma(-hk2, Jn2, etap)) * inv2R2;
+    out[n] = F * Jn;
+    Jn2 = Jn1;
+    Jn1 = Jn;
+    etap *= eta * eta;
+  }
+}
+#endif
 
 // Gamma(a) for a = 1/2 - j.
 QPMS_HD inline double gamma_half(int j) {
@@ -143,6 +245,69 @@ QPMS_HD inline cplx gamma_inc_half(int j, cplx z, int m) {
   return val;
 }
 
+#if defined(__HIPCC__)
+// Gamma(1/2 - j, z), j = 0..J, for real z (Im z = +-0 chooses the side of the cut,
+// principal branch) by the series of gamma_inc_half: its sums are real and share
+// the reciprocals of the half-integers, one for each power of z.
+template <int J>
+__device__ __forceinline__ void gamma_inc_half_real_series(cplx z, cplx (&G)[J + 1]) {
+  double sum[J + 1], term[J + 1], r[J + 1];
+#pragma unroll
+  for (int j = 0; j <= J; ++j) {
+    term[j] = 1.0 / (gamma_half(j) * (0.5 - j));   // 1 / Gamma(a + 1)
+    sum[j] = 0.0;
+    r[j] = 1.0 / (1.5 - j);                        // 1 / (a + 1 + k)
+  }
+  for (int k = 0; k < 200; ++k) {
+    bool done = k > 4;
+#pragma unroll
+    for (int j = 0; j <= J; ++j) {
+      sum[j] += term[j];
+      done = done && fabs(term[j]) < 1e-17 * fabs(sum[j]);
+      term[j] *= z.re * r[j];
+    }
+    if (done) break;
+#pragma unroll
+    for (int j = J; j > 0; --j) r[j] = r[j - 1];
+    r[0] = rcp_(2.5 + k);
+  }
+  const double ez = exp_(-z.re);
+  const cplx zi = cinv(z);
+  cplx p = csqrt_(z);
+#pragma unroll
+  for (int j = 0; j <= J; ++j) {
+    G[j] = gamma_half(j) * (mk(1.0, 0.0) - p * (ez * sum[j]));
+    p = p * zi;
+  }
+}
+#endif
+
+#if defined(__HIPCC__)
+// Gamma(1/2 - j, z), j = 0..J, for Re z > 0.5 (principal branch): gamma_half_scaled
+// with w(i sqrt z) for complex z. The continued fraction takes 100-340 dependent
+// steps of two complex divisions near |z| = 1, for each j.
+template <int J>
+__device__ __forceinline__ void gamma_half_complex(cplx z, const double *a, cplx (&G)[J + 1]) {
+  const double L = 4.7568284600108841;  // sqrt(32 / sqrt(2))
+  const cplx s = csqrt_(z), den = mk(L + s.re, s.im);
+  const cplx inv = conj(den) * rcp_(cabs2(den)), Z = mk(L - s.re, -s.im) * inv;
+  cplx p = mk(a[WEID_N - 1], 0.0);
+#pragma unroll
+  for (int m = WEID_N - 2; m >= 0; --m)
+    p = mk(fma(p.re, Z.re, fma(-p.im, Z.im, a[m])), fma(p.re, Z.im, p.im * Z.re));
+  cplx E = 1.7724538509055160273 * (inv * (2.0 * (p * inv) + mk(0.56418958354775628695, 0.0)));
+  const cplx ez = exp_(-z.re) * expi_(-z.im), zi = cinv(z);
+  cplx za = s;   // z^{1/2 - j + 1} at step j
+  G[0] = E * ez;
+#pragma unroll
+  for (int j = 1; j <= J; ++j) {
+    za = za * zi;
+    E = (E - za) * (1.0 / (0.5 - j));
+    G[j] = E * ez;
+  }
+}
+#endif
+
 // Gamma(1/2 - j, x) for real x > 0.5 on the principal branch: the continued
 // fraction of gamma_inc_half in real arithmetic (every quantity is real
 // there), for the evanescent orders of a real wavenumber. Returns the
@@ -166,12 +331,13 @@ QPMS_HD inline double gamma_inc_half_real_cf(int j, double x) {
   return hn;
 }
 
+#if defined(__HIPCC__)
 // erfcx(y) = e^{y^2} erfc(y) = w(iy) for real y >= 0: Weideman's expansion on
 // the imaginary axis, where Z = (L - y) / (L + y) is real and the whole
 // evaluation is real arithmetic (32 FMAs, one division, no exponential).
-QPMS_HD inline double erfcx_pos(double y, const double *a) {
+__device__ __forceinline__ double erfcx_pos(double y, const double *a) {
   const double L = 4.7568284600108841;  // sqrt(32 / sqrt(2))
-  const double d = 1.0 / (L + y);
+  const double d = rcp_(L + y);
   const double Z = (L - y) * d;
   double p = a[WEID_N - 1];
   for (int m = WEID_N - 2; m >= 0; --m) p = fma(p, Z, a[m]);
@@ -186,17 +352,20 @@ QPMS_HD inline double erfcx_pos(double y, const double *a) {
 // so the absolute error of every term stays at the rounding of O(1) terms;
 // for x <= 8 the relative error is below 6e-13 for j <= 4. This replaces a
 // continued fraction that needs 100-340 dependent iterations near x = 1.
+// Of x the root sx and its reciprocal are given.
 template <int J>
-QPMS_HD inline void gamma_half_scaled(double x, const double *a, double (&E)[J + 1]) {
-  const double sx = sqrt(x), xi = 1.0 / x;
+__device__ __forceinline__ void gamma_half_scaled(double sx, double isx, const double *a, double (&E)[J + 1]) {
+  const double xi = isx * isx;
   E[0] = 1.7724538509055160273 * erfcx_pos(sx, a);
   double xa = sx;  // x^{a}, a = 1/2 - j + 1 at step j
 #pragma unroll
   for (int j = 1; j <= J; ++j) {
     xa *= xi;
-    E[j] = (E[j - 1] - xa) / (0.5 - j);
+    E[j] = (E[j - 1] - xa) * (1.0 / (0.5 - j));
   }
 }
+
+#endif
 
 QPMS_HD inline double gamma_inc_half_real(int j, double x) {
   return gamma_inc_half_real_cf(j, x) * exp((-0.5 - j) * log(x) - x);

@@ -17,6 +17,9 @@
 
 int qh_launch_sigma_short(int LE, int xy, int ntrip, const double *tr_dev, int npts, const double *pts_dev,
 		double eta, const double *leg0_dev, int csphase, double *out_dev, double *err_dev, void *stream);
+int qh_launch_sigma_both(int LE, int ntrip, const double *tr_dev, int nR, const double *R_dev, int nK,
+		const double *K_dev, double eta, double area, const double *leg0_dev, int csphase, double *short_dev,
+		double *long_dev, void *stream);
 int qh_launch_sigma_long(int LE, int ntrip, const double *tr_dev, int npts, const double *K_dev,
 		double eta, double area, const double *leg0_dev, double *out_dev, double *err_dev, void *stream);
 int qh_launch_sigma0(int n, const double *k_dev, double eta, double leg00, double *out_dev, void *stream);
@@ -88,6 +91,9 @@ int qpms_hip_ewald3_sigma_batch_dev(const qpms_ewald3_constants_t *c, double eta
 		_Complex double *sigma_short_dev, _Complex double *sigma_long_dev, void *stream) {
 	qh_check_le(c->lMax);
 	const qh_e3dev *e = qh_e3_get(c);
+	if (sigma_short_dev && sigma_long_dev)
+		return qh_launch_sigma_both(c->lMax, (int)ntrip, triples_dev, (int)nR, R_dev, (int)nK, K_dev, eta, unitcell_area,
+			e->leg0, c->legendre_csphase, (double *)sigma_short_dev, (double *)sigma_long_dev, stream);
 	if (sigma_short_dev)
 		qh_launch_sigma_short(c->lMax, 1, (int)ntrip, triples_dev, (int)nR, R_dev, eta, e->leg0,
 			c->legendre_csphase, (double *)sigma_short_dev, NULL, stream);
