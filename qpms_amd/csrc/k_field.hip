@@ -16,9 +16,10 @@
 //                coefficients (vswf.c:611-655), turned to cartesian
 //                (vectors.h:272-291) and summed over particles
 //                (scatsystem.c:2013-2037). One thread per point; when points
-//                are few, the four waves of a workgroup share 64 points and
+//                are few, the waves of a workgroup share 64 points and
 //                split the particles.
 #include <hip/hip_runtime.h>
+#include "dev_ewald.hpp"
 #include "dev_specfunc.hpp"
 #include "qpms_internal.h"
 #include "dev_launch.hpp"
@@ -142,104 +143,119 @@ __global__ void k_neg_re_cdot(long n, const v2d *__restrict__ a, long sa, const 
 }
 
 
+// Which radial functions: any kind, at the origin too (regular waves); h_l of
+// complex and of real k r, formed directly at every argument (the outgoing field's
+// case; the origin is then a singular point, NaN).
+enum { RADIAL_ANY, RADIAL_HANKEL, RADIAL_HANKEL_REAL };
+
 // One particle's field at offset (dx, dy, dz) from it, added to E (cartesian).
 // c: the particle's 2 NE coefficients (electric block, then magnetic);
 // parity: multiply electric coefficients by (-1)^(l+1), magnetic by (-1)^l.
-// HANKEL: kind is 3 or 4 and h is formed directly at every argument (the
-// outgoing field's case; the origin is then a singular point, NaN).
-template <int LMAX, bool HANKEL>
+//
+// The angular functions of m >= 1 come from Q_l^m = P_l^m / sin(theta), which has
+// the recurrence of P_l^m and is finite on the axis:
+//   leg = N sin Q_l^m, pi = N m Q_l^m, tau = N (l cos Q_l^m - (l+m) Q_{l-1}^m),
+//   m = 0: tau = N P_l^1
+// (DLMF 14.10.5), so nothing is divided by sin(theta) and the poles' limits
+// (legendre.c:65-80) come out by themselves. +-m share them: with a = c_m e^{i m
+// phi}, b = (-1)^m c_{-m} e^{-i m phi} the sums take leg (a + b), tau (a + b) and
+// pi (a - b).
+template <int LMAX, int RADIAL>
 __device__ __forceinline__ void field_of_particle(double dx, double dy, double dz, cplx k, int kind,
                                                   const v2d *__restrict__ c, bool parity, cplx *E) {
   constexpr int NE = LMAX * (LMAX + 2);
   constexpr double PI_ = 3.14159265358979323846;
   // direction cosines of cart2sph's (theta, phi) (vectors.h:134-140): theta =
-  // pi/2 at r = 0, phi = atan2(dy, dx) (also on the z axis)
-  const double r = sqrt(dx * dx + dy * dy + dz * dz);
-  const double rho = sqrt(dx * dx + dy * dy);
-  const double ct = r != 0.0 ? dz / r : cos(PI_ / 2), st = r != 0.0 ? rho / r : 1.0;
-  double cf, sf;
-  if (rho != 0.0) {
-    cf = dx / rho;
-    sf = dy / rho;
-  } else {
-    const double phi = atan2(dy, dx);
-    cf = cos(phi);
-    sf = sin(phi);
-  }
+  // pi/2 at r = 0; phi = 0 or pi on the z axis
+  const double rho2 = dx * dx + dy * dy, r = sqrt(rho2 + dz * dz), rho = sqrt(rho2);
+  const double ir = qew::rcp_(r), irho = qew::rcp_(rho);
+  const double ct = r != 0.0 ? dz * ir : cos(PI_ / 2), st = r != 0.0 ? rho * ir : 1.0;
+  const double cf = rho != 0.0 ? dx * irho : copysign(1.0, dx), sf = rho != 0.0 ? dy * irho : 0.0;
+  cplx z[LMAX + 1], krinv;
   const cplx kr = k * r;
-  cplx z[LMAX + 1];
   const bool origin = (kr.re == 0.0 && kr.im == 0.0);
-  if (HANKEL) {
-    if (origin) {   // h_l is singular at the origin (as sph_bessel_fill gives it)
+  if constexpr (RADIAL == RADIAL_HANKEL_REAL) {
+    const double sg = (kind == 3) ? 1.0 : -1.0, zi = qew::rcp_(kr.re);   // NaN at the origin
+    const cplx e = qew::expi_(sg * kr.re);
+    z[0] = mk(sg * zi * e.im, -sg * zi * e.re);                          // -+i e^{+-ix}/x
+    z[1] = -(zi * zi) * (e * mk(kr.re, sg));
 #pragma unroll
-      for (int l = 0; l <= LMAX; ++l) z[l] = mk(NAN, NAN);
-    } else {
-      qsf::sph_hankel_direct<LMAX>(kind, kr, z);
+    for (int l = 1; l < LMAX; ++l) {
+      const double f = (double)(2 * l + 1) * zi;
+      z[l + 1] = mk(fma(f, z[l].re, -z[l - 1].re), fma(f, z[l].im, -z[l - 1].im));
     }
+    krinv = mk(zi, 0.0);
   } else {
-    qsf::sph_bessel_fill<LMAX>(kind, kr, z);
+    if (RADIAL == RADIAL_HANKEL) {
+      if (origin) {   // h_l is singular at the origin (as sph_bessel_fill gives it)
+#pragma unroll
+        for (int l = 0; l <= LMAX; ++l) z[l] = mk(NAN, NAN);
+      } else {
+        qsf::sph_hankel_direct<LMAX>(kind, kr, z);
+      }
+    } else {
+      qsf::sph_bessel_fill<LMAX>(kind, kr, z);
+    }
+    krinv = origin ? mk(0.0, 0.0) : cinv(kr);
   }
-  const cplx krinv = origin ? mk(0.0, 0.0) : cinv(kr);
-  const bool pole = (fabs(ct) == 1.0);   // legendre.c:65-80
-  double P[qsf::leg_n(LMAX)];
-  qsf::legendre_cs<LMAX>(ct, st, P);
+  double P[LMAX + 1], Q[LMAX + 1][LMAX + 1];   // P_l^0; Q_l^m
+  P[0] = 1.0;
+  P[1] = ct;
+#pragma unroll
+  for (int l = 2; l <= LMAX; ++l) P[l] = ((2 * l - 1) / (double)l) * (ct * P[l - 1]) - ((l - 1) / (double)l) * P[l - 2];
+  cplx em[LMAX + 1];   // e^{i m phi}
+  em[0] = mk(1.0, 0.0);
+#pragma unroll
+  for (int m = 1; m <= LMAX; ++m) {
+    em[m] = m == 1 ? mk(cf, sf) : em[m - 1] * mk(cf, sf);
+    Q[m][m] = m == 1 ? -1.0 : (-(2 * m - 1) * st) * Q[m - 1][m - 1];
+    Q[m - 1][m] = 0.0;
+#pragma unroll
+    for (int l = m + 1; l <= LMAX; ++l)
+      Q[l][m] = ((2 * l - 1) / (double)(l - m)) * (ct * Q[l - 1][m]) - ((l + m - 1) / (double)(l - m)) * Q[l - 2 < m ? m - 1 : l - 2][m];
+  }
   cplx Er = mk(0.0, 0.0), Et = mk(0.0, 0.0), Ef = mk(0.0, 0.0);
 #pragma unroll
   for (int l = 1; l <= LMAX; ++l) {
     // z_l / kr (1/3 for the regular l = 1 wave at the origin) and z_{l-1} - l z_l / kr
-    const cplx besfac = origin ? mk(l == 1 ? 1.0 / 3.0 : 0.0, 0.0) : z[l] * krinv;
-    const cplx besder = z[l - 1] - (double)l * besfac;
-    const double pe = (parity && !(l & 1)) ? -1.0 : 1.0;   // electric: (-1)^(l+1)
-    const double pm = (parity && (l & 1)) ? -1.0 : 1.0;    // magnetic: (-1)^l
+    cplx besfac, zl = z[l];
+    if constexpr (RADIAL == RADIAL_HANKEL_REAL) besfac = krinv.re * z[l];
+    else besfac = origin ? mk(l == 1 ? 1.0 / 3.0 : 0.0, 0.0) : z[l] * krinv;
+    cplx besder = z[l - 1] - (double)l * besfac;
+    if (parity) {   // uniform; electric: (-1)^(l+1), magnetic: (-1)^l
+      if (l & 1) zl = -zl;
+      else besfac = -besfac, besder = -besder;
+    }
     // angular sums of degree l; the radial factors multiply them once per l:
     // N = (l(l+1) leg z/kr e, tau besder e, pi besder i e), M = (0, pi z i e, -tau z e)
-    cplx sLegN = mk(0.0, 0.0), sTauN = mk(0.0, 0.0), sPiN = mk(0.0, 0.0), sPiM = mk(0.0, 0.0),
-         sTauM = mk(0.0, 0.0);
-    cplx em = mk(1.0, 0.0);   // e^{i m phi}
+    const int y0 = l * (l + 1) - 1;
+    const double n0 = sqrt((2 * l + 1) / (4 * PI_)) / sqrt((double)(l * (l + 1)));
+    const cplx c0 = mk(c[y0].x, c[y0].y), d0 = mk(c[NE + y0].x, c[NE + y0].y);
+    const double leg0 = n0 * P[l], tau0 = n0 * (st * Q[l][1]);
+    cplx sLegN = leg0 * c0, sTauN = tau0 * c0, sPiN = mk(0.0, 0.0), sPiM = mk(0.0, 0.0), sTauM = tau0 * d0;
 #pragma unroll
-    for (int m = 0; m <= l; ++m) {
-      if (m > 0) em = em * mk(cf, sf);
-      // normalised leg, pi, tau for +m (legendre.c:54-110, default normalisation)
-      double leg, pi, tau;
-      if (pole) {
-        const double fl = 0.25 * sqrt((2 * l + 1) / PI_);
-        const double lpar = (l & 1) ? -1.0 : 1.0;
-        leg = (m == 0) ? ((l & 1) ? ct : 1.0) * sqrt((2 * l + 1) / (4 * PI_ * l * (l + 1))) : 0.0;
-        pi = (m == 1) ? ((ct > 0) ? -1.0 : lpar) * fl : 0.0;     // -(...) * fl * csphase, csphase = -1
-        tau = (m == 1) ? -((ct > 0) ? 1.0 : lpar) * fl : 0.0;
-      } else {
-        double fr = 1.0;
+    for (int m = 1; m <= l; ++m) {
+      double fr = 1.0;
 #pragma unroll
-        for (int t = l - m + 1; t <= l + m; ++t) fr *= t;
-        const double nlm = sqrt((2 * l + 1) / (4 * PI_ * fr)) / sqrt((double)(l * (l + 1)));
-        const double Plm = P[qsf::leg_idx(l, m)];
-        const double Pl1 = (l - 1 >= m) ? P[qsf::leg_idx(l - 1, m)] : 0.0;
-        const double dP = ((l + m) * Pl1 - l * ct * Plm) / ((1.0 - ct) * (1.0 + ct));   // DLMF 14.10.5
-        leg = nlm * Plm;
-        pi = m / st * leg;
-        tau = -st * nlm * dP;
-      }
-#pragma unroll
-      for (int sgn = 0; sgn < (m == 0 ? 1 : 2); ++sgn) {
-        // -m: leg and tau carry (-1)^m, pi (-1)^(m+1); e^{-i m phi} = conj
-        const int mm = sgn ? -m : m;
-        const double fm = (sgn && (m & 1)) ? -1.0 : 1.0;
-        const double lg = fm * leg, ta = fm * tau, p_ = sgn ? -fm * pi : pi;
-        const cplx e = sgn ? conj(em) : em;
-        const int y = l * (l + 1) + mm - 1;
-        const v2d cn = c[y], cm = c[NE + y];
-        const cplx u = mk(pe * cn.x, pe * cn.y) * e, v = mk(pm * cm.x, pm * cm.y) * e;
-        sLegN = sLegN + lg * u;
-        sTauN = sTauN + ta * u;
-        sPiN = sPiN + p_ * u;
-        sPiM = sPiM + p_ * v;
-        sTauM = sTauM + ta * v;
-      }
+      for (int t = l - m + 1; t <= l + m; ++t) fr *= t;
+      const double nlm = sqrt((2 * l + 1) / (4 * PI_ * fr)) / sqrt((double)(l * (l + 1)));
+      const double q = nlm * Q[l][m], leg = st * q, pi = m * q;
+      const double tau = m == l ? (l * ct) * q : fma(l * ct, q, (-(l + m) * nlm) * Q[l - 1][m]);
+      const v2d cp = c[y0 + m], cn = c[y0 - m], dp = c[NE + y0 + m], dn = c[NE + y0 - m];
+      const cplx e = em[m], a = mk(cp.x, cp.y) * e, b = mk(cn.x, cn.y) * conj(e), f = mk(dp.x, dp.y) * e,
+                 g = mk(dn.x, dn.y) * conj(e);
+      const cplx ps = (m & 1) ? a - b : a + b, pd = (m & 1) ? a + b : a - b;
+      const cplx qs = (m & 1) ? f - g : f + g, qd = (m & 1) ? f + g : f - g;
+      sLegN = sLegN + leg * ps;
+      sTauN = sTauN + tau * ps;
+      sPiN = sPiN + pi * pd;
+      sPiM = sPiM + pi * qd;
+      sTauM = sTauM + tau * qs;
     }
-    const cplx zs = z[l] * sPiM, bs = besder * sPiN;
+    const cplx zs = zl * sPiM, bs = besder * sPiN;
     Er = Er + (double)(l * (l + 1)) * (besfac * sLegN);
     Et = Et + besder * sTauN + mk(-zs.im, zs.re);
-    Ef = Ef + mk(-bs.im, bs.re) - z[l] * sTauM;
+    Ef = Ef + mk(-bs.im, bs.re) - zl * sTauM;
   }
   E[0] = E[0] + (st * cf) * Er + (ct * cf) * Et - sf * Ef;
   E[1] = E[1] + (st * sf) * Er + (ct * sf) * Et + cf * Ef;
@@ -252,15 +268,18 @@ __device__ __forceinline__ void field_of_particle(double dx, double dy, double d
 // for the whole wave (scalar loads, read once per wave instead of once per
 // lane) and points too few to fill the device still give S times as many
 // waves. The S partial fields of a point are added in LDS in slice order
-// (deterministic). Up to lMax 3 the kernel is held to two waves per SIMD
-// (256 registers, a few values spilled), which measured 15 % faster than one.
-template <int LMAX, int S, bool HANKEL>
-__global__ __launch_bounds__(256, LMAX <= 3 ? 2 : 1) void k_scattered_e(int npts, const double *__restrict__ where, int npart,
+// (deterministic).
+//
+// What bounds it: FP64 vector instructions, 565 per wave and particle for lMax 3
+// and real k (84 % of their issue rate at 65,536 points and 1024 particles: 1.12
+// ms). With P_l^m divided by sin(theta) per (l, m), the poles apart, each sign of m
+// by itself and the library's sin, cos and exp it took 1300 and 2.80 ms.
+template <int LMAX, int S, int RADIAL>
+__global__ __launch_bounds__((S > 4 ? 64 * S : 256), (LMAX <= 3 ? 2 : 1)) void k_scattered_e(int npts, const double *__restrict__ where, int npart,
                                                      const double *__restrict__ pos, double k_re, double k_im,
                                                      int kind, const v2d *__restrict__ cvf, int parity,
                                                      v2d *__restrict__ out) {
-  static_assert(S == 1 || S == 2 || S == 4, "slices of a 4-wave workgroup");
-  constexpr int NB = 2 * LMAX * (LMAX + 2), G = 4 / S;   // point groups per workgroup
+  constexpr int NB = 2 * LMAX * (LMAX + 2), W = S > 4 ? S : 4, G = W / S;   // waves, point groups per workgroup
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int slice = __builtin_amdgcn_readfirstlane(wave % S), grp = wave / S;
   const int t = (blockIdx.x * G + grp) * 64 + lane;
@@ -270,11 +289,11 @@ __global__ __launch_bounds__(256, LMAX <= 3 ? 2 : 1) void k_scattered_e(int npts
   if (live) {
     const double wx = where[3 * t], wy = where[3 * t + 1], wz = where[3 * t + 2];
     for (int p = slice; p < npart; p += S)
-      field_of_particle<LMAX, HANKEL>(wx - pos[3 * p], wy - pos[3 * p + 1], wz - pos[3 * p + 2], k, kind,
+      field_of_particle<LMAX, RADIAL>(wx - pos[3 * p], wy - pos[3 * p + 1], wz - pos[3 * p + 2], k, kind,
                                       cvf + (size_t)p * NB, parity != 0, E);
   }
   if (S > 1) {
-    __shared__ double red[4][6][64];
+    __shared__ double red[W][6][64];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
       red[wave][2 * q][lane] = E[q].re;
@@ -350,24 +369,29 @@ extern "C" int qh_launch_scattered_e(int lMax, size_t npts, const double *where_
     qpms_hip_die(__FILE__, __LINE__, __func__, "too many points (%zu) or particles (%zu)", npts, npart);
   hipStream_t s = (hipStream_t)qh_stream(stream);
   // points too few to fill the device one thread each (fewer than 262,144,
-  // 4096 waves): the particles split over 4 waves per 64 points
-  const int S = (npart >= 4 && npts < 262144) ? 4 : 1;
-  const bool hankel = kind >= 3;
-  const dim3 grid((unsigned)((npts + 64 * (4 / S) - 1) / (64 * (4 / S)))), block(256);
+  // 4096 waves): the particles split over 4 waves per 64 points; over 8 where even
+  // their workgroups are fewer than the CUs (16,384: 1000 particles of lMax 3 at
+  // 10,000 points 325 us against 395 with 4; at 65,536, where 8 waves of a workgroup
+  // leave a third of the registers unused, 4 win: 1.12 against 1.20 ms)
+  const int S = (npart < 4 || npts >= 262144) ? 1 : npts < 16384 ? 8 : 4, W = S > 4 ? S : 4;
+  const int radial = kind < 3 ? RADIAL_ANY : k_im == 0.0 ? RADIAL_HANKEL_REAL : RADIAL_HANKEL;
+  const dim3 grid((unsigned)((npts + 64 * (W / S) - 1) / (64 * (W / S)))), block(64 * W);
   const v2d *c = (const v2d *)cvf_dev;
   v2d *o = (v2d *)out_dev;
 #define QH_SCE1(LM, SL, H) \
   QH_LAUNCH((k_scattered_e<LM, SL, H>), grid, block, 0, s, (int)npts, where_dev, (int)npart, pos_dev, k_re, \
                      k_im, kind, c, parity, o)
-#define QH_SCE(LM)                                   \
-  do {                                               \
-    if (S == 4) {                                    \
-      if (hankel) QH_SCE1(LM, 4, true);              \
-      else QH_SCE1(LM, 4, false);                    \
-    } else {                                         \
-      if (hankel) QH_SCE1(LM, 1, true);              \
-      else QH_SCE1(LM, 1, false);                    \
-    }                                                \
+#define QH_SCE2(LM, SL)                                                    \
+  do {                                                                     \
+    if (radial == RADIAL_HANKEL_REAL) QH_SCE1(LM, SL, RADIAL_HANKEL_REAL); \
+    else if (radial == RADIAL_HANKEL) QH_SCE1(LM, SL, RADIAL_HANKEL);      \
+    else QH_SCE1(LM, SL, RADIAL_ANY);                                      \
+  } while (0)
+#define QH_SCE(LM)               \
+  do {                           \
+    if (S == 8) QH_SCE2(LM, 8);  \
+    else if (S == 4) QH_SCE2(LM, 4); \
+    else QH_SCE2(LM, 1);         \
   } while (0)
   switch (lMax) {
     case 1: QH_SCE(1); break;
@@ -377,6 +401,7 @@ extern "C" int qh_launch_scattered_e(int lMax, size_t npts, const double *where_
     default: qpms_hip_die(__FILE__, __LINE__, __func__, "lMax %d not instantiated (1..4)", lMax);
   }
 #undef QH_SCE
+#undef QH_SCE2
 #undef QH_SCE1
   HIPCHK(hipGetLastError());
   return 0;
