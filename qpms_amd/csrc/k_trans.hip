@@ -3,7 +3,7 @@
 //  k_ab_batch<LMAX>   one lane per displacement point: the nelem x nelem A and
 //                     B arrays (translations.c:610-698).
 //  k_w_build<LMAX,M>  one wave64 per (destination particle R, 64 consecutive
-//                     source particles): the rows of particle R of the
+//                     source particles, group of y): the rows of particle R of the
 //                     translation matrix W (scatsystem.c:1180-1217) or of the
 //                     mode-problem matrix M = I - T W for diagonal T
 //                     (scatsystem.c:1283-1343).
@@ -19,6 +19,14 @@
 // writes the two matrix rows (E row: [A | B] per block, M row: [B | A]) as
 // contiguous 1 KiB non-temporal stores. Every element of W is written exactly
 // once: no memset pass.
+//
+// What bounds it: fetching its instructions (10 KB for one y of lMax 4, each run
+// once per wave) while particles are few, the stores when they are many (467
+// particles of lMax 3: 4.3 TB/s). A wave therefore takes a few y, and the groups of
+// y are outermost in the grid, so the waves of a CU run the same code at a time.
+// (y as a loop, its stores in it, made the compiler keep the products of all y in
+// scratch: 650 instead of 380 us for 200 particles of lMax 4. Stores aligned to 128
+// bytes, or plain ones, changed nothing.)
 #include <hip/hip_runtime.h>
 #include <utility>
 #include "dev_specfunc.hpp"
@@ -204,8 +212,10 @@ template <int LMAX, bool MODE_M, int... Ys>
 __device__ __forceinline__ void w_rows(const PairData<LMAX> &pd, const v2d *__restrict__ mA,
                                        const v2d *__restrict__ mB, v2d *lds, int lane, int R, int Rloc,
                                        int C0, int nvalid, const v2d *__restrict__ tdiagR,
-                                       v2d *__restrict__ W, size_t ld, std::integer_sequence<int, Ys...>) {
-  (w_row<LMAX, MODE_M, Ys>(pd, mA, mB, lds, lane, R, Rloc, C0, nvalid, tdiagR, W, ld), ...);
+                                       v2d *__restrict__ W, size_t ld, int y0, int y1,
+                                       std::integer_sequence<int, Ys...>) {
+  ((Ys >= y0 && Ys < y1 ? w_row<LMAX, MODE_M, Ys>(pd, mA, mB, lds, lane, R, Rloc, C0, nvalid, tdiagR, W, ld) : void()),
+   ...);
 }
 
 // With `node` set (Beyn quadrature chunks replayed as one graph), the
@@ -219,12 +229,13 @@ __global__ __launch_bounds__(64) void k_w_build(const double *__restrict__ pos, 
                                                 const int *__restrict__ ttype,
                                                 const v2d *__restrict__ tdiag, v2d *__restrict__ W,
                                                 size_t ld, const double *__restrict__ ntab,
-                                                const int *__restrict__ cursor, int slot) {
+                                                const int *__restrict__ cursor, int slot, int nblk, int rows) {
   constexpr int NE = Dims<LMAX>::NE, NB = Dims<LMAX>::NB;
   __shared__ v2d lds[64 * (NB + 1)];
   const int lane = threadIdx.x;
-  const int R = row_p0 + blockIdx.x / nchunks;
-  const int C0 = (blockIdx.x % nchunks) * 64;
+  const int blk = blockIdx.x % nblk, y0 = blockIdx.x / nblk * rows;   // groups of y outermost
+  const int R = row_p0 + blk / nchunks;
+  const int C0 = (blk % nchunks) * 64;
   const int C = C0 + lane;
   const int nsrc = min(64, npart - C0);
   const int nvalid = nsrc * NB;
@@ -244,7 +255,7 @@ __global__ __launch_bounds__(64) void k_w_build(const double *__restrict__ pos, 
   PairData<LMAX> pd;
   pair_setup_cart<LMAX>(dx, dy, dz, mk(k_re, k_im), kind, pd);
   const v2d *tdiagR = MODE_M ? tdiag + (size_t)ttype[R] * NB : nullptr;
-  w_rows<LMAX, MODE_M>(pd, mA, mB, lds, lane, R, R - row_p0, C0, nvalid, tdiagR, W, ld,
+  w_rows<LMAX, MODE_M>(pd, mA, mB, lds, lane, R, R - row_p0, C0, nvalid, tdiagR, W, ld, y0, y0 + rows,
                        std::make_integer_sequence<int, NE>{});
 }
 
@@ -312,13 +323,21 @@ static void launch_w(const qh_trans_tables *t, size_t npart, const double *pos_d
   const size_t nblk = row_np * (size_t)nchunks;
   if (nblk == 0) return;
   if (nblk > 0x7fffffffu) qpms_hip_die(__FILE__, __LINE__, __func__, "grid too large");
-  const dim3 grid((unsigned)nblk), block(64);
+  // Indices y per workgroup: one while that makes no more workgroups than the chip
+  // has SIMDs (lMax 4, 16 particles: 20 us, all 24 in one workgroup 190), up to four
+  // (120 particles 126 against 295, 233 particles 453 against 619; two or one 5-15 %
+  // slower there, for the pairs' functions evaluated again).
+  int rows = 1;
+  while (rows < 4 && nblk * ((t->nelem + rows - 1) / rows) > 1024) ++rows;
+  size_t groups = (t->nelem + rows - 1) / rows;
+  if (nblk * groups > 0x7fffffffu) { rows = t->nelem; groups = 1; }
+  const dim3 grid((unsigned)(nblk * groups)), block(64);
   const v2d *mA = (const v2d *)t->dA, *mB = (const v2d *)t->dB;
   const v2d *td = (const v2d *)tdiag;
   v2d *W = (v2d *)W_dev;
   switch (t->lMax) {
 #define QH_W_CASE(LM) case LM: QH_LAUNCH((k_w_build<LM, MODE_M>), grid, block, 0, s, pos_dev, (int)npart, \
-      (int)row_p0, nchunks, k_re, k_im, kind, mA, mB, ttype, td, W, ld, ntab, cursor, slot); break;
+      (int)row_p0, nchunks, k_re, k_im, kind, mA, mB, ttype, td, W, ld, ntab, cursor, slot, (int)nblk, rows); break;
     QH_W_CASE(1) QH_W_CASE(2) QH_W_CASE(3) QH_W_CASE(4)
 #undef QH_W_CASE
     default: qpms_hip_die(__FILE__, __LINE__, __func__, "lMax %d not instantiated (1..4)", t->lMax);
