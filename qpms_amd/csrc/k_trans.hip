@@ -1,7 +1,7 @@
 // VSWF translation coefficients on gfx950.
 //
-//  k_ab_batch<LMAX>   one lane per displacement point: the nelem x nelem A and
-//                     B arrays (translations.c:610-698).
+//  k_ab_batch<LMAX>   one lane per displacement point, waves per group of y: the
+//                     nelem x nelem A and B arrays (translations.c:610-698).
 //  k_w_build<LMAX,M>  one wave64 per (destination particle R, 64 consecutive
 //                     source particles, group of y): the rows of particle R of the
 //                     translation matrix W (scatsystem.c:1180-1217) or of the
@@ -140,9 +140,9 @@ __device__ __forceinline__ void ab_batch_row(const PairData<LMAX> &pd, const v2d
 
 template <int LMAX, int... Ys>
 __device__ __forceinline__ void ab_batch_all(const PairData<LMAX> &pd, const v2d *__restrict__ mA,
-                                             const v2d *__restrict__ mB, v2d *Aout, v2d *Bout,
+                                             const v2d *__restrict__ mB, v2d *Aout, v2d *Bout, int y0, int y1,
                                              std::integer_sequence<int, Ys...>) {
-  (ab_batch_row<LMAX, Ys>(pd, mA, mB, Aout, Bout), ...);
+  ((Ys >= y0 && Ys < y1 ? ab_batch_row<LMAX, Ys>(pd, mA, mB, Aout, Bout) : void()), ...);
 }
 
 template <int LMAX>
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(64) void k_ab_batch(int npts, const v2d *__restrict
                                                  const double *__restrict__ th, const double *__restrict__ ph,
                                                  int kind, const v2d *__restrict__ mA,
                                                  const v2d *__restrict__ mB, v2d *__restrict__ A,
-                                                 v2d *__restrict__ B) {
+                                                 v2d *__restrict__ B, int rows) {
   constexpr int NE = Dims<LMAX>::NE;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= npts) return;
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(64) void k_ab_batch(int npts, const v2d *__restrict
   const v2d k = kr[i];
   pair_setup<LMAX>(mk(k.x, k.y), th[i], ph[i], kind, pd);
   ab_batch_all<LMAX>(pd, mA, mB, A + (size_t)i * NE * NE, B + (size_t)i * NE * NE,
-                     std::make_integer_sequence<int, NE>{});
+                     blockIdx.y * rows, (blockIdx.y + 1) * rows, std::make_integer_sequence<int, NE>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -294,20 +294,33 @@ __global__ void k_mie(int lMax, int nsph, const double *__restrict__ prm, v2d *_
 #define HIPCHK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) \
   qpms_hip_die(__FILE__, __LINE__, __func__, "HIP error %d (%s) in %s", (int)e_, hipGetErrorString(e_), #x); } while (0)
 
+// Indices y per wave: one while that makes no more waves than the chip has SIMDs
+// (W of lMax 4, 16 particles: 20 us, all 24 in one wave 190; one pair of lMax 2: 32
+// us a call, 38 with all 8 in one), up to four (120 particles 126 against 295, 233
+// particles 453 against 619; two or one 5-15 % slower there, for the pairs'
+// functions evaluated again).
+static int rows_per_wave(size_t nblk, int nelem) {
+  int rows = 1;
+  while (rows < 4 && nblk * ((nelem + rows - 1) / rows) > 1024) ++rows;
+  return rows;
+}
+
 extern "C" int qh_launch_ab_batch(const qh_trans_tables *t, size_t npts, const double *kr_dev,
                                   const double *theta_dev, const double *phi_dev, int kind,
                                   double *A_dev, double *B_dev, void *stream) {
   if (npts == 0) return 0;
   hipStream_t s = (hipStream_t)qh_stream(stream);
-  const dim3 grid((unsigned)((npts + 63) / 64)), block(64);
+  const size_t nblk = (npts + 63) / 64;
+  const int rows = rows_per_wave(nblk, t->nelem);
+  const dim3 grid((unsigned)nblk, (unsigned)((t->nelem + rows - 1) / rows)), block(64);
   const v2d *mA = (const v2d *)t->dA, *mB = (const v2d *)t->dB;
   const v2d *kr = (const v2d *)kr_dev;
   v2d *A = (v2d *)A_dev, *B = (v2d *)B_dev;
   switch (t->lMax) {
-    case 1: QH_LAUNCH(k_ab_batch<1>, grid, block, 0, s, (int)npts, kr, theta_dev, phi_dev, kind, mA, mB, A, B); break;
-    case 2: QH_LAUNCH(k_ab_batch<2>, grid, block, 0, s, (int)npts, kr, theta_dev, phi_dev, kind, mA, mB, A, B); break;
-    case 3: QH_LAUNCH(k_ab_batch<3>, grid, block, 0, s, (int)npts, kr, theta_dev, phi_dev, kind, mA, mB, A, B); break;
-    case 4: QH_LAUNCH(k_ab_batch<4>, grid, block, 0, s, (int)npts, kr, theta_dev, phi_dev, kind, mA, mB, A, B); break;
+    case 1: QH_LAUNCH(k_ab_batch<1>, grid, block, 0, s, (int)npts, kr, theta_dev, phi_dev, kind, mA, mB, A, B, rows); break;
+    case 2: QH_LAUNCH(k_ab_batch<2>, grid, block, 0, s, (int)npts, kr, theta_dev, phi_dev, kind, mA, mB, A, B, rows); break;
+    case 3: QH_LAUNCH(k_ab_batch<3>, grid, block, 0, s, (int)npts, kr, theta_dev, phi_dev, kind, mA, mB, A, B, rows); break;
+    case 4: QH_LAUNCH(k_ab_batch<4>, grid, block, 0, s, (int)npts, kr, theta_dev, phi_dev, kind, mA, mB, A, B, rows); break;
     default: qpms_hip_die(__FILE__, __LINE__, __func__, "lMax %d not instantiated (1..4)", t->lMax);
   }
   HIPCHK(hipGetLastError());
@@ -323,14 +336,9 @@ static void launch_w(const qh_trans_tables *t, size_t npart, const double *pos_d
   const size_t nblk = row_np * (size_t)nchunks;
   if (nblk == 0) return;
   if (nblk > 0x7fffffffu) qpms_hip_die(__FILE__, __LINE__, __func__, "grid too large");
-  // Indices y per workgroup: one while that makes no more workgroups than the chip
-  // has SIMDs (lMax 4, 16 particles: 20 us, all 24 in one workgroup 190), up to four
-  // (120 particles 126 against 295, 233 particles 453 against 619; two or one 5-15 %
-  // slower there, for the pairs' functions evaluated again).
-  int rows = 1;
-  while (rows < 4 && nblk * ((t->nelem + rows - 1) / rows) > 1024) ++rows;
+  int rows = rows_per_wave(nblk, t->nelem);
   size_t groups = (t->nelem + rows - 1) / rows;
-  if (nblk * groups > 0x7fffffffu) { rows = t->nelem; groups = 1; }
+  if (nblk * groups >= (1u << 26)) { rows = t->nelem; groups = 1; }   // work-items of a dispatch
   const dim3 grid((unsigned)(nblk * groups)), block(64);
   const v2d *mA = (const v2d *)t->dA, *mB = (const v2d *)t->dB;
   const v2d *td = (const v2d *)tdiag;

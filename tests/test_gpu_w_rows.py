@@ -27,3 +27,16 @@ def test_rows_of_whole_matrix(gpu, lMax, npart):
                                                     npart * nb, None)
         L.qpms_hip_sync()
         assert np.array_equal(dW.to_array(np.complex128, (nb, npart * nb)), W[p])
+
+
+@pytest.mark.parametrize("lMax, npts", [(1, 1), (2, 1), (4, 1), (3, 65), (2, 8192), (2, 8200), (4, 3000)])
+def test_batches_of_pairs(gpu, lMax, npts):
+    """A batch's arrays against those of its points in batches of one."""
+    import qpms_amd
+    calc = qpms_amd.TransCalculator(lMax)
+    g = np.random.default_rng(npts)
+    kr, th, ph = g.uniform(1, 30, npts) + 0j, g.uniform(0, np.pi, npts), g.uniform(-3, 3, npts)
+    A, B = calc.get_AB_arrays_batch(kr, th, ph)
+    for i in sorted({0, npts // 2, npts - 1}):
+        a, b = calc.get_AB_arrays_batch(kr[i:i + 1], th[i:i + 1], ph[i:i + 1])
+        assert np.array_equal(a[0], A[i]) and np.array_equal(b[0], B[i])
