@@ -7,20 +7,24 @@
 // beyn.c:556-561 (zgetrf + zgetrs with l right-hand sides).
 //
 // LU structure (getrf_batched): outer blocks of LU_NB = 256 columns.
-//   k_ts_*        factor a tall strip of PW = 32 columns with tournament
-//                 pivoting: candidate rows chosen per chunk of 256 rows
-//                 staged in LDS, merged a chunk's worth of candidate sets at
-//                 a time, the winners moved to the top (recorded as
-//                 zgetrf-style interchanges) in every column by one gather;
-//                 the last level also inverts the strip's L11 and U11;
-//                 no workgroup waits for another;
-//   k_gemm_sub    C -= A B, or C = A B: L21 = A21 U11^{-1} and
-//                 U12 = L11^{-1} A12 (products with the inverses), the
-//                 rank-PW updates inside an outer block and the rank-256
-//                 trailing update A22 -= L21 U12 (the O(n^3) part, rocBLAS or
-//                 k_cgemm3m by size class). FP64 uses v_mfma_f64_16x16x4f64, FP32
-//                 v_mfma_f32_16x16x4f32; the complex product is four real
-//                 MFMA chains on de-interleaved LDS tiles.
+//   k_strip       factors a tall strip of PW = 32 columns with partial pivoting
+//                 in one launch, the rows in registers; its workgroups agree on
+//                 each pivot through memory. They wait for one another, so they
+//                 announce themselves first, and where they do not all get onto
+//                 the device in time one of them does the strip alone;
+//   k_ts_*        the same with tournament pivoting, no workgroup waiting for
+//                 another: only for blocks beside the trailing update whose
+//                 strips have more workgroups than there are CUs left for them;
+//   k_swap_u      the strip's interchanges and U = L11^{-1} A12 in the rest of
+//                 its outer block, by substitution; k_u12 the block's U12 in the
+//                 columns beyond;
+//   k_gemm_sub    C -= A B (k_gemm_cu beside the trailing update): the rank-PW
+//                 updates inside an outer block and the rank-256 trailing update
+//                 A22 -= L21 U12 (the O(n^3) part, rocBLAS or k_cgemm3m by size
+//                 class). FP64 uses v_mfma_f64_16x16x4f64, FP32
+//                 v_mfma_f32_16x16x4f32; the complex product is four real MFMA
+//                 chains on de-interleaved LDS tiles.
+// Solves (getrs_batched): k_tri, both sweeps in one launch.
 // Every kernel takes a batch index in blockIdx.z with per-matrix strides, so
 // the Beyn quadrature nodes factor in one launch sequence.
 #include <hip/hip_runtime.h>
@@ -1925,12 +1929,11 @@ static size_t getrf_ws_bytes(int n, int batch) {
   return (size_t)batch * LuWS<T>(n, batch, false).bytes;
 }
 
-// Blocked right-looking LU with tournament-pivoted panels of `batch` n x n
-// matrices (stride sA), in place. Outer blocks of LU_NB columns; inside a
-// block the columns are factorised PW at a time (k_ts_*), the block's
-// remaining columns updated by products with the strip's L11^{-1} and a GEMM
-// (K = PW); then U12 = L11^{-1} A12 by PW rows the same way, and the trailing
-// A22 -= L21 U12 (K = LU_NB).
+// Blocked right-looking LU of `batch` n x n matrices (stride sA), in place. Outer
+// blocks of LU_NB columns; inside a block the columns are factorised PW at a time
+// (k_strip), the block's remaining columns updated by substitution (k_swap_u) and a
+// GEMM (K = PW); then U12 = L11^{-1} A12 in one launch (k_u12), and the trailing A22
+// -= L21 U12 (K = LU_NB).
 // ipiv (1-based, stride sP) lists the row interchanges as zgetrf's does;
 // perm (optional) tracks P; info[z] gets the first zero pivot. ws:
 // getrf_ws_bytes<T>(n, batch) bytes, or nullptr for a library-owned buffer
@@ -2418,14 +2421,16 @@ static void getrs_batched(int n, int nrhs, int batch, const typename C2<T>::t *L
   const int nblk = (n + TR_B - 1) / TR_B, nslab = (nrhs + TR_C - 1) / TR_C;
   const long slabb = (long)((tr_slab_bytes<T>(n, nrhs) + 255) / 256 * 256), sW = slabb * nslab;
   qh_zero(ws, (size_t)batch * sW, s);
-  // A workgroup's next block, up to nblk products of 64 x 64 blocks (2 us each),
-  // has to be ready when the chain (4 to 7 us a block) gets there: nblk / 4 of
-  // them keep up. A quarter of those the device holds (256 in FP64, 512 in FP32)
-  // leaves room for the solves of other streams, whose workgroups wait for one
-  // another too, hence no more than that for small systems, in batches either.
-  const long quarter = sizeof(T) == 8 ? 64 : 128;
-  const long room = std::min((long)TR_MEET, std::max(quarter, (long)nslab * nblk / 4));
-  const int G = (int)std::max(1L, std::min((long)nblk, room / ((long)nslab * batch)));
+  // One slab: a workgroup's next block, up to nblk products of 64 x 64 blocks (2 us
+  // each), has to be ready when the chain (4 to 7 us a block) gets there: nblk / 4
+  // of them keep up. Several slabs or matrices share what the device holds (256 in
+  // FP64, 512 in FP32), more of them take turns: a 16-matrix batch of order 9216
+  // with 64 right-hand sides (FP32) takes 23 ms with two workgroups per slab, 12 with
+  // eight. A slab gets no more than a quarter of the device, so that of the slabs
+  // of four streams one is always complete and the others wait for its end only.
+  const long quarter = sizeof(T) == 8 ? 64 : 128, slabs = (long)nslab * batch;
+  const int G = (int)std::max(1L, std::min({(long)nblk, (long)TR_MEET, slabs == 1 ? std::max(quarter, (long)nblk / 4)
+                                                                                  : std::min(quarter, 4 * quarter / slabs)}));
   QH_LAUNCH(k_tri<T>, dim3(G, nslab, batch), dim3(256), tr_lds<T>(), s, n, nrhs, LU, lda, sA, perm, sP, B, ldb, sB,
             (char *)ws, sW, slabb, wait);
   HIPCHK(hipGetLastError());
