@@ -25,8 +25,8 @@ one (extinction, log-determinant, Beyn singular values and eigenvalues).
 
 `roofline`: the FP32 LU of a mode-problem matrix of order 44880 -- the order
 of the largest request of the default timed segment, a 32-node contour whose
-node factorisations are most of the segment's GPU time: tournament-pivoted
-panels plus trailing complex GEMMs on MFMA -- timed live with HIP events on
+node factorisations are most of the segment's GPU time: pivoted panels
+plus trailing complex GEMMs on MFMA -- timed live with HIP events on
 the library stream and priced at 8/3 n^3 real flops against the FP32 matrix
 peak; `traffic` comes from the committed rocprofv3 counter summary of the
 same probe. `roofline_lu16380` is the same at order 16380. `w_build`: the plain
@@ -276,7 +276,7 @@ def measure_lu(L, ev, stream, n_part=1496, reps=3, calib=False):
             # HBM bytes per factorisation from the two rocprofv3 --pmc passes of
             # this probe (FETCH_SIZE, WRITE_SIZE, copy-kernel calibration)
             "traffic": profile_traffic(f"lu_fp32_order{n}"),
-            "kernel": f"FP32 LU, order {n} (tournament panels + trailing GEMM)",
+            "kernel": f"FP32 LU, order {n} (panels + trailing GEMM)",
             "avg_launch_ms": avg, "algorithmic_flops_per_launch": flops}
 
 
