@@ -263,12 +263,21 @@ __device__ __forceinline__ void short_triple(const double *__restrict__ T /* bx 
   }
 }
 
-template <int LE, bool XY, bool ERR>
-__global__ __launch_bounds__((64 * ew_waves<LE, (XY && !ERR)>())) void k_sigma_short(
+// Launch bounds of the kernels by kind of k (one wave per triple): the real ones need
+// half the registers without the others' arithmetic beside them, so two waves fit a
+// SIMD up to LE 7 (2048 points x 3 shifts, LE 7: 307 us against 498 with one kernel
+// for both kinds and one wave per SIMD; few triples are better off with one launch).
+#define EW_BOUNDS(LE, KIND, SMALL) \
+  __launch_bounds__((KIND ? 64 : 64 * ew_waves<LE, SMALL>()), (KIND && LE <= (KIND == 1 ? 7 : 5) ? 2 : 1))
+
+template <int LE, bool XY, bool ERR, int KIND>
+__global__ EW_BOUNDS(LE, KIND, (XY && !ERR)) void k_sigma_short(
     const double *__restrict__ tr, int npts, const double *__restrict__ pts, double eta,
     const double *__restrict__ leg0, int csphase, v2d *__restrict__ out, double *__restrict__ err) {
   constexpr size_t NSC = (LE + 1) * (LE + 1);
-  short_triple<LE, XY, ERR>(tr + 8 * (size_t)blockIdx.x, npts, pts, eta, leg0, csphase, out + blockIdx.x * NSC,
+  const double *T = tr + 8 * (size_t)blockIdx.x;
+  if (KIND && (T[4] == 0.0) != (KIND == 1)) return;
+  short_triple<LE, XY, ERR, KIND>(T, npts, pts, eta, leg0, csphase, out + blockIdx.x * NSC,
                             ERR ? err + blockIdx.x * NSC : nullptr);
 }
 
@@ -503,23 +512,21 @@ __device__ __forceinline__ void long_triple(const double *__restrict__ T, int np
   }
 }
 
-template <int LE, bool ERR>
-__global__ __launch_bounds__((64 * ew_waves<LE, !ERR>())) void k_sigma_long(
+template <int LE, bool ERR, int KIND>
+__global__ EW_BOUNDS(LE, KIND, !ERR) void k_sigma_long(
     const double *__restrict__ tr, int npts, const double *__restrict__ Kp, double eta, double area,
     const double *__restrict__ leg0, v2d *__restrict__ out, double *__restrict__ err) {
   constexpr size_t NSC = (LE + 1) * (LE + 1);
-  long_triple<LE, ERR>(tr + 8 * (size_t)blockIdx.x, npts, Kp, eta, area, leg0, out + blockIdx.x * NSC,
+  const double *T = tr + 8 * (size_t)blockIdx.x;
+  if (KIND && (T[4] == 0.0) != (KIND == 1)) return;
+  long_triple<LE, ERR, KIND>(T, npts, Kp, eta, area, leg0, out + blockIdx.x * NSC,
                        ERR ? err + blockIdx.x * NSC : nullptr);
 }
 
 // Both sums of every triple in one launch, in-plane shifts: the long-range ones
-// first, they take longer. KIND 1, 2 (one wave per triple): only the triples of
-// real, complex k; the real ones need half the registers without the others'
-// arithmetic beside them, so two waves fit a SIMD up to LE 7 (2048 points, LE 7: 307
-// us against 498 with one kernel for both and one wave; few triples are better off
-// with one launch).
+// first, they take longer.
 template <int LE, int KIND>
-__global__ __launch_bounds__((KIND ? 64 : 64 * ew_waves<LE>()), (KIND && LE <= (KIND == 1 ? 7 : 5) ? 2 : 1)) void k_sigma_both(
+__global__ EW_BOUNDS(LE, KIND, true) void k_sigma_both(
     int ntrip, const double *__restrict__ tr, int nR, const double *__restrict__ R, int nK,
     const double *__restrict__ Kp, double eta, double area, const double *__restrict__ leg0, int csphase,
     v2d *__restrict__ ss, v2d *__restrict__ sl) {
@@ -760,11 +767,14 @@ extern "C" int qh_launch_sigma_short(int LE, int xy, int ntrip, const double *tr
   if (ntrip <= 0) return 0;
   hipStream_t s = (hipStream_t)qh_stream(stream);
   const dim3 g(ntrip), b = triple_threads(LE, xy && !err_dev, ntrip);
-#define QH_SS1(L, X, E) QH_LAUNCH((k_sigma_short<L, X, E>), g, b, 0, s, tr_dev, npts, pts_dev, eta, leg0_dev, \
+#define QH_SS1(L, X, E, K) QH_LAUNCH((k_sigma_short<L, X, E, K>), g, b, 0, s, tr_dev, npts, pts_dev, eta, leg0_dev, \
       csphase, (v2d *)out_dev, err_dev)
 #define QH_SS(L) case L: \
-    if (xy) { if (err_dev) QH_SS1(L, true, true); else QH_SS1(L, true, false); } \
-    else { if (err_dev) QH_SS1(L, false, true); else QH_SS1(L, false, false); } \
+    if (xy) { \
+      if (err_dev) QH_SS1(L, true, true, 0); \
+      else if (b.x > 64) QH_SS1(L, true, false, 0); \
+      else { QH_SS1(L, true, false, 1); QH_SS1(L, true, false, 2); } \
+    } else { if (err_dev) QH_SS1(L, false, true, 0); else QH_SS1(L, false, false, 0); } \
     break;
   switch (LE) {
     QH_SS(3) QH_SS(5) QH_SS(7) QH_SS(9)
@@ -783,14 +793,19 @@ extern "C" int qh_launch_sigma_long(int LE, int ntrip, const double *tr_dev, int
   hipStream_t s = (hipStream_t)qh_stream(stream);
   ensure_weid();   // the evanescent orders use the erfcx expansion
   const dim3 g(ntrip), b = triple_threads(LE, !err_dev, ntrip);
-#define QH_SL(L) case L: if (err_dev) QH_LAUNCH((k_sigma_long<L, true>), g, b, 0, s, tr_dev, npts, K_dev, eta, \
-      area, leg0_dev, (v2d *)out_dev, err_dev); else QH_LAUNCH((k_sigma_long<L, false>), g, b, 0, s, tr_dev, \
-      npts, K_dev, eta, area, leg0_dev, (v2d *)out_dev, err_dev); break;
+#define QH_SL1(L, E, K) QH_LAUNCH((k_sigma_long<L, E, K>), g, b, 0, s, tr_dev, npts, K_dev, eta, area, leg0_dev, \
+      (v2d *)out_dev, err_dev)
+#define QH_SL(L) case L: \
+    if (err_dev) QH_SL1(L, true, 0); \
+    else if (b.x > 64) QH_SL1(L, false, 0); \
+    else { QH_SL1(L, false, 1); QH_SL1(L, false, 2); } \
+    break;
   switch (LE) {
     QH_SL(3) QH_SL(5) QH_SL(7) QH_SL(9)
     default: qpms_hip_die(__FILE__, __LINE__, __func__, "Ewald lMax %d not instantiated (3, 5, 7, 9)", LE);
   }
 #undef QH_SL
+#undef QH_SL1
   HIPCHK(hipGetLastError());
   return 0;
 }

@@ -66,6 +66,21 @@ def test_batch_against_single(gpu, LE, n, nR, nK):
 
 
 @pytest.mark.parametrize("LE", [3, 5, 7, 9])
+def test_one_sum_against_both(gpu, LE):
+    """Enough triples for one wave each in launches of one sum; of both, and few."""
+    L, R, K = points(70, 130)
+    e3c = L.qpms_ewald3_constants_init(LE, -1)
+    t = triples(1100, np.random.default_rng(LE))
+    ss, sl = batch(L, e3c, LE, t, R, K)
+    close(batch(L, e3c, LE, t, R, K, "short")[0], ss, LE)
+    close(batch(L, e3c, LE, t, R, K, "long")[1], sl, LE)
+    few = t[:200]
+    close(batch(L, e3c, LE, few, R, K, "short")[0], ss[:200], LE)
+    close(batch(L, e3c, LE, few, R, K, "long")[1], sl[:200], LE)
+    L.qpms_ewald3_constants_free(e3c)
+
+
+@pytest.mark.parametrize("LE", [3, 5, 7, 9])
 @pytest.mark.parametrize("n, nK", [(1, 2435), (63, 15), (65, 17), (300, 0), (300, 161)])
 def test_shifts_against_single(gpu, LE, n, nK):
     import qpms_amd
