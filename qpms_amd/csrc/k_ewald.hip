@@ -177,12 +177,16 @@ __device__ __forceinline__ void short_triple(const double *__restrict__ T /* bx 
   auto points = [&](auto real) {
   constexpr bool REAL = decltype(real)::value;
   for (int ip = threadIdx.x; ip < npts; ip += blockDim.x) {
-    const double rx = pts[3 * ip] - T[5], ry = pts[3 * ip + 1] - T[6], rz = pts[3 * ip + 2] - T[7];
-    const double r = sqrt(rx * rx + ry * ry + rz * rz);
+    double rx = pts[3 * ip] - T[5], ry = pts[3 * ip + 1] - T[6], rz = pts[3 * ip + 2] - T[7];
+    double r = sqrt(rx * rx + ry * ry + rz * rz);
     // R = s: the lattice point coinciding with the particle (the origin for
     // s = 0, translations.c:981-987) carries no short-range term.
     const bool none = r == 0.0 || r * r * eta * eta - kap2re > 746.0;
-    if (__all(none)) continue;   // else zeros in such lanes: the sums are not held twice
+    if (__all(none)) continue;
+    // Else such lanes add zeros (the sums are not held twice): their I_n are zeroed
+    // below, and another place makes every other factor finite, which rz / r at r = 0
+    // and the phases of a point at infinity are not.
+    if (none) { rx = r = 1.0; ry = rz = 0.0; }
     const cplx eb = qew::expi_(T[0] * rx + T[1] * ry + T[2] * rz);
     // e^{i phi}, phi = atan2(ry, rx); on the z axis only m = 0 terms survive
     const double rho = XY ? r : sqrt(rx * rx + ry * ry), irho = qew::rcp_(rho);
@@ -218,7 +222,8 @@ __device__ __forceinline__ void short_triple(const double *__restrict__ T /* bx 
         for (int m = 1; m <= LE; ++m) em[m] = em[m - 1] * e1;
 #pragma unroll
         for (int n = 0; n <= LE; ++n) {
-          const cplx base = (pre[n] * In[n]) * eb;
+          cplx base = (pre[n] * In[n]) * eb;
+          if (none) base = mk(0.0, 0.0);   // (2/k)^{n+1} may overflow
 #pragma unroll
           for (int m = -n; m <= n; ++m) {
             const int am = cabsi(m);
@@ -473,11 +478,12 @@ __device__ __forceinline__ void long_triple(const double *__restrict__ T, int np
   auto points = [&](auto real) {
     constexpr bool REAL = decltype(real)::value;
     for (int ip = threadIdx.x; ip < npts; ip += blockDim.x) {
-      const double Kx = Kp[2 * ip], Ky = Kp[2 * ip + 1];
-      const LongPoint at = long_place(T, Kx, Ky);
+      double Kx = Kp[2 * ip], Ky = Kp[2 * ip + 1];
+      LongPoint at = long_place(T, Kx, Ky);
       double rk, gG[LE / 2 + 1];
       const int ev = REAL ? long_evanescent<LE>(at.rb, k.re, eta, rk, gG) : 0;
       if (REAL && __all(ev == 2)) continue;
+      if (REAL && ev == 2) { Kx = Ky = 0.0; at.e1 = mk(1.0, 0.0); }   // zeros times finite phases, at infinity too
       const cplx ph = shifted ? qew::expi_(Kx * T[5] + Ky * T[6]) : mk(1.0, 0.0);
       if (REAL && __any(ev == 1)) long_terms<LE>(rk, gG, ph, at.e1, add);
       if (!REAL || __any(ev == 0)) {
@@ -557,8 +563,10 @@ __global__ __launch_bounds__(64) void k_long_coef(const double *__restrict__ T, 
   bool live = true;
   double rk, gG[LE / 2 + 1];
   const int ev = k.im == 0.0 ? long_evanescent<LE>(at.rb, k.re, eta, rk, gG) : 0;
-  if (ev) {
+  if (ev == 1) {
     long_terms<LE>(rk, gG, mk(1.0, 0.0), at.e1, keep);
+  } else if (ev == 2) {
+    live = false;
   } else {
     cplx rc, gc[LE / 2 + 1];
     live = k.im == 0.0 ? long_general<LE, true>(at.rb, k, eta, rc, gc) : long_general<LE, false>(at.rb, k, eta, rc, gc);
