@@ -685,8 +685,7 @@ int qpms_hip_zgetrf_dev(size_t n, _Complex double *A_dev, int *ipiv_dev, void *s
  * 16 MiB device array of the library, so the order is limited to
  * qpms_hip_zgetrf_noalloc_max_n() (125,952); a larger n returns -1
  * with a message on stderr and touches nothing. Every call on a GPU shares
- * that GPU's array: calls that overlap on one GPU (other host threads, or
- * other streams before this call's synchronisation) race. Same results as
+ * that GPU's array, so calls of several host threads take turns. Same results as
  * qpms_hip_zgetrf_dev up to the rounding of the trailing GEMM (hand-written
  * MFMA kernel here). */
 int qpms_hip_zgetrf_dev_noalloc(size_t n, _Complex double *A_dev, int *ipiv_dev, void *stream);

@@ -303,14 +303,15 @@ beyn_result_t *beyn_solve_v(size_t m, size_t l, beyn_function_M_t M, beyn_functi
 	qh_h2d(dV, Vhat, ml * sizeof(complex double), NULL);
 	complex double *Mh = NULL, *dM = NULL, *Xh = NULL;
 	int *dpiv = NULL, *dperm = NULL, *dinfo = NULL;
-	void *dwork = NULL;
+	void *dwork = NULL;   /* of the factorisation, then of the solve */
 	if (!M_inv_Vhat) {
 		QH_MALLOC(Mh, m * m * sizeof(complex double));
 		dM = qh_dmalloc(m * m * sizeof(complex double));
 		dpiv = qh_dmalloc(m * sizeof(int));
 		dperm = qh_dmalloc(m * sizeof(int));
 		dinfo = qh_dmalloc(sizeof(int));
-		dwork = qh_dmalloc(qh_getrs_ws_bytes(64, (int)m, (int)l, 1));
+		const size_t lub = qh_getrf_ws_bytes(64, (int)m, 1), trb = qh_getrs_ws_bytes(64, (int)m, (int)l, 1);
+		dwork = qh_dmalloc(lub > trb ? lub : trb);
 	} else {
 		QH_MALLOC(Xh, ml * sizeof(complex double));
 	}
@@ -326,7 +327,7 @@ beyn_result_t *beyn_solve_v(size_t m, size_t l, beyn_function_M_t M, beyn_functi
 				qpms_hip_solve_mixed_dev(m, l, dM, dV, dX, 1e-17, 30, NULL);   /* refine to the FP64 floor */
 			} else {
 				qh_memset(dinfo, 0, sizeof(int), NULL);
-				qh_getrf_batched_f64((int)m, 1, (double *)dM, 0, dpiv, dperm, dinfo, NULL);
+				qh_getrf_batched_wsla_f64((int)m, 1, (double *)dM, 0, dpiv, dperm, dinfo, dwork, 1, NULL);
 				qh_copy_c64((long)ml, (const double *)dV, (double *)dX, NULL);
 				qh_getrs_ws_f64((int)m, (int)l, 1, (const double *)dM, 0, dperm, (double *)dX, 0, dwork, NULL);
 			}

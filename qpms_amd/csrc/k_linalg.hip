@@ -1559,10 +1559,10 @@ static bool use_rocblas() {
   return v == 1;
 }
 
-// Per-stream state of the LU driver: a rocBLAS handle bound to the stream
-// and the lookahead side stream with its two events. Created on a stream's
-// first use; qh_stream_release() destroys it, and callers that destroy a
-// stream (the serving loop's lanes) must call it first, so that a later
+// Per-stream state of the LU driver: a rocBLAS handle bound to the stream, the
+// lookahead's two events, and the workspace of callers that bring none. Created
+// on a stream's first use; qh_stream_release() destroys it, and callers that
+// destroy a stream (the serving loop's lanes) must call it first, so that a later
 // stream created at the same address never inherits a dead stream's state.
 struct LaCtx {
   hipEvent_t go, done;   // ordering of the caller's stream against the device's side stream
@@ -1574,6 +1574,8 @@ struct StreamState {
   rocblas_handle blas;   // nullptr until the first library GEMM on the stream
   bool la;               // lookahead context created
   LaCtx lc;
+  char *ws;              // see ws_for
+  size_t ws_bytes;
 };
 static std::mutex g_tab_mu;
 static StreamState g_tab[STREAM_TAB];
@@ -1601,6 +1603,20 @@ static rocblas_handle blas_for(hipStream_t s) {
     e->blas = h;
   }
   return e->blas;
+}
+
+// Workspace of the factorisations on a stream whose callers bring none. It holds
+// words that a strip's workgroups wait on, so no two streams may share one.
+static char *ws_for(hipStream_t s, size_t bytes) {
+  std::lock_guard<std::mutex> g(g_tab_mu);
+  StreamState *e = state_for(s);
+  if (bytes > e->ws_bytes) {
+    HIPCHK(hipStreamSynchronize(s));   // earlier factorisations may use it
+    qh_dfree(e->ws);
+    e->ws = (char *)qh_dmalloc(bytes);
+    e->ws_bytes = bytes;
+  }
+  return e->ws;
 }
 
 // CUs kept free of the side stream's trailing update, so that the next
@@ -1660,8 +1676,8 @@ static LaCtx *la_for(hipStream_t s, hipStream_t *side, bool *masked) {
   return &e->lc;
 }
 
-// Destroys the per-stream state of `stream` (rocBLAS handle, lookahead
-// events), after waiting for its work on the shared side stream.
+// Destroys the per-stream state of `stream` (rocBLAS handle, lookahead events,
+// workspace), after waiting for its work on the shared side stream.
 extern "C" void qh_stream_release(void *stream) {
   hipStream_t s = (hipStream_t)stream;
   std::lock_guard<std::mutex> g(g_tab_mu);
@@ -1674,6 +1690,7 @@ extern "C" void qh_stream_release(void *stream) {
       HIPCHK(hipEventDestroy(e.lc.done));
     }
     if (e.blas) rocblas_destroy_handle(e.blas);
+    qh_dfree(e.ws);   // waits for what uses it
     g_tab[i] = g_tab[--g_ntab];
     return;
   }
@@ -1935,12 +1952,11 @@ static size_t getrf_ws_bytes(int n, int batch) {
 // GEMM (K = PW); then U12 = L11^{-1} A12 in one launch (k_u12), and the trailing A22
 // -= L21 U12 (K = LU_NB).
 // ipiv (1-based, stride sP) lists the row interchanges as zgetrf's does;
-// perm (optional) tracks P; info[z] gets the first zero pivot. ws:
-// getrf_ws_bytes<T>(n, batch) bytes, or nullptr for a library-owned buffer
-// (single-stream callers only).
+// perm (optional) tracks P; info[z] gets the first zero pivot. ws: the call's own
+// until its work is done, LuWS<T>(n, batch, pp).bytes per matrix.
 template <class T>
 static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long sA, int *ipiv, long sP,
-                          int *perm, int *dinfo, hipStream_t s, char *ws = nullptr, bool lookahead = true,
+                          int *perm, int *dinfo, hipStream_t s, char *ws, bool lookahead = true,
                           bool own_gemm = false, bool pp = false, st_u64 wait = ST_LIMIT) {
   typedef typename C2<T>::t cT;
   constexpr int PW = PanelW<T>::W;
@@ -1950,17 +1966,6 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
   const LuWS<T> lay(n, batch, pp);
   const long sW = (long)lay.bytes;
   const long setb = (long)PanelWS<T>::set_bytes();
-  if (!ws) {
-    static char *own = nullptr;
-    static size_t own_bytes = 0;
-    const size_t need = (size_t)sW * batch;
-    if (need > own_bytes) {
-      if (own) { HIPCHK(hipStreamSynchronize(s)); qh_dfree(own); }
-      own = (char *)qh_dmalloc(need);
-      own_bytes = need;
-    }
-    ws = own;
-  }
   const dim3 bts(TS_THREADS);
   ts_prepare<T>();
   char *bufA = ws + lay.buf_a, *bufB = ws + lay.buf_b, *fin0 = ws + lay.fin;
@@ -2438,10 +2443,11 @@ static void getrs_batched(int n, int nrhs, int batch, const typename C2<T>::t *L
 
 extern "C" int qpms_hip_zgetrf_dev(size_t n, _Complex double *A_dev, int *ipiv_dev, void *stream) {
   hipStream_t s = (hipStream_t)qh_stream(stream);
-  int *dinfo = (int *)qh_dmalloc(sizeof(int));
+  // the info word and the workspace, this call's own
+  int *dinfo = (int *)qh_dmalloc(256 + (n < (1u << 22) ? LuWS<double>((int)n, 1, true).bytes : 0));
   HIPCHK(hipMemsetAsync(dinfo, 0, sizeof(int), s));
-  getrf_batched<double>((int)n, 1, (v2d *)A_dev, (long)n, 0, ipiv_dev, 0, nullptr, dinfo, s, nullptr, true, false,
-                        /*pp=*/true);
+  getrf_batched<double>((int)n, 1, (v2d *)A_dev, (long)n, 0, ipiv_dev, 0, nullptr, dinfo, s, (char *)dinfo + 256,
+                        true, false, /*pp=*/true);
   int info = 0;
   HIPCHK(hipMemcpyAsync(&info, dinfo, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
@@ -2456,10 +2462,11 @@ extern "C" int qpms_hip_zgetrf_dev(size_t n, _Complex double *A_dev, int *ipiv_d
 extern "C" int qh_getrf_pp(int prec, int n, double *A, int *ipiv, int *info, unsigned long long wait, void *stream) {
   hipStream_t s = (hipStream_t)qh_stream(stream);
   qh_zero(info, sizeof(int), s);
+  char *ws = ws_for(s, prec == 32 ? LuWS<float>(n, 1, true).bytes : LuWS<double>(n, 1, true).bytes);
   if (prec == 32)
-    getrf_batched<float>(n, 1, (v2f *)A, n, 0, ipiv, 0, nullptr, info, s, nullptr, true, false, true, wait);
+    getrf_batched<float>(n, 1, (v2f *)A, n, 0, ipiv, 0, nullptr, info, s, ws, true, false, true, wait);
   else
-    getrf_batched<double>(n, 1, (v2d *)A, n, 0, ipiv, 0, nullptr, info, s, nullptr, true, false, true, wait);
+    getrf_batched<double>(n, 1, (v2d *)A, n, 0, ipiv, 0, nullptr, info, s, ws, true, false, true, wait);
   return 0;
 }
 
@@ -2561,6 +2568,7 @@ constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)16 << 20;
 static __device__ __align__(256) char scratch[NOALLOC_SCRATCH_BYTES];
 constexpr int NOALLOC_MAX_DEV = 64;
 static char *g_scratch_ptr[NOALLOC_MAX_DEV];   // device address of `scratch`, per device
+static std::mutex g_scratch_mu[NOALLOC_MAX_DEV];   // held by the call that uses the array, until its work is done
 
 // Called by the library's initialisation with the device current (once per
 // device); records the device address of the scratch array.
@@ -2593,6 +2601,7 @@ extern "C" int qpms_hip_zgetrf_dev_noalloc(size_t n, _Complex double *A_dev, int
   if (!base) qpms_hip_die(__FILE__, __LINE__, __func__, "scratch of device %d not initialised", dev);
   if (256 + LuWS<double>((int)n, 1, true).bytes > NOALLOC_SCRATCH_BYTES)
     qpms_hip_die(__FILE__, __LINE__, __func__, "scratch too small for order %zu", n);
+  std::lock_guard<std::mutex> turn(g_scratch_mu[dev]);
   int *dinfo = (int *)base;
   qh_zero(dinfo, 256, s);   // a kernel: the info word must start at zero on every call
   getrf_batched<double>((int)n, 1, (v2d *)A_dev, (long)n, 0, ipiv_dev, 0, nullptr, dinfo, s, base + 256,
@@ -2627,11 +2636,14 @@ extern "C" int qh_launch_block_tw(size_t nr, size_t L, const double *T, const do
 }
 
 // ---------------------------------------------------------------------------
-// Batched LU / solve entry points used by Beyn and the serving loop.
+// Batched LU / solve entry points used by Beyn and the serving loop. Without a
+// workspace of the caller's: that of the stream, one thread at a time.
 // ---------------------------------------------------------------------------
 extern "C" int qh_getrf_batched_f64(int n, int batch, double *A, long sA, int *ipiv, int *perm, int *info,
                                     void *stream) {
-  getrf_batched<double>(n, batch, (v2d *)A, n, sA, ipiv, n, perm, info, (hipStream_t)qh_stream(stream));
+  hipStream_t s = (hipStream_t)qh_stream(stream);
+  if (n <= 0 || batch <= 0) return 0;
+  getrf_batched<double>(n, batch, (v2d *)A, n, sA, ipiv, n, perm, info, s, ws_for(s, getrf_ws_bytes<double>(n, batch)));
   return 0;
 }
 extern "C" size_t qh_getrf_ws_bytes(int prec, int n, int batch) {
@@ -2713,7 +2725,9 @@ extern "C" int qh_getrs_batched_f64(int n, int nrhs, int batch, const double *LU
 }
 extern "C" int qh_getrf_batched_f32(int n, int batch, float *A, long sA, int *ipiv, int *perm, int *info,
                                     void *stream) {
-  getrf_batched<float>(n, batch, (v2f *)A, n, sA, ipiv, n, perm, info, (hipStream_t)qh_stream(stream));
+  hipStream_t s = (hipStream_t)qh_stream(stream);
+  if (n <= 0 || batch <= 0) return 0;
+  getrf_batched<float>(n, batch, (v2f *)A, n, sA, ipiv, n, perm, info, s, ws_for(s, getrf_ws_bytes<float>(n, batch)));
   return 0;
 }
 // (work: n x nrhs x batch entries of scratch, as an earlier form of the solve
@@ -2802,10 +2816,11 @@ extern "C" int qpms_hip_solve_mixed_dev(size_t n_, size_t nrhs_, const _Complex 
   int *dinfo = (int *)qh_dmalloc(sizeof(int));
   double *R = (double *)qh_dmalloc(nb * sizeof(v2d));
   float *R32 = (float *)qh_dmalloc(nb * sizeof(v2f));
-  void *W32 = qh_dmalloc(getrs_ws_bytes<float>(n, nrhs, 1));
+  // words of the solves, and before them of the factorisation
+  void *W32 = qh_dmalloc(std::max(getrs_ws_bytes<float>(n, nrhs, 1), getrf_ws_bytes<float>(n, 1)));
   HIPCHK(hipMemsetAsync(dinfo, 0, sizeof(int), s));
   qh_d2f(nn, (const double *)A_dev, A32, s);
-  getrf_batched<float>(n, 1, (v2f *)A32, n, 0, ipiv, 0, perm, dinfo, s);
+  getrf_batched<float>(n, 1, (v2f *)A32, n, 0, ipiv, 0, perm, dinfo, s, (char *)W32);
   HIPCHK(hipMemsetAsync(X_dev, 0, nb * sizeof(v2d), s));
   const double normA = qh_norm2_c64(nn, (const double *)A_dev, s);
   const double normB = qh_norm2_c64(nb, (const double *)B_dev, s);
@@ -2837,11 +2852,11 @@ extern "C" int qpms_hip_solve_mixed_dev(size_t n_, size_t nrhs_, const _Complex 
   int *ip = (int *)qh_dmalloc(n * sizeof(int));
   int *pm = (int *)qh_dmalloc(n * sizeof(int));
   int *inf = (int *)qh_dmalloc(sizeof(int));
-  void *work = qh_dmalloc(getrs_ws_bytes<double>(n, nrhs, 1));
+  void *work = qh_dmalloc(std::max(getrs_ws_bytes<double>(n, nrhs, 1), getrf_ws_bytes<double>(n, 1)));
   HIPCHK(hipMemsetAsync(inf, 0, sizeof(int), s));
   qh_copy_c64(nn, (const double *)A_dev, A64, s);
   qh_copy_c64(nb, (const double *)B_dev, (double *)X_dev, s);
-  getrf_batched<double>(n, 1, (v2d *)A64, n, 0, ip, 0, pm, inf, s);
+  getrf_batched<double>(n, 1, (v2d *)A64, n, 0, ip, 0, pm, inf, s, (char *)work);
   getrs_batched<double>(n, nrhs, 1, (const v2d *)A64, n, 0, pm, 0, (v2d *)X_dev, nrhs, 0, work, s);
   HIPCHK(hipStreamSynchronize(s));
   qh_dfree(A64); qh_dfree(ip); qh_dfree(pm); qh_dfree(inf); qh_dfree(work);

@@ -77,7 +77,10 @@ int qh_getrs_batched_f64(int n, int nrhs, int batch, const double *LU, long sA, 
 int qh_getrf_batched_f32(int n, int batch, float *A, long sA, int *ipiv, int *perm, int *info, void *stream);
 int qh_getrs_batched_f32(int n, int nrhs, int batch, const float *LU, long sA, const int *perm,
 		float *B, long sB, float *work, void *stream);
-/* The same with caller's scratch of qh_getrs_ws_bytes (prec 32, 64): no allocation, no wait. */
+/* The same with caller's scratch of qh_getrf_ws_bytes / qh_getrs_ws_bytes (prec 32, 64): no allocation, no wait. */
+size_t qh_getrf_ws_bytes(int prec, int n, int batch);
+int qh_getrf_batched_wsla_f64(int n, int batch, double *A, long sA, int *ipiv, int *perm, int *info, void *ws,
+		int lookahead, void *stream);
 size_t qh_getrs_ws_bytes(int prec, int n, int nrhs, int batch);
 int qh_getrs_ws_f64(int n, int nrhs, int batch, const double *LU, long sA, const int *perm,
 		double *B, long sB, void *ws, void *stream);
