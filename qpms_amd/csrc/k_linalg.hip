@@ -2088,16 +2088,20 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
 // of G owns the 64-row blocks g, g + G, ... of 16 right-hand-side columns. For a
 // block it subtracts the products with the blocks solved before (each wave a
 // quarter of their columns, by matrix instructions, the sums added in a fixed
-// order), multiplies with the inverse of its diagonal block, which it made while
-// others were solving, and publishes the result; backward the same from below.
+// order), substitutes with its diagonal block, and publishes the result; backward the
+// same from below.
 //
-// What bounds it: the chain of blocks, 6.3 us each in FP64 and 4.1 in FP32 (the
-// words' way to the next workgroup, then 64 matrix instructions in a row for the
-// last block's columns and up to 64 for the inverse). As launches per 64-row block
-// (a wave substituting, 18-22 us, then an update, 17 us) an FP64 solve of order
-// 9216 took 10.5 ms, now 2.0; per 256-row block (130 us + 70 us) an FP32 one of
-// order 9990 with 32 right-hand sides 16 ms, now 1.8. Loading the next product's
-// operands or words ahead gained nothing.
+// What bounds it: the chain of blocks, 7 to 8 us each in FP64 and 5 in FP32 for up to
+// four columns, 11 to 14 and 7 to 10 for 16 (the words' way to the next workgroup, 64
+// matrix instructions in a row for the last block's columns, 2 of the 7 us, and the
+// substitution, 2 to 3 us). As launches per 64-row block (a wave substituting, 18-22
+// us, then an update, 17 us) an FP64 solve of order 9216 took 10.5 ms, now 2.4; per
+// 256-row block (130 us + 70 us) an FP32 one of order 9990 with 32 right-hand sides 16
+// ms, now 3.1. With the diagonal block's inverse, made while others were solving, in
+// the substitution's place the blocks took 6.3 and 4.1 us, but the error (FP64 factors
+// of random matrices and of clusters', orders 64 to 512, against 80 bits) was 1.3 to 2
+// times that of the launches' substitution; now it is 0.2 to 1.0 times. Loading the
+// next product's operands or words ahead gained nothing.
 //
 // Published values carry a tag (1 forward, 2 backward) beside each 32 bits, as
 // the strips' words do, so a reader needs no flag. Forward values are all read
@@ -2108,7 +2112,7 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
 // ---------------------------------------------------------------------------
 constexpr int TR_B = 64, TR_C = 16, TR_VS = TR_B + 1, TR_XS = TR_C + 1;
 constexpr int TR_MEET = 256;   // most workgroups of a slab
-template <class T> constexpr size_t tr_lds() {   // diagonal block, the waves' sums, the diagonal's reciprocals
+template <class T> constexpr size_t tr_lds() {   // the diagonal block without its diagonal, the waves' sums, the diagonal
   return (size_t)(TR_B * TR_VS + 4 * TR_B * TR_XS + TR_B) * sizeof(typename C2<T>::t);
 }
 template <class T> constexpr size_t tr_slab_bytes(int n, int nrhs) {
@@ -2123,96 +2127,167 @@ __device__ __forceinline__ void tr_each(F f, std::integer_sequence<int, K...>) {
   (f(std::integral_constant<int, K>{}), ...);
 }
 
-// The 64 x 64 triangular block V (LDS, row stride TR_VS; UPPER: with dinv its
-// diagonal's reciprocals; zeros in the other triangle) is replaced by its inverse,
-// all 256 threads. W: scratch. UPPER works on the block turned
-// round (row and column i for 63 - i), where it is lower triangular. The four
-// 16 x 16 diagonal blocks by substitution, one per wave, four lanes per column;
-// then [A 0; B C] of twice the size, whose inverse's corner is -C^-1 (B A^-1), by
-// matrix instructions, twice. Substitution with the whole block (64 steps in a
-// row, each waiting for LDS) took 35 us, this way 5. The solutions' errors in FP64
-// (80-bit reference, orders 64 to 1024) are 1.3 to 2 times those of
-// substitution throughout, 4e-16 for systems near the identity; a residual
-// correction per block brought 1.0 to 1.4 times for twice the chain.
-template <class T, bool UPPER>
-__device__ __forceinline__ void tr_invert(typename C2<T>::t *V, const typename C2<T>::t *dinv, typename C2<T>::t *W,
-                                          int wave, int lane) {
+// 1 / d 2^e in two parts (the second the first one's error) for a diagonal entry d of
+// U, e = 0 unless its square or reciprocal might leave the range. A product with both
+// parts is as good as a division by d, and no division waits in the chain of rows.
+template <class T> struct TrRecip {
+  typename C2<T>::t hi, lo;
+  int e;
+};
+template <class T>
+__device__ __forceinline__ TrRecip<T> tr_recip(typename C2<T>::t d) {
+#pragma clang fp contract(off)
   typedef typename C2<T>::t cT;
-  typedef typename MF<T>::acc acc_t;
-  auto at = [&](int r, int c) -> cT & { return V[UPPER ? (TR_B - 1 - r) * TR_VS + TR_B - 1 - c : r * TR_VS + c]; };
-  const int cls = lane & 3, col = lane >> 2, o = 16 * wave, lr = lane & 15, lk = lane >> 4;
-  {
-    cT x[4];
+  constexpr T BIG = sizeof(T) == 8 ? T(0x1p500) : T(0x1p60f);
+  TrRecip<T> r;
+  const T m = fmax(fabs(d.x), fabs(d.y));
+  r.e = 0;
+  if (m > 0 && m < T(INFINITY) && !(m > 1 / BIG && m < BIG)) {
+    r.e = ilogb(m);
+    d = cT{ldexp(d.x, -r.e), ldexp(d.y, -r.e)};
+  }
+  r.hi = cdiv<T>(cT{1, 0}, d);
+  // 1 - d hi, exactly but for the products' own errors: the two products of the real
+  // part add up to one, those of the imaginary part to nothing
+  const T a = d.x * r.hi.x, b = -d.y * r.hi.y, ea = fma(d.x, r.hi.x, -a), eb = fma(-d.y, r.hi.y, -b);
+  const T c = d.x * r.hi.y, f = d.y * r.hi.x, ec = fma(d.x, r.hi.y, -c), ef = fma(d.y, r.hi.x, -f);
+  const cT err = cT{((1 - fmax(a, b)) - fmin(a, b)) - (ea + eb), -(c + f) - (ec + ef)};
+  r.lo = cmul<T>(err, r.hi);
+  return r;
+}
+
+// The value of lane K: of the lane's row of 16 (LN = 16), of the wave.
+template <int LN, int K> __device__ __forceinline__ unsigned tr_lane(unsigned v) {
+  if constexpr (LN == 16) return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + K, 0xF, 0xF, true);   // row_newbcast
+  else return (unsigned)__builtin_amdgcn_readlane((int)v, K);
+}
+template <int LN, int K> __device__ __forceinline__ float tr_bc(float v) { return __uint_as_float(tr_lane<LN, K>(__float_as_uint(v))); }
+template <int LN, int K> __device__ __forceinline__ double tr_bc(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = tr_lane<LN, K>((unsigned)b), hi = tr_lane<LN, K>((unsigned)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// v / d
+template <class T>
+__device__ __forceinline__ typename C2<T>::t tr_div(typename C2<T>::t v, const TrRecip<T> &d, bool scaled) {
+  typedef typename C2<T>::t cT;
+  const cT h = d.hi, l = d.lo;
+  const cT y = cT{fma(v.x, h.x, fma(-v.y, h.y, fma(v.x, l.x, -v.y * l.y))), fma(v.x, h.y, fma(v.y, h.x, fma(v.x, l.y, v.y * l.x)))};
+  return scaled ? cT{ldexp(y.x, -d.e), ldexp(y.y, -d.e)} : y;
+}
+
+// Substitution with a triangular block of LN R rows at V (LDS, row stride TR_VS;
+// strictly lower or upper, zeros elsewhere; UPPER: dinv the lane's diagonal entries'
+// reciprocals), LN lanes per column: x[q] is row LN q + cls of the lane's column,
+// less[q] what the rows solved before the block take from it. The row's other products
+// are added to less, and the sum subtracted once: subtracted one by one they cost a
+// rounding of x's size each. Every step's solved entry goes round the column's lanes.
+// All lanes add: the zeros keep the solved rows, but for an entry that is no finite
+// number; with any of those, or diagonal entries near the limits of the range, the rows
+// are solved again, under conditions. V's entries come four steps ahead.
+// What bounds it: a step's instructions, with one wave on a SIMD; with a wave on all
+// four, V's way from LDS as much.
+template <class T, bool UPPER, int LN, int R>
+__device__ __forceinline__ void tr_substitute(const typename C2<T>::t *V, const TrRecip<T> (&dinv)[R], int cls,
+                                              typename C2<T>::t (&x)[R], typename C2<T>::t (&less)[R]) {
+  typedef typename C2<T>::t cT;
+  constexpr int N = LN * R;
+  bool odd = false;
+  if (UPPER)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) x[q] = cT{4 * q + cls == col ? T(1) : T(0), 0};
-    auto step = [&](auto kc) {
-      constexpr int K = decltype(kc)::value;
-      cT v = cT{su_bc<(K & 3)>(x[K / 4].x), su_bc<(K & 3)>(x[K / 4].y)};
-      if (UPPER) {
-        v = cmul<T>(v, dinv[TR_B - 1 - o - K]);
-        if (cls == (K & 3)) x[K / 4] = v;
-      }
+    for (int q = 0; q < R; ++q) odd |= dinv[q].e != 0;
+  const bool scaled = __any(odd);
+  cT l[2][4][R], pre[R], pim[R], rest[R];   // 8 steps' products with l's real and imaginary part; x - less
 #pragma unroll
-      for (int q = K / 4; q < 4; ++q) {
-        const cT l = at(o + 4 * q + cls, o + K);
-        const cT y = cT{fma(-l.x, v.x, fma(l.y, v.y, x[q].x)), fma(-l.x, v.y, fma(-l.y, v.x, x[q].y))};
-        if (q > K / 4 || cls > (K & 3)) x[q] = y;
+  for (int q = 0; q < R; ++q) {
+    pre[q] = pim[q] = cT{0, 0};
+    rest[q] = x[q] - less[q];
+  }
+  auto load = [&](auto cc) {   // the entries of steps 4 C .. 4 C + 3
+    constexpr int C = decltype(cc)::value, Q = UPPER ? R - 1 - 4 * C / LN : 4 * C / LN;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int col = UPPER ? N - 1 - 4 * C - i : 4 * C + i;
+#pragma unroll
+      for (int q = UPPER ? 0 : Q; q <= (UPPER ? Q : R - 1); ++q) l[C & 1][i][q] = V[(LN * q + cls) * TR_VS + col];
+    }
+    asm volatile("" ::: "memory");   // not earlier than here, nor later
+  };
+  load(std::integral_constant<int, 0>{});
+  auto chunk = [&](auto cc) {
+    constexpr int C = decltype(cc)::value, Q = UPPER ? R - 1 - 4 * C / LN : 4 * C / LN;
+    if constexpr (C + 1 < N / 4) load(std::integral_constant<int, C + 1>{});
+    auto step = [&](auto ic) {
+      constexpr int I = decltype(ic)::value, K = UPPER ? LN - 1 - (4 * C + I) % LN : (4 * C + I) % LN;
+      cT v = rest[Q] - cT{pre[Q].x - pim[Q].y, pre[Q].y + pim[Q].x};
+      if (UPPER) v = tr_div<T>(v, dinv[Q], false);
+      v = cT{tr_bc<LN, K>(v.x), tr_bc<LN, K>(v.y)};
+#pragma unroll
+      for (int q = UPPER ? 0 : Q; q <= (UPPER ? Q : R - 1); ++q) {
+        const cT e = l[C & 1][I][q];
+        pre[q] = cT{fma(e.x, v.x, pre[q].x), fma(e.x, v.y, pre[q].y)};
+        pim[q] = cT{fma(e.y, v.x, pim[q].x), fma(e.y, v.y, pim[q].y)};
       }
+      __builtin_amdgcn_sched_barrier(0);   // put off, the other rows' products would hold their factors in registers
     };
-    tr_each(step, std::make_integer_sequence<int, 16>{});
-    // only this wave reads its block
+    tr_each(step, std::make_integer_sequence<int, 4>{});
+    if constexpr (C % 2 == 1 && C + 1 < N / 4) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      at(o + 4 * q + cls, o + col) = x[q];
-  }
-  __syncthreads();
-  // 32 x 32: wave w the real (even) or imaginary (odd) parts for pair w / 2
-  const int pair = wave >> 1, part = wave & 1, a0 = 32 * pair, c0 = a0 + 16;
-  T *Wt = reinterpret_cast<T *>(W);
-  auto corner = [&](auto &&A, auto &&X) {
-    acc_t p = acc_t{0, 0, 0, 0};
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const cT a = A(lr, 4 * ks + lk), x = X(4 * ks + lk, lr);
-      p = MF<T>::mma(part ? a.y : a.x, x.x, p);
-      p = MF<T>::mma(part ? a.x : -a.y, x.y, p);
-    }
-    return p;
-  };
-  {
-    const acc_t p = corner([&](int r, int k) { return at(c0 + r, a0 + k); }, [&](int k, int c) { return at(a0 + k, a0 + c); });
-#pragma unroll
-    for (int e = 0; e < 4; ++e) Wt[2 * ((16 * pair + MF<T>::row(lk, e)) * TR_XS + lr) + part] = p[e];
-  }
-  __syncthreads();
-  {
-    const acc_t p = corner([&](int r, int k) { return at(c0 + r, c0 + k); }, [&](int k, int c) { return W[(16 * pair + k) * TR_XS + c]; });
-#pragma unroll
-    for (int e = 0; e < 4; ++e) reinterpret_cast<T *>(&at(c0 + MF<T>::row(lk, e), a0 + lr))[part] = -p[e];
-  }
-  __syncthreads();
-  // 64 x 64: a 16 x 16 tile of the corner per wave, without the triangles' zero tiles
-  const int ti = wave >> 1, tj = wave & 1;
-  auto product = [&](int k0, int k1, auto &&A, auto &&X, acc_t &re, acc_t &im) {
-    re = im = acc_t{0, 0, 0, 0};
-#pragma unroll 4
-    for (int ks = k0; ks < k1; ++ks) {
-      const cT a = A(16 * ti + lr, 4 * ks + lk), x = X(4 * ks + lk, 16 * tj + lr);
-      re = MF<T>::mma(a.x, x.x, re);
-      im = MF<T>::mma(a.x, x.y, im);
-      re = MF<T>::mma(-a.y, x.y, re);
-      im = MF<T>::mma(a.y, x.x, im);
+      for (int q = UPPER ? 0 : Q; q <= (UPPER ? Q : R - 1); ++q) {
+        less[q] += cT{pre[q].x - pim[q].y, pre[q].y + pim[q].x};
+        pre[q] = pim[q] = cT{0, 0};
+        rest[q] = x[q] - less[q];
+      }
     }
   };
-  acc_t re, im;
-  product(4 * tj, 8, [&](int r, int k) { return at(32 + r, k); }, [&](int k, int c) { return at(k, c); }, re, im);
+  cT start[R];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) W[(16 * ti + MF<T>::row(lk, e)) * TR_VS + 16 * tj + lr] = cT{re[e], im[e]};
-  __syncthreads();
-  product(0, 4 * ti + 4, [&](int r, int k) { return at(32 + r, 32 + k); }, [&](int k, int c) { return W[k * TR_VS + c]; }, re, im);
+  for (int q = 0; q < R; ++q) start[q] = less[q];
+  tr_each(chunk, std::make_integer_sequence<int, N / 4>{});
 #pragma unroll
-  for (int e = 0; e < 4; ++e) at(32 + 16 * ti + MF<T>::row(lk, e), 16 * tj + lr) = cT{-re[e], -im[e]};
-  __syncthreads();
+  for (int q = 0; q < R; ++q) {
+    less[q] += cT{pre[q].x - pim[q].y, pre[q].y + pim[q].x};
+    odd |= !(fabs(less[q].x) + fabs(less[q].y) < T(INFINITY));
+  }
+  if (__any(odd)) {
+#pragma unroll
+    for (int q = 0; q < R; ++q) less[q] = start[q];
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      const int Q = UPPER ? R - 1 - u : u;
+#pragma unroll 1
+      for (int j = 0; j < LN; j += 8) {   // the same roundings as above
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          pre[q] = pim[q] = cT{0, 0};
+          rest[q] = x[q] - less[q];
+        }
+#pragma unroll 1
+        for (int i = j; i < j + 8; ++i) {
+          const int k = UPPER ? LN - 1 - i : i, from = (threadIdx.x & 63 & -LN) | k;
+          cT v = rest[Q] - cT{pre[Q].x - pim[Q].y, pre[Q].y + pim[Q].x};
+          if (UPPER) v = tr_div<T>(v, dinv[Q], scaled);
+          v = cT{__shfl(v.x, from), __shfl(v.y, from)};
+#pragma unroll
+          for (int q = UPPER ? 0 : Q; q <= (UPPER ? Q : R - 1); ++q) {
+            const cT e = V[(LN * q + cls) * TR_VS + LN * Q + k];
+            if (q != Q || (UPPER ? cls < k : cls > k)) {
+              pre[q] = cT{fma(e.x, v.x, pre[q].x), fma(e.x, v.y, pre[q].y)};
+              pim[q] = cT{fma(e.y, v.x, pim[q].x), fma(e.y, v.y, pim[q].y)};
+            }
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < R; ++q) less[q] += cT{pre[q].x - pim[q].y, pre[q].y + pim[q].x};
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    x[q] -= less[q];
+    if (UPPER) x[q] = tr_div<T>(x[q], dinv[q], scaled);
+  }
 }
 
 template <class T>
@@ -2239,15 +2314,15 @@ __device__ __forceinline__ void tr_publish(st_u64 *at, unsigned tag, typename C2
 }
 
 template <class T>
-__global__ __launch_bounds__(256, 1) void k_tri(int n, int nrhs, const typename C2<T>::t *LU, long lda, long sA,
+__global__ __launch_bounds__(256, (sizeof(T) == 4 ? 2 : 1)) void k_tri(int n, int nrhs, const typename C2<T>::t *LU, long lda, long sA,
                                                 const int *perm, long sP, typename C2<T>::t *B, long ldb, long sB,
                                                 char *ws, long sW, long slabb, st_u64 limit) {
   typedef typename C2<T>::t cT;
   typedef typename MF<T>::acc acc_t;
   constexpr int EW = st_ew<T>();
   extern __shared__ __align__(16) char smem_raw[];
-  cT *V = reinterpret_cast<cT *>(smem_raw);   // the diagonal block, then its inverse
-  cT *S = V + TR_B * TR_VS, *dinv = S + 4 * TR_B * TR_XS;
+  cT *V = reinterpret_cast<cT *>(smem_raw);
+  cT *S = V + TR_B * TR_VS, *D = S + 4 * TR_B * TR_XS;
   __shared__ int go;
   const int z = blockIdx.z, t = threadIdx.x, lane = t & 63, lr = lane & 15, lk = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -2271,26 +2346,31 @@ __global__ __launch_bounds__(256, 1) void k_tri(int n, int nrhs, const typename 
     const int mine = (nblk - 1 - g) / G + 1;   // blocks of this workgroup
     for (int b = 0; b < mine; ++b) {
       const int i = g + G * (UPPER ? mine - 1 - b : b), r0 = i * TR_B;
-      // the diagonal block and its inverse
+      // the diagonal block
       {
         cT v[16];
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
           const int e = t + 256 * q, r = e >> 6, c = e & 63;
           const bool in = r0 + r < n && r0 + c < n && (UPPER ? c >= r : c < r);
-          v[q] = in ? LU[(long)(r0 + r) * lda + r0 + c] : cT{r == c ? T(1) : T(0), 0};
+          v[q] = in ? LU[(long)(r0 + r) * lda + r0 + c] : cT{UPPER && r == c ? T(1) : T(0), 0};
         }
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
           const int e = t + 256 * q, r = e >> 6, c = e & 63;
-          V[r * TR_VS + c] = v[q];
+          if (UPPER && r == c) D[r] = v[q];
+          V[r * TR_VS + c] = r == c ? cT{0, 0} : v[q];
         }
         __syncthreads();
-        if (UPPER) {
-          if (t < TR_B) dinv[t] = cdiv<T>(cT{1, 0}, V[t * TR_VS + t]);
-          __syncthreads();
+      }
+      TrRecip<T> dinv[2][2], dinv1[1];   // its diagonal's reciprocals, as the substitutions take them
+      if (UPPER) {
+        if (cs > 4) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) dinv[q >> 1][q & 1] = tr_recip<T>(D[16 * q + lr]);
+        } else {
+          dinv1[0] = tr_recip<T>(D[lane]);
         }
-        tr_invert<T, UPPER>(V, dinv, S, wave, lane);
       }
       // this wave's 16 rows of the right-hand side, as results of matrix
       // instructions: rows of P B, or what the forward sweep left
@@ -2318,9 +2398,23 @@ __global__ __launch_bounds__(256, 1) void k_tri(int n, int nrhs, const typename 
         ri[e] = v.y;
       }
       // less the products with the blocks solved before, a quarter of their columns per wave
+      // (block by block, added in LDS: as one chain over all blocks their rounding
+      // errors were twice as large at order 1024)
       acc_t pr[4], pi[4];
+      auto sums = [&](bool first) {
 #pragma unroll
-      for (int T_ = 0; T_ < 4; ++T_) { pr[T_] = acc_t{0, 0, 0, 0}; pi[T_] = acc_t{0, 0, 0, 0}; }
+        for (int T_ = 0; T_ < 4; ++T_) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            cT &at = S[(wave * TR_B + 16 * T_ + MF<T>::row(lk, e)) * TR_XS + lr];
+            const cT v = cT{pr[T_][e], pi[T_][e]};
+            at = first ? v : at + v;
+          }
+          pr[T_] = pi[T_] = acc_t{0, 0, 0, 0};
+        }
+      };
+#pragma unroll
+      for (int T_ = 0; T_ < 4; ++T_) pr[T_] = pi[T_] = acc_t{0, 0, 0, 0};
       const int nb = UPPER ? nblk - 1 - i : i;
       for (int q = 0; q < nb; ++q) {
         const int k0 = (UPPER ? nblk - 1 - q : q) * TR_B + 16 * wave + lk;
@@ -2359,44 +2453,81 @@ __global__ __launch_bounds__(256, 1) void k_tri(int n, int nrhs, const typename 
             pr[T_] = MF<T>::mma(-a[T_][ks].y, x[ks].y, pr[T_]);
             pi[T_] = MF<T>::mma(a[T_][ks].y, x[ks].x, pi[T_]);
           }
+        if (q + 1 < nb) sums(q == 0);
       }
-#pragma unroll
-      for (int T_ = 0; T_ < 4; ++T_)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          S[(wave * TR_B + 16 * T_ + MF<T>::row(lk, e)) * TR_XS + lr] = cT{pr[T_][e], pi[T_][e]};
+      sums(nb <= 1);
       __syncthreads();
+      cT sum[4];
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const cT v = S[(k * TR_B + 16 * wave + MF<T>::row(lk, e)) * TR_XS + lr];
-          rr[e] -= v.x;
-          ri[e] -= v.y;
-        }
-      // times the inverse, 16 rows per wave, the triangle's columns only; shared in
-      // sums that no other wave reads
-      auto shared = [&](int r) { return S + (long)((r >> 4) * TR_B + r) * TR_XS + lr; };
-#pragma unroll
-      for (int e = 0; e < 4; ++e) *shared(16 * wave + MF<T>::row(lk, e)) = cT{rr[e], ri[e]};
-      __syncthreads();
-      acc_t yr = acc_t{0, 0, 0, 0}, yi = acc_t{0, 0, 0, 0};
-#pragma unroll 4
-      for (int ks = UPPER ? 4 * wave : 0; ks < (UPPER ? 16 : 4 * wave + 4); ++ks) {
-        const cT a = V[(16 * wave + lr) * TR_VS + 4 * ks + lk], x = *shared(4 * ks + lk);
-        yr = MF<T>::mma(a.x, x.x, yr);
-        yi = MF<T>::mma(a.x, x.y, yi);
-        yr = MF<T>::mma(-a.y, x.y, yr);
-        yi = MF<T>::mma(a.y, x.x, yi);
+      for (int e = 0; e < 4; ++e) {
+        const cT *at = S + (16 * wave + MF<T>::row(lk, e)) * TR_XS + lr;
+        sum[e] = (at[0] + at[TR_B * TR_XS]) + (at[2 * TR_B * TR_XS] + at[3 * TR_B * TR_XS]);
       }
-      if (lr < cs) {
+      // a wave's rows and their sums to the lanes that solve their columns, in parts that
+      // no other wave reads
+      auto part = [&](int r, int c, int p) { return S + (long)(((r >> 4) ^ p) * TR_B + r) * TR_XS + c; };
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int r = rw + MF<T>::row(lk, e);
-          const cT v = cT{yr[e], yi[e]};
-          tr_publish<T>(X + ((long)r * cs + lr) * EW, tag, v);
-          if (UPPER && r < n && lr < nc) B[(long)r * ldb + lr] = v;
+      for (int e = 0; e < 4; ++e) {
+        const int r = 16 * wave + MF<T>::row(lk, e);
+        *part(r, lr, 0) = cT{rr[e], ri[e]};
+        *part(r, lr, 1) = sum[e];
+      }
+      __syncthreads();
+      auto done = [&](int row, int c, cT x) {
+        const int r = r0 + row;
+        if (c < cs) tr_publish<T>(X + ((long)r * cs + c) * EW, tag, x);
+        if (UPPER && r < n && c < nc) B[(long)r * ldb + c] = x;
+      };
+      // up to four columns a wave each (order 1040, one column: 223 us in FP64, 151 in
+      // FP32, against 259 and 191 with 16 lanes), more 16 lanes each
+      if (cs <= 4) {
+        if (wave < cs) {
+          cT xs[1] = {*part(lane, wave, 0)}, ls[1] = {*part(lane, wave, 1)};
+          tr_substitute<T, UPPER, 64, 1>(V, dinv1, lane, xs, ls);
+          done(lane, wave, xs[0]);
         }
+      } else {   // the block's halves one after the other (as one 11.4, 7.8 us a block, so 10.7, 6.9)
+        const int c = 4 * wave + lk;
+        auto half = [&](auto hc) {
+          constexpr int H = decltype(hc)::value, o = 32 * H;
+          constexpr bool SECOND = UPPER ? H == 0 : H == 1;
+          if (4 * wave < cs) {   // uniform
+            cT xs[2], ls[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              const int r = o + 16 * q + lr;
+              xs[q] = *part(r, c, 0);
+              ls[q] = *part(r, c, 1);
+              if (SECOND) ls[q] += *part(r, c, 2) + *part(r, c, 3);
+            }
+            tr_substitute<T, UPPER, 16, 2>(V + o * TR_VS + o, dinv[H], lr, xs, ls);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              const int r = o + 16 * q + lr;
+              done(r, c, xs[q]);
+              if (!SECOND) *part(r, c, 0) = xs[q];
+            }
+          }
+        };
+        half(std::integral_constant<int, UPPER ? 1 : 0>{});
+        __syncthreads();
+        {   // what the first half takes from the second: 16 rows and 16 columns of V per wave
+          constexpr int o0 = UPPER ? 32 : 0, o1 = 32 - o0;
+          const int rt = o1 + 16 * (wave & 1), kt = o0 + 16 * (wave >> 1);
+          acc_t rx = acc_t{0, 0, 0, 0}, iy = rx, ix = rx, ry = rx;   // short chains, for their rounding errors too
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) {
+            const cT a = V[(rt + lr) * TR_VS + kt + 4 * ks + lk], x = *part(kt + 4 * ks + lk, lr, 0);
+            rx = MF<T>::mma(a.x, x.x, rx);
+            ry = MF<T>::mma(a.x, x.y, ry);
+            iy = MF<T>::mma(a.y, x.y, iy);
+            ix = MF<T>::mma(a.y, x.x, ix);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) *part(rt + MF<T>::row(lk, e), lr, 2 + (wave >> 1)) = cT{rx[e] - iy[e], ry[e] + ix[e]};
+        }
+        __syncthreads();
+        half(std::integral_constant<int, UPPER ? 0 : 1>{});
       }
       __syncthreads();
     }
