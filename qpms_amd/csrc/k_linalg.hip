@@ -13,8 +13,8 @@
 //                 announce themselves first, and where they do not all get onto
 //                 the device in time one of them does the strip alone;
 //   k_ts_*        the same with tournament pivoting, no workgroup waiting for
-//                 another: only for blocks beside the trailing update whose
-//                 strips have more workgroups than there are CUs left for them;
+//                 another: for strips of more workgroups than may wait for one
+//                 another (strip_most);
 //   k_swap_u      the strip's interchanges and U = L11^{-1} A12 in the rest of
 //                 its outer block, by substitution; k_u12 the block's U12 in the
 //                 columns beyond;
@@ -920,6 +920,9 @@ __device__ __noinline__ void st_alone(int m, int w, typename C2<T>::t *S, long l
   }
 }
 
+// Strips and slabs left to one workgroup so far (tests and probes read it).
+__device__ unsigned g_alone;
+
 // Everybody here? (one wave) Announces workgroup g with `tag` in the words `at`
 // and waits for the others; returns 1 (go on), 0 (leave) or -1 (do the strip
 // alone).
@@ -935,6 +938,7 @@ __device__ __forceinline__ int st_rendezvous(int g, int G, unsigned tag, st_u64 
   if (lane == 0 && __hip_atomic_compare_exchange_strong(state, &seen, stop ? ST_ALONE : ST_GO, __ATOMIC_RELAXED,
                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
     seen = stop ? -1 : ST_GO;
+  if (lane == 0 && seen == -1) atomicAdd(&g_alone, 1u);
   seen = __builtin_amdgcn_readfirstlane(seen);
   return seen == ST_ALONE ? 0 : seen;
 }
@@ -1917,12 +1921,20 @@ extern "C" void qh_lu_prepare(void) {
   qh_cgemm3m_prepare();
 }
 
-// Whether a factorisation may use the tournament for some of its blocks (see
-// getrf_batched): single matrices with strips of more workgroups than CUs are
-// kept free beside the trailing update.
+// Most workgroups of a strip that wait for one another: those of a quarter of the
+// device (64 CUs, two FP64 workgroups or one FP32 one each), as for the slabs of the
+// solves, so that of four hardware queues' launches one is always complete. Beside a
+// trailing update, as many as CUs are kept free of it. (Two strips that share those
+// end with the update: the side stream's next one waits for one of them.)
 template <class T>
-static bool may_tournament(int n, int batch, bool pp) {
-  return !pp && batch == 1 && use_lookahead() && st_groups<T>(n) > lu_reserve_cus();
+static int strip_most(bool beside) {
+  return beside ? lu_reserve_cus() : sizeof(T) == 8 ? 128 : 64;
+}
+// Whether a factorisation may use the tournament for some of its blocks (see
+// getrf_batched): single matrices with strips of more workgroups than that.
+template <class T>
+static bool may_tournament(int n, int batch, bool pp, int most) {
+  return !pp && batch == 1 && (st_groups<T>(n) > most || (use_lookahead() && st_groups<T>(n) > strip_most<T>(true)));
 }
 // Workspace of one matrix: the strips' words, the tournament's two candidate
 // buffers (the second holds the first merge level's output, a set per workgroup
@@ -1930,9 +1942,9 @@ static bool may_tournament(int n, int batch, bool pp) {
 template <class T>
 struct LuWS {
   size_t strip, buf_a, buf_b, fin, bytes;   // offsets, total
-  LuWS(int n, int batch, bool pp) {
+  LuWS(int n, int batch, bool pp, int most = strip_most<T>(false)) {
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t sets = may_tournament<T>(n, batch, pp) ? (size_t)PanelWS<T>::sets(n) : 0;
+    const size_t sets = may_tournament<T>(n, batch, pp, most) ? (size_t)PanelWS<T>::sets(n) : 0;
     strip = 0;
     buf_a = up((size_t)st_ws_bytes<T>(n));
     buf_b = buf_a + sets * PanelWS<T>::set_bytes();
@@ -1953,17 +1965,18 @@ static size_t getrf_ws_bytes(int n, int batch) {
 // -= L21 U12 (K = LU_NB).
 // ipiv (1-based, stride sP) lists the row interchanges as zgetrf's does;
 // perm (optional) tracks P; info[z] gets the first zero pivot. ws: the call's own
-// until its work is done, LuWS<T>(n, batch, pp).bytes per matrix.
+// until its work is done, LuWS<T>(n, batch, pp, most).bytes per matrix.
 template <class T>
 static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long sA, int *ipiv, long sP,
                           int *perm, int *dinfo, hipStream_t s, char *ws, bool lookahead = true,
-                          bool own_gemm = false, bool pp = false, st_u64 wait = ST_LIMIT) {
+                          bool own_gemm = false, bool pp = false, st_u64 wait = ST_LIMIT,
+                          int most = strip_most<T>(false)) {
   typedef typename C2<T>::t cT;
   constexpr int PW = PanelW<T>::W;
   const dim3 b256(256);
   if (n <= 0 || batch <= 0) return;
   if (n >= (1 << 22)) qpms_hip_die(__FILE__, __LINE__, __func__, "order %d above the pivot search's 2^22 rows", n);
-  const LuWS<T> lay(n, batch, pp);
+  const LuWS<T> lay(n, batch, pp, most);
   const long sW = (long)lay.bytes;
   const long setb = (long)PanelWS<T>::set_bytes();
   const dim3 bts(TS_THREADS);
@@ -1975,17 +1988,22 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
   // The strips of the outer block [k0, k0 + nb): pivots, interchanges on the
   // block's own columns, L21, then the block's remaining columns by TRSM and the
   // rank-w update. Touches only the block's columns (rows >= k0). wcu: beside a
-  // trailing update, as whole-CU workgroups; strips of more workgroups than CUs
-  // are free then go by tournament, whose workgroups do not wait for each other.
+  // trailing update, as whole-CU workgroups. Strips of more workgroups than
+  // strip_most go by tournament, whose workgroups do not wait for each other
+  // (single matrices, where the caller leaves the pivots to the library).
   auto block_strips = [&](int k0, int nb, hipStream_t st, bool wcu) {
     constexpr int F = ts_fan<T>();
-    const bool tour = wcu && st_groups<T>(n - k0) > lu_reserve_cus();
+    const bool tour = !pp && batch == 1 && st_groups<T>(n - k0) > (wcu ? strip_most<T>(true) : most);
     const WholeCu<T> &W = whole_cu<T>();
-    const size_t l_asg = W.gemm_assign, l_sub = W.gemm_sub;
+    const dim3 bcu(gcu_q<T>() * 256);
+    auto gcu_grid = [](int M, int N) {
+      const int nt = ((M + GT - 1) / GT) * ((N + GT - 1) / GT);
+      return dim3(std::min((nt + gcu_q<T>() - 1) / gcu_q<T>(), 4096));
+    };
     for (int j0 = 0; j0 < nb; j0 += PW) {
       const int w = min(PW, nb - j0), c0 = k0 + j0;
       char *fin = fin0 + (long)(j0 / PW) * finb;
-      const int rest = k0 + nb - (c0 + w);
+      const int rest = k0 + nb - (c0 + w), mr = n - c0 - w;
       if (!tour) {   // the strip factored in place (L21 included), its interchanges and U on the block's other columns
         QH_LAUNCH(k_strip<T>, dim3(st_groups<T>(n - c0), 1, batch), dim3(st_w<T>() * 64), wcu ? W.strip : 0, st, n, c0, w,
                   A, lda, sA, ws, sW, (long)(fin - ws), wait, ipiv, sP, dinfo);
@@ -2009,20 +2027,14 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
         if (nl + nu > 0)
           QH_LAUNCH(k_swap_u<T>, dim3(nl + nu), b256, W.swap_u, st, n, c0, w, A, lda, sA, fin, sW, k0, k0 + nb, nl,
                     (int *)nullptr, sP);
-      }
-      const int mr = n - c0 - w;
-      if (wcu) {   // single matrix, whole-CU launches (k_gemm_cu: several tiles per CU, K <= PW)
-        const dim3 bcu(gcu_q<T>() * 256);
-        auto gcu_grid = [](int M, int N) {
-          const int nt = ((M + GT - 1) / GT) * ((N + GT - 1) / GT);
-          return dim3(std::min((nt + gcu_q<T>() - 1) / gcu_q<T>(), 4096));
-        };
-        if (mr > 0 && tour)   // L21 = A21 U11^{-1}
-          QH_LAUNCH((k_gemm_cu<T, true>), gcu_grid(mr, w), bcu, l_asg, st, mr, w, w, A + (long)(c0 + w) * lda + c0,
-                    lda, reinterpret_cast<const cT *>(fin + PanelWS<T>::UINV_OFF), (long)PW,
+        if (mr > 0)   // L21 = A21 U11^{-1}
+          QH_LAUNCH((k_gemm_cu<T, true>), gcu_grid(mr, w), bcu, W.gemm_assign, st, mr, w, w,
+                    A + (long)(c0 + w) * lda + c0, lda, reinterpret_cast<const cT *>(fin + PanelWS<T>::UINV_OFF), (long)PW,
                     A + (long)(c0 + w) * lda + c0, lda);
+      }
+      if (wcu) {   // single matrix, whole-CU launches (k_gemm_cu: several tiles per CU, K <= PW)
         if (rest > 0 && mr > 0)   // the block's next columns: A22 -= L21 U
-          QH_LAUNCH((k_gemm_cu<T, false>), gcu_grid(mr, rest), bcu, l_sub, st, mr, rest, w,
+          QH_LAUNCH((k_gemm_cu<T, false>), gcu_grid(mr, rest), bcu, W.gemm_sub, st, mr, rest, w,
                     A + (long)(c0 + w) * lda + c0, lda, A + (long)c0 * lda + c0 + w, lda,
                     A + (long)(c0 + w) * lda + c0 + w, lda);
         continue;
@@ -2064,7 +2076,7 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
       // A strip's workgroups wait for each other, so each needs one of the CUs kept
       // free for it: beside the update on a shared CU the slowest held all of them up
       // (order 9216: 1.8 ms for the first strip of a block, 0.1 ms alone).
-      const bool split = la && nr > nb1 && !(pp && st_groups<T>(nr) > lu_reserve_cus());
+      const bool split = la && nr > nb1 && !(pp && st_groups<T>(nr) > strip_most<T>(true));
       if (nr > nb1) {
         hipStream_t sg = split ? side : s;
         if (split) {
@@ -2111,7 +2123,7 @@ static void getrf_batched(int n, int batch, typename C2<T>::t *A, long lda, long
 // them takes all blocks and the others leave.
 // ---------------------------------------------------------------------------
 constexpr int TR_B = 64, TR_C = 16, TR_VS = TR_B + 1, TR_XS = TR_C + 1;
-constexpr int TR_MEET = 256;   // most workgroups of a slab
+constexpr int TR_MEET = 128;   // most workgroups of a slab
 template <class T> constexpr size_t tr_lds() {   // the diagonal block without its diagonal, the waves' sums, the diagonal
   return (size_t)(TR_B * TR_VS + 4 * TR_B * TR_XS + TR_B) * sizeof(typename C2<T>::t);
 }
@@ -2557,16 +2569,15 @@ static void getrs_batched(int n, int nrhs, int batch, const typename C2<T>::t *L
   const int nblk = (n + TR_B - 1) / TR_B, nslab = (nrhs + TR_C - 1) / TR_C;
   const long slabb = (long)((tr_slab_bytes<T>(n, nrhs) + 255) / 256 * 256), sW = slabb * nslab;
   qh_zero(ws, (size_t)batch * sW, s);
-  // One slab: a workgroup's next block, up to nblk products of 64 x 64 blocks (2 us
-  // each), has to be ready when the chain (4 to 7 us a block) gets there: nblk / 4
-  // of them keep up. Several slabs or matrices share what the device holds (256 in
-  // FP64, 512 in FP32), more of them take turns: a 16-matrix batch of order 9216
-  // with 64 right-hand sides (FP32) takes 23 ms with two workgroups per slab, 12 with
-  // eight. A slab gets no more than a quarter of the device, so that of the slabs
-  // of four streams one is always complete and the others wait for its end only.
+  // A workgroup's next block, up to nblk products of 64 x 64 blocks (2 us each), has to
+  // be ready when the chain (5 to 14 us a block) gets there: nblk / 4 of them keep up
+  // with one slab. A slab gets no more than a quarter of the device (which holds 256
+  // workgroups in FP64, 512 in FP32), so that of the slabs of four hardware queues one
+  // is always complete and the others wait for its end only. Several slabs or matrices
+  // share the device, more of them take turns: a 16-matrix batch of order 9216 with 64
+  // right-hand sides (FP32) takes 23 ms with two workgroups per slab, 12 with eight.
   const long quarter = sizeof(T) == 8 ? 64 : 128, slabs = (long)nslab * batch;
-  const int G = (int)std::max(1L, std::min({(long)nblk, (long)TR_MEET, slabs == 1 ? std::max(quarter, (long)nblk / 4)
-                                                                                  : std::min(quarter, 4 * quarter / slabs)}));
+  const int G = (int)std::max(1L, std::min({(long)nblk, (long)TR_MEET, quarter, 4 * quarter / slabs}));
   QH_LAUNCH(k_tri<T>, dim3(G, nslab, batch), dim3(256), tr_lds<T>(), s, n, nrhs, LU, lda, sA, perm, sP, B, ldb, sB,
             (char *)ws, sW, slabb, wait);
   HIPCHK(hipGetLastError());
@@ -2598,6 +2609,21 @@ extern "C" int qh_getrf_pp(int prec, int n, double *A, int *ipiv, int *info, uns
     getrf_batched<float>(n, 1, (v2f *)A, n, 0, ipiv, 0, nullptr, info, s, ws, true, false, true, wait);
   else
     getrf_batched<double>(n, 1, (v2d *)A, n, 0, ipiv, 0, nullptr, info, s, ws, true, false, true, wait);
+  return 0;
+}
+
+// The LU of one matrix with the tournament for strips of more than `most`
+// workgroups, no lookahead; waits. Tests reach it at small orders.
+extern "C" int qh_getrf_most(int prec, int n, double *A, int *ipiv, int *perm, int *info, int most, void *stream) {
+  hipStream_t s = (hipStream_t)qh_stream(stream);
+  qh_zero(info, sizeof(int), s);
+  char *ws = (char *)qh_dmalloc(prec == 32 ? LuWS<float>(n, 1, false, most).bytes : LuWS<double>(n, 1, false, most).bytes);
+  if (prec == 32)
+    getrf_batched<float>(n, 1, (v2f *)A, n, 0, ipiv, n, perm, info, s, ws, false, false, false, ST_LIMIT, most);
+  else
+    getrf_batched<double>(n, 1, (v2d *)A, n, 0, ipiv, n, perm, info, s, ws, false, false, false, ST_LIMIT, most);
+  HIPCHK(hipStreamSynchronize(s));
+  qh_dfree(ws);
   return 0;
 }
 
@@ -2809,6 +2835,13 @@ extern "C" int qh_getrf_batched_wsla_f64(int n, int batch, double *A, long sA, i
   getrf_batched<double>(n, batch, (v2d *)A, n, sA, ipiv, n, perm, info, (hipStream_t)qh_stream(stream), (char *)ws,
                         lookahead != 0);
   return 0;
+}
+// Strips of factorisations and slabs of solves that one workgroup had to do alone,
+// since the library was loaded (waits for the device).
+extern "C" unsigned qh_alone_count(void) {
+  unsigned n = 0;
+  HIPCHK(hipMemcpyFromSymbol(&n, HIP_SYMBOL(g_alone), sizeof n));
+  return n;
 }
 // Solves with batched factorisations. The workspace form neither allocates nor
 // waits.

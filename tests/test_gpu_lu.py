@@ -163,3 +163,26 @@ def test_getrs_batched_many_rhs(gpu, prec, n, nrhs, batch):
     for z in range(batch):
         ref = np.linalg.solve(As[z].astype(np.complex128), Bs[z].astype(np.complex128))
         assert np.max(np.abs(X[z] - ref)) / np.max(np.abs(ref)) < tol
+
+
+@pytest.mark.parametrize("prec", ["f32", "f64"])
+@pytest.mark.parametrize("n, most", [(33, 0), (300, 0), (777, 0), (1300, 1)])
+def test_strips_by_tournament(gpu, prec, n, most):
+    """Strips of more workgroups than may wait for one another, not beside a trailing
+    update (with orders above 32768 in earnest): pivots by tournament in the first
+    blocks, by k_strip in the last."""
+    import qpms_amd
+    L = qpms_amd.lib()
+    dt = np.complex64 if prec == "f32" else np.complex128
+    A = rand(n, n).astype(dt)
+    dA, di = qpms_amd.DeviceBuffer.from_array(A), qpms_amd.DeviceBuffer(4)
+    dp, dq = qpms_amd.DeviceBuffer(4 * n), qpms_amd.DeviceBuffer(4 * n)
+    L.qh_getrf_most.argtypes = [ctypes.c_int, ctypes.c_int] + [ctypes.c_void_p] * 4 + [ctypes.c_int, ctypes.c_void_p]
+    L.qh_getrf_most(32 if prec == "f32" else 64, n, dA.ptr, dp.ptr, dq.ptr, di.ptr, most, None)
+    piv = dp.to_array(np.int32, (n,))
+    assert di.to_array(np.int32, (1,))[0] == 0
+    check_plu(A.astype(complex), dA.to_array(dt, (n, n)).astype(complex), piv, 1e-5 if prec == "f32" else 1e-13)
+    p = np.arange(n)
+    for i in range(n):
+        p[[i, piv[i] - 1]] = p[[piv[i] - 1, i]]
+    assert np.array_equal(dq.to_array(np.int32, (n,)), p)

@@ -48,3 +48,51 @@ def test_calls_of_several_threads(gpu, entry):
     for s in streams:
         L.qh_stream_release(s)
         assert L.hipStreamDestroy(s) == 0
+
+
+def test_waiting_launches_of_several_streams(gpu):
+    """Four streams at once, strips of 12 and 20 workgroups and solves with as many as
+    a slab may have: none is left to one workgroup, and every result is the one of the
+    call alone."""
+    import qpms_amd
+    L, vp, up = qpms_amd.lib(), ctypes.c_void_p, qpms_amd.DeviceBuffer.from_array
+    L.qh_getrf_ws_bytes.restype = L.qh_getrs_ws_bytes.restype = ctypes.c_size_t
+
+    def call(n, s, out, reps):
+        rng = np.random.default_rng(n)
+        A = rng.standard_normal((n, n), np.float32) + 1j * rng.standard_normal((n, n), np.float32)
+        A = A.astype(complex)
+        A[range(n), range(n)] += 3 * np.sqrt(n)
+        dp, dq, di = qpms_amd.DeviceBuffer(4 * n), qpms_amd.DeviceBuffer(4 * n), up(np.zeros(1, np.int32))
+        ws = qpms_amd.DeviceBuffer(max(L.qh_getrf_ws_bytes(64, n, 1), L.qh_getrs_ws_bytes(64, n, 1, 1)))
+        for _ in range(reps):
+            dA, dB = up(A), up(A[:, :1].copy())
+            i = ctypes.c_int
+            L.qh_getrf_batched_wsla_f64(i(n), i(1), vp(dA.ptr), ctypes.c_long(0), vp(dp.ptr), vp(dq.ptr), vp(di.ptr),
+                                        vp(ws.ptr), i(1), s)
+            for _ in range(20):
+                L.qh_getrs_ws_f64(i(n), i(1), i(1), vp(dA.ptr), ctypes.c_long(0), vp(dq.ptr), vp(dB.ptr),
+                                  ctypes.c_long(0), vp(ws.ptr), s)
+            assert L.hipStreamSynchronize(s) == 0
+            out.append(dB.to_array(complex, (n, 1)).tobytes())
+
+    orders = [3000, 5000, 3000, 5000]
+    streams = [ctypes.c_void_p() for _ in orders]
+    for s in streams:
+        assert L.hipStreamCreateWithFlags(ctypes.byref(s), ctypes.c_uint(1)) == 0
+    alone, together = [[] for _ in orders], [[] for _ in orders]
+    for n, s, o in zip(orders[:2], streams, alone):
+        call(n, s, o, 1)
+    before = L.qh_alone_count()
+    threads = [threading.Thread(target=call, args=(n, s, o, 3)) for n, s, o in zip(orders, streams, together)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert L.qh_alone_count() == before
+    for k, o in enumerate(together):
+        assert len(o) == 3 and set(o) == set(alone[k % 2])
+    L.qh_stream_release.argtypes = [ctypes.c_void_p]
+    for s in streams:
+        L.qh_stream_release(s)
+        assert L.hipStreamDestroy(s) == 0
