@@ -824,6 +824,15 @@ extern "C" int qh_launch_sigma_both(int LE, int ntrip, const double *tr_dev, int
   if (ntrip <= 0) return 0;
   hipStream_t s = (hipStream_t)qh_stream(stream);
   ensure_weid();
+  // a dispatch takes fewer than 2^26 waves, two for a triple
+  constexpr int MOST = 1 << 24;
+  if (ntrip > MOST) {
+    const size_t nsc2 = 2 * (size_t)(LE + 1) * (LE + 1);
+    for (int t = 0; t < ntrip; t += std::min(MOST, ntrip - t))
+      qh_launch_sigma_both(LE, std::min(MOST, ntrip - t), tr_dev + 8 * (size_t)t, nR, R_dev, nK, K_dev, eta, area,
+                           leg0_dev, csphase, short_dev + nsc2 * t, long_dev + nsc2 * t, stream);
+    return 0;
+  }
   const dim3 g(2 * (unsigned)ntrip), b = triple_threads(LE, true, 2L * ntrip);
 #define QH_SB1(L, K) QH_LAUNCH((k_sigma_both<L, K>), g, b, 0, s, ntrip, tr_dev, nR, R_dev, nK, K_dev, eta, area, \
       leg0_dev, csphase, (v2d *)short_dev, (v2d *)long_dev)

@@ -104,3 +104,23 @@ def test_shifts_against_single(gpu, LE, n, nK):
     some = sorted({0, n // 2, n - 1})
     close(got[some], np.vstack([batch(L, e3c, LE, t[i:i + 1], R, K, "long")[1] for i in some]), LE)
     L.qpms_ewald3_constants_free(e3c)
+
+
+def test_more_triples_than_one_dispatch_takes(gpu):
+    """2^25 + 3 triples in one call: the first, the last and those around 2^24."""
+    import qpms_amd
+    L, R, K = points(1, 1)
+    e3c = L.qpms_ewald3_constants_init(3, -1)
+    few, n, nsc = triples(1003, np.random.default_rng(1)), (1 << 25) + 3, 16
+    up = qpms_amd.DeviceBuffer.from_array
+    dt, dR, dK = up(np.resize(few, (n, 8))), up(R), up(K)
+    ds, dl = qpms_amd.DeviceBuffer(16 * nsc * n), qpms_amd.DeviceBuffer(16 * nsc * n)
+    L.qpms_hip_ewald3_sigma_batch_dev(e3c, ec.ETA, ec.AREA, n, dt.ptr, 1, dR.ptr, 1, dK.ptr, ds.ptr, dl.ptr, None)
+    L.qpms_hip_sync()
+    ss, sl = batch(L, e3c, 3, few, R, K)
+    got = np.empty((2, nsc), complex)
+    for t in (0, (1 << 24) - 2, 1 << 24, (1 << 25) - 1, n - 2):
+        for d, ref in ((ds, ss), (dl, sl)):
+            L.qpms_hip_memcpy_d2h(got.ctypes.data, d.ptr + 16 * nsc * t, got.nbytes)
+            close(got, ref[[t % 1003, (t + 1) % 1003]], 3)
+    L.qpms_ewald3_constants_free(e3c)
