@@ -2130,7 +2130,9 @@ template <class T> constexpr size_t tr_lds() {   // the diagonal block without i
 template <class T> constexpr size_t tr_slab_bytes(int n, int nrhs) {
   return 256 + TR_MEET * 8 + (size_t)((n + TR_B - 1) / TR_B) * TR_B * (nrhs < TR_C ? nrhs : TR_C) * st_ew<T>() * 8;
 }
+constexpr int TR_MOST = 64 * TR_C;   // most right-hand sides of a launch (a grid's rows, and the words' memory)
 template <class T> constexpr size_t tr_ws_bytes(int n, int nrhs) {
+  if (nrhs > TR_MOST) nrhs = TR_MOST;
   return (size_t)((nrhs + TR_C - 1) / TR_C) * ((tr_slab_bytes<T>(n, nrhs) + 255) / 256 * 256);
 }
 
@@ -2565,6 +2567,11 @@ static void getrs_batched(int n, int nrhs, int batch, const typename C2<T>::t *L
                           const int *perm, long sP, typename C2<T>::t *B, long ldb, long sB, void *ws, hipStream_t s,
                           st_u64 wait = ST_LIMIT) {
   if (n <= 0 || nrhs <= 0 || batch <= 0) return;
+  if (nrhs > TR_MOST) {   // in turns
+    for (int j = 0; j < nrhs; j += std::min(TR_MOST, nrhs - j))
+      getrs_batched<T>(n, std::min(TR_MOST, nrhs - j), batch, LU, lda, sA, perm, sP, B + j, ldb, sB, ws, s, wait);
+    return;
+  }
   tr_prepare<T>();
   const int nblk = (n + TR_B - 1) / TR_B, nslab = (nrhs + TR_C - 1) / TR_C;
   const long slabb = (long)((tr_slab_bytes<T>(n, nrhs) + 255) / 256 * 256), sW = slabb * nslab;

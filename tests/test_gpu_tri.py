@@ -55,3 +55,26 @@ def test_rows_by_pivots(gpu, n):
     dA, dp, dB = [qpms_amd.DeviceBuffer.from_array(v) for v in (np.eye(n, dtype=complex), ipiv, B.astype(complex))]
     L.qpms_hip_zgetrs_dev(ctypes.c_size_t(n), ctypes.c_size_t(2), dA.ptr, dp.ptr, dB.ptr, None)
     assert np.array_equal(dB.to_array(np.complex128, (n, 2)), want)
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("n, nrhs", [(70, 1024), (70, 1025), (200, 3000), (3, 1100000)])
+def test_more_columns_than_one_launch_takes(gpu, prec, n, nrhs):
+    """Every column is the one of a solve of its own, to rounding (condition below 10);
+    the words' memory does not grow with the columns."""
+    import qpms_amd
+    L = qpms_amd.lib()
+    dt, eps = (np.complex128, 2.3e-16) if prec == 64 else (np.complex64, 1.2e-7)
+    rng = np.random.default_rng(n)
+    LU = (rng.uniform(-1, 1, (n, n)) + 1j * rng.uniform(-1, 1, (n, n))) / (2 * np.sqrt(n))
+    LU[range(n), range(n)] = rng.uniform(1, 2, n)
+    B = rng.normal(size=(n, nrhs)) + 1j * rng.normal(size=(n, nrhs))
+    dA, dB, dp = [qpms_amd.DeviceBuffer.from_array(v)
+                  for v in (LU.astype(dt), B.astype(dt), np.arange(n, dtype=np.int32))]
+    L.qh_getrs_wait.argtypes = [ctypes.c_int] * 4 + [ctypes.c_void_p] * 3 + [ctypes.c_ulonglong, ctypes.c_void_p]
+    L.qh_getrs_wait(prec, n, nrhs, 1, dA.ptr, dp.ptr, dB.ptr, 10 ** 7, None)
+    X = dB.to_array(dt, (n, nrhs))
+    x = scipy.linalg.solve_triangular(LU, scipy.linalg.solve_triangular(LU, B, lower=True, unit_diagonal=True))
+    assert np.max(np.abs(X - x)) < 64 * np.sqrt(n) * eps * np.max(np.abs(x))
+    L.qh_getrs_ws_bytes.restype = ctypes.c_size_t
+    assert L.qh_getrs_ws_bytes(prec, n, nrhs, 1) == L.qh_getrs_ws_bytes(prec, n, min(nrhs, 1024), 1)
