@@ -122,3 +122,21 @@ def test_points_at_infinity(gpu, n):
         for i in (0, n - 1):
             close(a[i], b[i], LE)
     L.qpms_ewald3_constants_free(e3c)
+
+
+@pytest.mark.parametrize("n", [1, 2, 29, 58, 1001, 344, 2 ** 20 + 1, 3 * 10 ** 8])
+def test_phase_next_to_multiples_of_half_pi(gpu, n):
+    """One K point: the sum's lowest coefficient is i e^{i K s} times a real number.
+    Both parts of the phase to a few units in the last place of their own."""
+    import qpms_amd
+    L, LE = ec.lib_ewald(), 3
+    e3c = L.qpms_ewald3_constants_init(LE, -1)
+    nsc, up = (LE + 1) ** 2, qpms_amd.DeviceBuffer.from_array
+    x = n * (math.pi / 2)
+    dt, dK, sl = up(np.array([[0, 0, 0, x / 10, 0, 1.0, 0, 0]])), up(np.array([[x, 0.0]])), up(np.zeros(nsc, complex))
+    L.qpms_hip_ewald3_sigma_batch_dev(e3c, x / 4, 1.0, 1, dt.ptr, 0, dK.ptr, 1, dK.ptr, None, sl.ptr, None)
+    L.qpms_hip_sync()
+    v = sl.to_array(complex, (nsc,))[0] / 1j
+    v /= np.copysign(abs(v), v.real * math.cos(x))
+    assert abs(v.real / math.cos(x) - 1) < 2e-15 and abs(v.imag / math.sin(x) - 1) < 2e-15
+    L.qpms_ewald3_constants_free(e3c)
