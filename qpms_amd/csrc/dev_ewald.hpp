@@ -28,6 +28,7 @@
 namespace qew {
 
 constexpr int WEID_N = 32;
+constexpr int WEID_GN = 40;   // of the incomplete Gamma functions' expansions
 
 // exp, sin and cos, and a reciprocal, for loops whose registers are sums: the
 // library's keep their polynomials' coefficients in vector registers over the loop
@@ -285,27 +286,37 @@ __device__ __forceinline__ void gamma_inc_half_real_series(cplx z, cplx (&G)[J +
 #endif
 
 #if defined(__HIPCC__)
-// Gamma(1/2 - j, z), j = 0..J, for Re z > 0.5 (principal branch): gamma_half_scaled
-// with w(i sqrt z) for complex z. The continued fraction takes 100-340 dependent
+// Gamma(1/2 - j, z), j = 0..J (J >= 1), for Re z > 0.5 (principal branch). With s = sqrt z
+//   e^z Gamma(1/2 - J, z) = s^{1 - 2J} / Gamma(J + 1/2) int e^{-t^2} t^{2J} / (s^2 + t^2) dt
+// is w(i s) with t^{2J} beside the weight e^{-t^2}, hence Weideman's expansion with
+// coefficients a of that weight, and the lower j follow by the recurrence in the
+// direction that keeps relative errors: all within 10 units in the last place for
+// 0.5 < Re z, |Im z| < 160. The other direction, from w(i s) itself, loses a factor |z|
+// a step (1e-9 at |z| = 300, j = 3). The continued fraction takes 100-340 dependent
 // steps of two complex divisions near |z| = 1, for each j.
 template <int J>
 __device__ __forceinline__ void gamma_half_complex(cplx z, const double *a, cplx (&G)[J + 1]) {
-  const double L = 4.7568284600108841;  // sqrt(32 / sqrt(2))
+  const double L = 5.3182958969449885;  // sqrt(40 / sqrt(2))
   const cplx s = csqrt_(z), den = mk(L + s.re, s.im);
   const cplx inv = conj(den) * rcp_(cabs2(den)), Z = mk(L - s.re, -s.im) * inv;
-  cplx p = mk(a[WEID_N - 1], 0.0);
+  cplx p = mk(a[WEID_GN - 1], 0.0);
 #pragma unroll
-  for (int m = WEID_N - 2; m >= 0; --m)
+  for (int m = WEID_GN - 2; m >= 0; --m)
     p = mk(fma(p.re, Z.re, fma(-p.im, Z.im, a[m])), fma(p.re, Z.im, p.im * Z.re));
-  cplx E = 1.7724538509055160273 * (inv * (2.0 * (p * inv) + mk(0.56418958354775628695, 0.0)));
+  cplx E = inv * (2.0 * (p * inv) + mk(1.0, 0.0));
   const cplx ez = exp_(-z.re) * expi_(-z.im), zi = cinv(z);
-  cplx za = s;   // z^{1/2 - j + 1} at step j
-  G[0] = E * ez;
+  cplx za[J + 1];   // z^{1/2 - j}
+  za[0] = s;
 #pragma unroll
   for (int j = 1; j <= J; ++j) {
-    za = za * zi;
-    E = (E - za) * (1.0 / (0.5 - j));
-    G[j] = E * ez;
+    za[j] = za[j - 1] * zi;
+    E = E * zi;
+  }
+  G[J] = E * ez;
+#pragma unroll
+  for (int j = J; j >= 1; --j) {
+    E = za[j] + (0.5 - j) * E;
+    G[j - 1] = E * ez;
   }
 }
 #endif

@@ -31,6 +31,7 @@ typedef double v2d __attribute__((ext_vector_type(2)));
   qpms_hip_die(__FILE__, __LINE__, __func__, "HIP error %d (%s) in %s", (int)e_, hipGetErrorString(e_), #x); } while (0)
 
 __constant__ double c_weid[qew::WEID_N];
+__constant__ double c_weid_gamma[4][qew::WEID_GN];   // of Gamma(1/2 - J, z), J = 1..4
 
 namespace {
 
@@ -100,6 +101,14 @@ template <int LE, bool SMALL = true> constexpr int ew_waves() { return SMALL && 
 // loop they would take 64 registers.
 __device__ __forceinline__ const double *weid() {
   const double *a = c_weid;
+  asm volatile("" : "+s"(a));
+  return a;
+}
+
+template <int J>
+__device__ __forceinline__ const double *weid_gamma() {
+  static_assert(J >= 1 && J <= 4, "expansions for J = 1..4");
+  const double *a = c_weid_gamma[J - 1];
   asm volatile("" : "+s"(a));
   return a;
 }
@@ -435,7 +444,7 @@ __device__ __forceinline__ bool long_general(double rb, cplx k, double eta, cplx
   if constexpr (kreal) {   // z <= 0.5, or NaN
     qew::gamma_inc_half_real_series<JM>(z, G);
   } else if (z.re > 0.5 && branch == 0) {
-    qew::gamma_half_complex<JM>(z, weid(), G);
+    qew::gamma_half_complex<JM>(z, weid_gamma<JM>(), G);
   } else {
 #pragma unroll
     for (int j = 0; j <= JM; ++j) G[j] = qew::gamma_inc_half(j, z, branch);
@@ -728,36 +737,42 @@ __global__ void k_sigma_total(int ntrip, int nsc, const v2d *__restrict__ ss, co
 
 // ---------------------------------------------------------------------------
 // Weideman coefficients (host): a_m, m = 1..N, of Weideman's eq. (3.6), from
-// the discrete Fourier sum over t_k = L tan(theta_k / 2), theta_k = k pi / M.
+// the discrete Fourier sum over t_k = L tan(theta_k / 2), theta_k = k pi / M,
+// with t^{2J} beside the weight e^{-t^2}: those of w (J = 0), or times
+// pi / Gamma(J + 1/2) those of gamma_half_complex.
 // ---------------------------------------------------------------------------
-static void weideman_coefficients(double *a) {
-  const int N = qew::WEID_N, M = 2 * N, M2 = 2 * M;
-  const double L = sqrt(N / sqrt(2.0));
-  double f[2 * 2 * qew::WEID_N];
-  f[0] = 0.0;
-  for (int k = -M + 1; k <= M - 1; ++k) {
-    const double th = k * M_PI / M, tt = L * tan(th / 2);
-    f[k + M] = exp(-tt * tt) * (L * L + tt * tt);
+static void weideman_coefficients(int N, int J, double *a) {
+  const int M = 2 * N, M2 = 2 * M;
+  const long double pi = 3.14159265358979323846264338327950288L, L = sqrtl(N / sqrtl(2.0L));
+  long double f[4 * 64], scale = 1.0L;
+  if (J > 0) {
+    scale = sqrtl(pi);
+    for (int j = 0; j < J; ++j) scale /= j + 0.5L;
   }
-  double g[2 * 2 * qew::WEID_N];
-  for (int i = 0; i < M2; ++i) g[i] = f[(i + M) % M2];  // fftshift
+  f[0] = 0.0L;
+  for (int k = -M + 1; k <= M - 1; ++k) {
+    const long double tt = L * tanl(k * pi / M / 2);
+    f[k + M] = expl(-tt * tt) * powl(tt * tt, J) * (L * L + tt * tt);
+  }
   for (int m = 1; m <= N; ++m) {
     long double s = 0;
-    for (int i = 0; i < M2; ++i) s += (long double)g[i] * cosl(2.0L * M_PI * (long double)i * m / M2);
-    a[m - 1] = (double)(s / M2);
+    for (int i = 0; i < M2; ++i) s += f[(i + M) % M2] * cosl(2.0L * pi * (long double)i * m / M2);   // fftshift
+    a[m - 1] = (double)(scale * s / M2);
   }
 }
 
 static std::once_flag g_weid_once;
 static void ensure_weid() {
   std::call_once(g_weid_once, [] {
-    double a[qew::WEID_N];
-    weideman_coefficients(a);
+    double a[qew::WEID_N], g[4][qew::WEID_GN];
+    weideman_coefficients(qew::WEID_N, 0, a);
+    for (int J = 1; J <= 4; ++J) weideman_coefficients(qew::WEID_GN, J, g[J - 1]);
     HIPCHK(hipMemcpyToSymbol(HIP_SYMBOL(c_weid), a, sizeof a, 0, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpyToSymbol(HIP_SYMBOL(c_weid_gamma), g, sizeof g, 0, hipMemcpyHostToDevice));
   });
 }
 
-extern "C" void qh_weideman_coefficients(double *a) { weideman_coefficients(a); }
+extern "C" void qh_weideman_coefficients(double *a) { weideman_coefficients(qew::WEID_N, 0, a); }
 
 // Waves per triple: as many as the launch leaves wavefront slots for (2048 of these
 // kernels fit on the chip), so that a few triples don't wait for one wave's walk
