@@ -69,11 +69,7 @@ template <class T> __device__ __forceinline__ typename C2<T>::t cdiv(typename C2
 
 
 // ---------------------------------------------------------------------------
-// C[M x N] -= A[M x K] * B[K x N] (complex, row-major), MFMA; with ASSIGN,
-// C = A B. Every workgroup reads its whole K extent before it writes its C
-// tile, so C may be A (N <= 64: one column tile) or B (M <= 64: one row
-// tile), which the strip updates use to apply 32 x 32 triangular inverses in
-// place.
+// C[M x N] -= A[M x K] * B[K x N] (complex, row-major), MFMA.
 // Block: 256 threads = 4 waves, C tile 64 x 64, each wave a 32 x 32 quadrant
 // made of 2 x 2 MFMA 16x16 tiles, K step 16 (= 4 MFMA k-steps of 4).
 // LDS tiles are de-interleaved: Ar, Ai [64][16+1], Br, Bi [16][64+1].
@@ -103,7 +99,7 @@ template <> struct MF<float> {
 
 constexpr int GT = 64, GK = 16;
 
-template <class T, bool ASSIGN = false>
+template <class T>
 __global__ __launch_bounds__(256) void k_gemm_sub(int M, int N, int K, const typename C2<T>::t *A, long lda, long sA,
                                                   const typename C2<T>::t *B, long ldb, long sB,
                                                   typename C2<T>::t *C, long ldc, long sC) {
@@ -167,14 +163,10 @@ __global__ __launch_bounds__(256) void k_gemm_sub(int M, int N, int K, const typ
       for (int i = 0; i < 4; ++i) {
         const int row = m0 + wm + a * 16 + MF<T>::row(lk, i), col = n0 + wn + b * 16 + lr;
         if (row < M && col < N) {
-          if (ASSIGN) {
-            C[(long)row * ldc + col] = cT{pr[a][b][i], pi[a][b][i]};
-          } else {
-            cT c = C[(long)row * ldc + col];
-            c.x -= pr[a][b][i];
-            c.y -= pi[a][b][i];
-            C[(long)row * ldc + col] = c;
-          }
+          cT c = C[(long)row * ldc + col];
+          c.x -= pr[a][b][i];
+          c.y -= pi[a][b][i];
+          C[(long)row * ldc + col] = c;
         }
       }
   }
@@ -1765,9 +1757,9 @@ static bool use_lookahead() {
   return v == 1;
 }
 
-// C -= A B (or C = A B, ASSIGN) for K <= PW: the strip's products (L21 =
-// A21 U11^{-1}, U = L11^{-1} A12, the in-block rank-PW update) when they run
-// as whole-CU workgroups beside the trailing update (one workgroup per CU).
+// C -= A B (or C = A B, ASSIGN) for K <= PW: the products of strips (the
+// in-block rank-PW update, L21 = A21 U11^{-1} after a tournament) that run as
+// whole-CU workgroups, beside the trailing update (one workgroup per CU).
 // The workgroup is gcu_q quarters of 256 threads, each quarter on its own
 // 64 x 64 tile of C, so that a CU has that many tiles in flight; a tile's A
 // (64 x K) and B (K x 64) are staged whole (one load round trip for the
