@@ -56,6 +56,10 @@ template <> struct C2<float> { typedef v2f t; };
 template <class T> __device__ __forceinline__ typename C2<T>::t cmul(typename C2<T>::t a, typename C2<T>::t b) {
   return typename C2<T>::t{a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
 }
+// y - a b with one rounding of y's size (as two chained FMAs a part it is two)
+template <class T> __device__ __forceinline__ typename C2<T>::t cless(typename C2<T>::t y, typename C2<T>::t a, typename C2<T>::t b) {
+  return typename C2<T>::t{y.x - fma(a.x, b.x, -a.y * b.y), y.y - fma(a.x, b.y, a.y * b.x)};
+}
 template <class T> __device__ __forceinline__ typename C2<T>::t cdiv(typename C2<T>::t a, typename C2<T>::t b) {
   // Smith's algorithm
   if (fabs(b.x) >= fabs(b.y)) {
@@ -904,7 +908,7 @@ __device__ __noinline__ void st_alone(int m, int w, typename C2<T>::t *S, long l
         S[(long)i * lda + j] = l;
         for (int c = j + 1; c < w; ++c) {
           const cT u = S[(long)j * lda + c], y = S[(long)i * lda + c];
-          S[(long)i * lda + c] = cT{fma(-l.x, u.x, fma(l.y, u.y, y.x)), fma(-l.x, u.y, fma(-l.y, u.x, y.y))};
+          S[(long)i * lda + c] = cless<T>(y, l, u);
         }
       }
     }
@@ -1158,9 +1162,9 @@ __global__ __launch_bounds__(st_w<T>() * 64, 2) void k_strip(int n, int c0, int 
       const cT l = cmul<T>(cT{a0, b0}, rcp);
 #pragma unroll
       for (int c = 1; c < 4; ++c) {
-        const T fa = fma(-l.x, P[c].x, fma(l.y, P[c].y, ya[c])), fb = fma(-l.x, P[c].y, fma(-l.y, P[c].x, yb[c]));
-        ya[c - 1] = (e && c < open) ? fa : ya[c];
-        yb[c - 1] = (e && c < open) ? fb : yb[c];
+        const cT f = cless<T>(cT{ya[c], yb[c]}, l, P[c]);
+        ya[c - 1] = (e && c < open) ? f.x : ya[c];
+        yb[c - 1] = (e && c < open) ? f.y : yb[c];
       }
       ya[3] = e ? l.x : a0;
       yb[3] = e ? l.y : b0;
@@ -1214,12 +1218,9 @@ __global__ __launch_bounds__(st_w<T>() * 64, 2) void k_strip(int n, int c0, int 
           cT u[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) u[r] = sh.urow[r][4 * (4 * ct + oq) + oc];
-          auto sub = [](cT a, cT l, cT b) {
-            return cT{fma(-l.x, b.x, fma(l.y, b.y, a.x)), fma(-l.x, b.y, fma(-l.y, b.x, a.y))};
-          };
-          u[1] = sub(u[1], L[0], u[0]);
-          u[2] = sub(sub(u[2], L[1], u[0]), L[3], u[1]);
-          u[3] = sub(sub(sub(u[3], L[2], u[0]), L[4], u[1]), L[5], u[2]);
+          u[1] = cless<T>(u[1], L[0], u[0]);
+          u[2] = cless<T>(cless<T>(u[2], L[1], u[0]), L[3], u[1]);
+          u[3] = cless<T>(cless<T>(cless<T>(u[3], L[2], u[0]), L[4], u[1]), L[5], u[2]);
           const bool use = 4 * ct + oq > 0 && i + 4 * ct + oq < 8 && sh.nz[4 * i + cq];   // an open column
           ur[ct] = use ? st_own4(cq, u[0].x, u[1].x, u[2].x, u[3].x) : T(0);
           ui[ct] = use ? st_own4(cq, u[0].y, u[1].y, u[2].y, u[3].y) : T(0);
@@ -1258,14 +1259,15 @@ __global__ __launch_bounds__(st_w<T>() * 64, 2) void k_strip(int n, int c0, int 
         for (int ct = 0; ct < 2; ++ct) {
           if (ct == 1 && i >= 4) continue;   // finished columns (uniform)
 #pragma unroll
-          for (int T_ = 0; T_ < RT; ++T_) {
-            xr[T_][ct] = MF<T>::mma(-ur[ct], ma[T_], xr[T_][ct]);
-            xi[T_][ct] = MF<T>::mma(-ui[ct], ma[T_], xi[T_][ct]);
-          }
-#pragma unroll
-          for (int T_ = 0; T_ < RT; ++T_) {
-            xr[T_][ct] = MF<T>::mma(ui[ct], mb[T_], xr[T_][ct]);
-            xi[T_][ct] = MF<T>::mma(-ur[ct], mb[T_], xi[T_][ct]);
+          for (int T_ = 0; T_ < RT; ++T_) {   // the four products' sum, then one rounding of x's size
+            acc_t pr = acc_t{0, 0, 0, 0}, pi = pr;
+            pr = MF<T>::mma(ur[ct], ma[T_], pr);
+            pi = MF<T>::mma(ui[ct], ma[T_], pi);
+            pr = MF<T>::mma(-ui[ct], mb[T_], pr);
+            pi = MF<T>::mma(ur[ct], mb[T_], pi);
+            xr[T_][ct] -= pr;
+            xi[T_][ct] -= pi;
+            if (WIDE) __builtin_amdgcn_sched_barrier(0);   // else more sums at a time than registers
           }
         }
       }
@@ -1387,27 +1389,33 @@ constexpr int SU_LS = PW_ + 1;   // LDS row stride of the lower block
 template <class T, class Out>
 __device__ __forceinline__ void su_solve(const typename C2<T>::t *L, int cls, typename C2<T>::t (&x)[8], Out out) {
   typedef typename C2<T>::t cT;
+  cT less[8];   // the rows' products so far, subtracted as a sum: one rounding of x's size
+#pragma unroll
+  for (int q = 0; q < 8; ++q) less[q] = cT{0, 0};
 #pragma unroll 1
   for (int kb = 0; kb < 8; ++kb) {
     auto step = [&](auto kc) {
       constexpr int K = decltype(kc)::value;
-      const cT v = cT{su_bc<K>(x[0].x), su_bc<K>(x[0].y)};
+      const cT w = x[0] - less[0], v = cT{su_bc<K>(w.x), su_bc<K>(w.y)};
       const int k = 4 * kb + K;
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         if (q >= 8 - kb) continue;   // rows beyond the block (uniform)
         const cT l = L[(4 * (kb + q) + cls) * SU_LS + k];
-        const cT y = cT{fma(-l.x, v.x, fma(l.y, v.y, x[q].x)), fma(-l.x, v.y, fma(-l.y, v.x, x[q].y))};
-        if (q > 0 || cls > K) x[q] = y;
+        const cT y = cT{fma(l.x, v.x, fma(-l.y, v.y, less[q].x)), fma(l.x, v.y, fma(l.y, v.x, less[q].y))};
+        if (q > 0 || cls > K) less[q] = y;
       }
     };
     step(std::integral_constant<int, 0>{});
     step(std::integral_constant<int, 1>{});
     step(std::integral_constant<int, 2>{});
     step(std::integral_constant<int, 3>{});
-    out(kb, x[0]);
+    out(kb, x[0] - less[0]);
 #pragma unroll
-    for (int q = 0; q < 7; ++q) x[q] = x[q + 1];
+    for (int q = 0; q < 7; ++q) {
+      x[q] = x[q + 1];
+      less[q] = less[q + 1];
+    }
   }
 }
 

@@ -124,3 +124,22 @@ def test_blocks_by_tournament(gpu):
     assert int(di.to_array(np.int32, (1,))[0]) == 0
     # rows of a random matrix: |L| <= 2 or so per level of the tournament, errors of n products
     check_plu(A, dA.to_array(np.complex128, (n, n)), dp.to_array(np.int32, (n,)), 1e-13)
+
+
+@pytest.mark.parametrize("n", [30, 100, 260])
+@pytest.mark.parametrize("wait", [10 ** 7, 0])
+def test_error_of_elimination(gpu, n, wait):
+    """Errors of the factors of I - T W of weak scatterers no larger than those of
+    elimination column by column: the mean (of the logarithms) over 6 systems, each
+    ratio spread by 1.2 or so, below 1.15."""
+    ratio = []
+    for seed in range(6):
+        rng = np.random.default_rng(seed)
+        A = rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))
+        A = np.eye(n) - A / (2.5 * np.sqrt(n)) * 10.0 ** rng.uniform(-3, 0, n)[:, None]
+        LU, piv, _ = getrf_pp(A, 64, wait)
+        plain, rp = eliminate(A)
+        ref, xp = eliminate(A.astype(np.clongdouble))
+        assert np.array_equal(piv, xp) and np.array_equal(rp, xp)
+        ratio.append(float(np.linalg.norm(LU - ref) / np.linalg.norm(plain - ref)))
+    assert np.exp(np.mean(np.log(ratio))) < 1.15
