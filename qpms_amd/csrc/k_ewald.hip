@@ -12,9 +12,9 @@
 // What bounds the sums: FP64 vector instructions (16,000 per triple of LE 7, 433
 // R and 2435 K points), and for few triples the length of one wave's walk. Real
 // wavenumbers leave nearly everything but the phases real, and both signs of m
-// share the phases' steps: 2048 (beta, k) x 3 shifts take 307 us (580 with complex
+// share the phases' steps: 2048 (beta, k) x 3 shifts take 309 us (580 with complex
 // arithmetic throughout), one (beta, k) 25 us (138 with one wave per triple); with
-// complex k 483 us per 1024 (2190 with continued fractions).
+// complex k 450 us per 1024 (2190 with continued fractions).
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cmath>

@@ -21,12 +21,15 @@
 // once: no memset pass.
 //
 // What bounds it: fetching its instructions (10 KB for one y of lMax 4, each run
-// once per wave) while particles are few, the stores when they are many (467
-// particles of lMax 3: 4.3 TB/s). A wave therefore takes a few y, and the groups of
+// once per wave) while particles are few, the stores when they are many. Their rate
+// goes with where a row starts in a 128-byte line (456 to 514 particles of lMax 3,
+// 2331 to 2336 of lMax 1): 5.0 to 5.4 TB/s on its start, 4.7 to 5.1 where rows shift by
+// 64 bytes, 4.1 to 4.4 by 32 or 96 (467 particles of lMax 3, 4.3). A wave therefore takes a few y, and the groups of
 // y are outermost in the grid, so the waves of a CU run the same code at a time.
 // (y as a loop, its stores in it, made the compiler keep the products of all y in
-// scratch: 650 instead of 380 us for 200 particles of lMax 4. Stores aligned to 128
-// bytes, or plain ones, changed nothing.)
+// scratch: 650 instead of 380 us for 200 particles of lMax 4. At 467, a wave's stores
+// cut at 128-byte boundaries, or plain ones, changed nothing: the lines where two rows
+// or two waves meet are still written in parts.)
 #include <hip/hip_runtime.h>
 #include <utility>
 #include "dev_specfunc.hpp"
